@@ -1,0 +1,482 @@
+// gemm_split.hip — products of F32 operands on the 16-bit matrix cores of
+// gfx950 (the VAE's convolutions, src/vae_decoder.cpp:26-58, and the F32
+// weights of ggml_mul_mat / conv_cl, src/mmdit.cpp:13-34):
+//
+//   Y[n, m] = sum_k X[n, k] * W[m, k] + bias[m]
+//
+// Every operand value v is held as two halves of its scaled value: with e the
+// exponent of a bound on |v| over its row or tensor, s = v * 2^(15 - e) (exact;
+// |s| < 2^15), hi = fp16(s), lo = fp16(s - hi). s - hi is exact, so hi + lo is s
+// to 2^-23 of s (or 2^-25 absolute where lo is subnormal: 2^-40 of the bound).
+// Three fp16 MFMAs sum x_hi w_hi + x_hi w_lo + x_lo w_hi in fp32; what is left
+// out, x_lo w_lo, is at most 2^-22 of |x w| with a random sign per term, below
+// what summing K terms in fp32 rounds away, and one MFMA adds 32 products with
+// one rounding of the sum where the fp32 MFMA adds 4. Against 64-bit results
+// the products are as close as the fp32 MFMA's or closer (measured: 30 s VAE
+// decode 1.2e-4 with fp32 MFMAs, see the drivers' tests), at 2.5 PFLOP/s / 3
+// against 157 TFLOP/s.
+//
+// Layout: a row of C values (C % 32 == 0) is C 4-byte words in groups of 32 values, one
+// 128-byte line each: [32 hi][32 lo]. So rows, strides and bytes are those of
+// the f32 rows, and a 32-wide K step of a row is one line.
+#include "tsk_common.h"
+#include "tsk_internal.h"
+#include "tsk_runtime.h"
+
+namespace tsk {
+
+namespace {
+
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((__vector_size__(4 * sizeof(_Float16)))) _Float16 f16x4;
+
+constexpr int NT = 256;
+constexpr int BK = 32;
+
+__device__ __forceinline__ bool finite_f(float v) { return fabsf(v) <= 3.4028234664e38f; }
+
+// the smallest e with b < 2^e (b >= 0), from -112 on: 2^(15 - e) stays finite
+__device__ __forceinline__ int bound_exp(float b) {
+    const int e = (int) (__float_as_uint(b) >> 23) - 126;
+    return e < -112 ? -112 : e;
+}
+__device__ __forceinline__ float exp2_int(int e) { return __uint_as_float((uint32_t) (e + 127) << 23); }
+
+__device__ __forceinline__ void split4(const float (&v)[4], float scale, f16x4 &hi, f16x4 &lo) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float s = v[r] * scale;
+        hi[r] = (_Float16) s;
+        lo[r] = (_Float16) (s - (float) hi[r]);
+    }
+}
+// word offset of channel c's group and the halfword of its hi inside a split row
+__device__ __forceinline__ void store_split4(uint32_t *row, int c, const f16x4 hi, const f16x4 lo) {
+    uint16_t *g = (uint16_t *) (row + (c & ~31)) + (c & 31);
+    *(f16x4 *) g = hi;
+    *(f16x4 *) (g + 32) = lo;
+}
+
+// raise a slot to m (>= 0, finite): the slot only grows, so a stale read can
+// only cause an atomic that changes nothing
+__device__ __forceinline__ void raise_slot(float *slot, float m) {
+    if (m > __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax((int *) slot, __float_as_int(m));
+}
+
+// fp32 product of one output, for results that are not finite in the split
+// products: an infinity or NaN in its operands (finite ones cannot overflow:
+// |s| < 2^15). The f32 operands give what fp32 products give.
+__device__ __forceinline__ float f32_dot(const SplitGemm &p, int m, int n, int k0, int k1) {
+    float s = 0.0f;
+    const float *w = p.wf + (int64_t) m * p.ld_wf;
+    if (p.conv_ic) {
+        const int b = n / p.conv_ow, o = n - b * p.conv_ow;
+        for (int k = k0; k < k1; ++k) {
+            const int kw = k / p.conv_ic, ic = k - kw * p.conv_ic;
+            const int iw = o * p.conv_s + kw * p.conv_d - p.conv_p;
+            if (iw >= 0 && iw < p.conv_iw) s = fmaf(p.xf[(int64_t) b * p.xf_batch + (int64_t) iw * p.ld_xf + ic], w[k], s);
+        }
+    } else {
+        for (int k = k0; k < k1; ++k) s = fmaf(p.xf[(int64_t) n * p.ld_xf + k], w[k], s);
+    }
+    return s;
+}
+
+// Workgroup = 2 x 2 waves of TM x TN 16x16 tiles; operand lines by direct
+// global -> LDS loads into a two-stage ring of 32-wide K steps (line chunk c of
+// a row at slot c ^ ((row / 2) % 8): the 16 rows of a fragment read hit
+// distinct banks). Per step and 64 x 64 wave tile: 16 16-byte LDS reads for 48
+// MFMAs of 16 cycles; two workgroups per CU.
+template <int TM, int TN, bool SNAKE>
+__global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
+    constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
+    constexpr int ROWS = BM + BN, STAGE = ROWS * BK;          // words per stage
+    constexpr int NWL = ROWS / 8, WLW = NWL / 4;             // wave-loads (8 rows) per stage, per wave
+    static_assert(NWL % 4 == 0, "whole wave-loads per wave");
+    constexpr int LDT = BM + 4;
+    constexpr int RING = 2 * STAGE, EPI_F = BN * LDT;
+    __shared__ __attribute__((aligned(16))) float smem[RING > EPI_F ? RING : EPI_F];
+
+    // workgroup -> tile. L % 8 is the XCD: with deal 1 every m tile of a token
+    // tile runs on one XCD (its L2 fetches the activation rows once), with
+    // deal 2 every token tile of an (m tile, slice) pair (the weights once)
+    int tm, tn, z;
+    {
+        const int L = (int) blockIdx.x, q = L >> 3, S = p.splits;
+        if (p.deal == 1) {
+            const int t = (q / p.tiles_m) * 8 + (L & 7);
+            if (t >= p.tiles_n * S) return;
+            tm = q % p.tiles_m;
+            tn = t % p.tiles_n;
+            z = t / p.tiles_n;
+        } else if (p.deal == 2) {
+            const int t = (q / p.tiles_n) * 8 + (L & 7);
+            if (t >= p.tiles_m * S) return;
+            tn = q % p.tiles_n;
+            tm = t / S;
+            z = t % S;
+        } else {
+            tm = L % p.tiles_m;
+            tn = L / p.tiles_m % p.tiles_n;
+            z = L / (p.tiles_m * p.tiles_n);
+        }
+    }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lg = lane >> 4;
+    const int wm = wave & 1, wn = wave >> 1;
+    const int bm0 = tm * BM, bn0 = tn * BN;
+
+    // activation rows relative to the tile's first row, so that 32-bit byte
+    // offsets reach every row of the tile whatever the tensor's size
+    int64_t r0 = bn0;
+    if (p.conv_ic) {
+        const int b = bn0 / p.conv_ow, o = bn0 - b * p.conv_ow;
+        r0 = (int64_t) b * p.conv_iw + min(max(o * p.conv_s - p.conv_p, 0), p.conv_iw - 1);
+    }
+    const int64_t x_left = (p.x_rows - r0) * p.ld_x * 4;
+    const int x_range = (int) min(x_left, (int64_t) 0x7fffffff);
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *) p.w, (short) 0, (int) ((int64_t) p.M * p.ld_w * 4), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *) (p.x + r0 * p.ld_x), (short) 0, x_range, 0x00020000);
+    constexpr uint32_t PAST = 0x80000000u;                   // beyond every range: reads zero
+    uint32_t voff[WLW];                                      // byte offsets of this lane's chunks
+    bool isw[WLW];                                           // wave-uniform
+    int xb[WLW], xi[WLW];                                    // activation rows: item's first row - r0, first position
+#pragma unroll
+    for (int q = 0; q < WLW; ++q) {
+        const int j = wave * WLW + q, R = 8 * j + (lane >> 3);
+        const uint32_t c16 = (uint32_t) ((lane & 7) ^ ((R >> 1) & 7)) * 16;
+        xb[q] = xi[q] = 0;
+        isw[q] = j < BM / 8;
+        if (isw[q]) {
+            voff[q] = bm0 + R < p.M ? (uint32_t) ((int64_t) (bm0 + R) * p.ld_w * 4) + c16 : PAST;
+        } else {
+            const int n = bn0 + R - BM;
+            if (p.conv_ic) {
+                const int b = n / p.conv_ow, o = n - b * p.conv_ow;
+                xb[q] = (int) ((int64_t) b * p.conv_iw - r0);
+                xi[q] = n < p.N ? o * p.conv_s - p.conv_p : INT32_MIN / 2;
+            } else {
+                voff[q] = n < p.N ? (uint32_t) (((int64_t) n - r0) * p.ld_x * 4) + c16 : PAST;
+            }
+        }
+    }
+    const int nk_all = p.K / BK, kt0 = (int) ((int64_t) z * nk_all / p.splits);
+    const int nk = (int) ((int64_t) (z + 1) * nk_all / p.splits) - kt0;
+    // the tap and channel step of the next load
+    int ic_left = 0, kw = 0;
+    uint32_t sw = (uint32_t) kt0 * 128, sx = sw;
+    auto set_tap = [&]() {
+#pragma unroll
+        for (int q = 0; q < WLW; ++q) {
+            if (isw[q]) continue;
+            const int R = 8 * (wave * WLW + q) + (lane >> 3);
+            const int iw = xi[q] + kw * p.conv_d;
+            const uint32_t c16 = (uint32_t) ((lane & 7) ^ ((R >> 1) & 7)) * 16;
+            voff[q] = iw >= 0 && iw < p.conv_iw ? (uint32_t) ((xb[q] + iw) * (int) p.ld_x * 4) + c16 : PAST;
+        }
+    };
+    if (p.conv_ic) {
+        const int steps = p.conv_ic / BK;
+        kw = kt0 / steps;
+        sx = (uint32_t) (kt0 - kw * steps) * 128;
+        ic_left = steps - (kt0 - kw * steps);
+        set_tap();
+    }
+    auto issue = [&](int slot) {
+        float *st = smem + slot * STAGE;
+#pragma unroll
+        for (int q = 0; q < WLW; ++q) {
+            // (arguments of template-dependent type, voff[q] itself, would leave
+            // the kernel uninstantiated on the host side)
+            const int j = wave * WLW + q;
+            const uint32_t off = voff[q];
+            if (isw[q])
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_void *) (st + j * 8 * BK), 16, off, sw, 0, 0);
+            else
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_void *) (st + j * 8 * BK), 16, off, sx, 0, 0);
+        }
+        sw += 128;
+        sx += 128;
+        if (p.conv_ic && --ic_left == 0) {
+            ++kw;
+            sx = 0;
+            ic_left = p.conv_ic / BK;
+            set_tap();
+        }
+    };
+
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
+    auto at = [](int row, int c) { return row * BK + ((c ^ ((row >> 1) & 7)) << 2); };
+    if (nk > 0) issue(0);
+    for (int it = 0; it < nk; ++it) {
+        // this wave's loads of the step have landed, then every wave's; the
+        // barrier also ends every wave's reads of the other slot
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (it + 1 < nk) issue((it + 1) & 1);
+        const float *st = smem + (it & 1) * STAGE;
+        f16x8 ah[TM], al[TM], bh[TN], bl[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            ah[i] = *(const f16x8 *) &st[at((wm * TM + i) * 16 + lr, lg)];
+            al[i] = *(const f16x8 *) &st[at((wm * TM + i) * 16 + lr, 4 + lg)];
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            bh[j] = *(const f16x8 *) &st[at(BM + (wn * TN + j) * 16 + lr, lg)];
+            bl[j] = *(const f16x8 *) &st[at(BM + (wn * TN + j) * 16 + lr, 4 + lg)];
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
+    }
+
+    // ---- epilogue: the accumulators as the workgroup's [BN][BM] tile in LDS,
+    // then four consecutive outputs of one token per thread
+    __syncthreads();                                          // the ring's last reads are done
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            *(f32x4 *) &smem[((wn * TN + j) * 16 + lr) * LDT + (wm * TM + i) * 16 + 4 * lg] = acc[i][j];
+    __syncthreads();
+    constexpr int G = BM / 4;
+    static_assert(NT % G == 0, "fixed channel group per thread");
+    const int ml = (tid % G) * 4, m0 = bm0 + ml;
+    const bool mok = m0 < p.M;                                // M % 4 == 0: all four or none
+    float bv[4] = {0, 0, 0, 0}, ea[4], eb[4];
+    int we[4] = {0, 0, 0, 0};
+    float oscale = 0.0f, ym = 0.0f, sm = 0.0f;
+    if (mok) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (p.bias) bv[r] = p.bias[m0 + r];
+            we[r] = p.we[m0 + r] - 30;
+        }
+        if constexpr (SNAKE) {
+            const int c0 = m0 % p.period;                     // period % 4 == 0: c0 + 3 < period
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                ea[r] = p.ea[c0 + r];
+                eb[r] = p.eb[c0 + r];
+            }
+        }
+    }
+    if constexpr (SNAKE) {
+        if (p.yp) {
+            // |y| <= sum |w| max |x| + max |bias| (+ max |old y|), |snake(y)| <= |y| + max eb
+            // (l1 and badd hold these maxima and 1 % for the roundings)
+            float bound = p.l1 * *p.amax_x + p.badd;
+            if (p.amax_old) bound += 1.01f * *p.amax_old;
+            const int eo = bound_exp(bound);
+            oscale = exp2_int(15 - eo);
+            if (blockIdx.x == 0 && tid == 0) *p.e_out = eo;
+        }
+    }
+    const int k_lo = kt0 * BK, k_hi = (kt0 + nk) * BK;
+    for (int nl = tid / G; nl < BN; nl += NT / G) {
+        const int n = bn0 + nl;
+        if (n >= p.N || !mok) break;
+        const f32x4 a4 = *(const f32x4 *) &smem[nl * LDT + ml];
+        const int xe = p.xe[p.xe_per_row ? n : 0];
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float a = __builtin_ldexpf(a4[r], xe + we[r]);
+            if (!SNAKE && !finite_f(a4[r])) a = f32_dot(p, m0 + r, n, k_lo, k_hi);
+            o[r] = a + bv[r];
+        }
+        if constexpr (!SNAKE) {
+            if (p.y_bf16) {
+                uint16_t *yr = (uint16_t *) p.y + (int64_t) n * p.ld_y + m0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) yr[r] = f32_to_bf16_bits(o[r]);
+            } else {
+                *(f32x4 *) ((float *) p.y + (int64_t) z * p.part_stride + (int64_t) n * p.ld_y + m0) =
+                    f32x4{o[0], o[1], o[2], o[3]};
+            }
+        } else {
+            if (p.y) {
+                float *yr = (float *) p.y + (int64_t) n * p.ld_y + m0;
+                if (p.accumulate) {
+                    const f32x4 old = *(const f32x4 *) yr;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[r] = old[r] + o[r];
+                }
+                *(f32x4 *) yr = f32x4{o[0], o[1], o[2], o[3]};
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (finite_f(o[r])) ym = fmaxf(ym, fabsf(o[r]));
+            }
+            float sv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float sn = sinf(o[r] * ea[r]);
+                sv[r] = o[r] + (sn * sn) * eb[r];
+                if (finite_f(sv[r])) sm = fmaxf(sm, fabsf(sv[r]));
+            }
+            if (p.yp) {
+                f16x4 hi, lo;
+                split4(sv, oscale, hi, lo);
+                store_split4(p.yp + (int64_t) n * p.ld_y, m0, hi, lo);
+            } else {
+                *(f32x4 *) (p.y2 + (int64_t) n * p.ld_y + m0) = f32x4{sv[0], sv[1], sv[2], sv[3]};
+            }
+        }
+    }
+    if constexpr (SNAKE) {
+        ym = wave_max(ym);
+        sm = wave_max(sm);
+        if (lane == 0) {
+            if (p.amax_y) raise_slot(p.amax_y, ym);
+            if (p.amax_s) raise_slot(p.amax_s, sm);
+        }
+    }
+}
+
+template <int TM, int TN>
+void launch_split_tiles(const SplitGemm &p, int grid, hipStream_t s) {
+    if (p.ea) launch_kernel((gemm_split_kernel<TM, TN, true>), dim3(grid), dim3(NT), 0, s, p);
+    else launch_kernel((gemm_split_kernel<TM, TN, false>), dim3(grid), dim3(NT), 0, s, p);
+}
+
+// one workgroup: max |x| over n values into slot[0] and its exponent into
+// e[0]; slots 1 .. nslot - 1 cleared
+__global__ __launch_bounds__(1024) void split_begin_kernel(const float *x, int64_t n, float *slot, int nslot, int *e) {
+    __shared__ float red[16];
+    float m = 0.0f;
+    for (int64_t i = threadIdx.x; i < n; i += 1024) {
+        const float a = fabsf(x[i]);
+        if (finite_f(a)) m = fmaxf(m, a);
+    }
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    for (int i = threadIdx.x; i < nslot; i += 1024)
+        if (i) slot[i] = 0.0f;
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < 16; ++i) m = fmaxf(m, red[i]);
+        slot[0] = m;
+        e[0] = bound_exp(m);
+    }
+}
+
+// x [C][T] -> split rows [T][C] at exponent e[0]; one thread per (4 channels, t)
+__global__ __launch_bounds__(256) void split_transpose_kernel(const float *x, int C, int T, const int *e, uint32_t *y) {
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    const int t = (int) (i % T), c = (int) (i / T) * 4;
+    if (c >= C) return;
+    const float scale = exp2_int(15 - *e);
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = x[(int64_t) (c + r) * T + t];
+    f16x4 hi, lo;
+    split4(v, scale, hi, lo);
+    store_split4(y + (int64_t) t * C, c, hi, lo);
+}
+
+// f32 rows -> split rows at their own exponents, one wave per row: the row's
+// maximum, then its groups (8 lanes each). In place works: a wave has loaded
+// all of a group before it writes it, and no other wave reads the row.
+__device__ __forceinline__ void split_row(const float *x, int cols, uint32_t *y, int *e) {
+    const int lane = threadIdx.x & 63;
+    float m = 0.0f;
+    for (int c = 4 * lane; c < cols; c += 256) {
+        const f32x4 v = *(const f32x4 *) (x + c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (finite_f(v[r])) m = fmaxf(m, fabsf(v[r]));
+    }
+    const int ex = bound_exp(wave_max(m));
+    if (lane == 0) *e = ex;
+    const float scale = exp2_int(15 - ex);
+    for (int c = 4 * lane; c < cols; c += 256) {
+        const f32x4 v = *(const f32x4 *) (x + c);
+        const float a[4] = {v[0], v[1], v[2], v[3]};
+        f16x4 hi, lo;
+        split4(a, scale, hi, lo);
+        store_split4(y, c, hi, lo);
+    }
+}
+
+__global__ __launch_bounds__(NT) void split_rows_kernel(const float *x, int64_t ld_x, int64_t rows, int cols,
+                                                        uint32_t *y, int *e) {
+    const int64_t row = (int64_t) blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+    if (row < rows) split_row(x + row * ld_x, cols, y + row * cols, e + row);
+}
+
+}  // namespace
+
+hipError_t launch_split_rows(const float *x, int64_t ld_x, int64_t rows, int cols, uint32_t *y, int *e, hipStream_t s) {
+    if (cols % BK || ld_x % 4 || rows < 1) return hipErrorInvalidValue;
+    launch_kernel(split_rows_kernel, dim3((unsigned) ((rows + NT / 64 - 1) / (NT / 64))), dim3(NT), 0, s, x, ld_x, rows,
+                  cols, y, e);
+    return hipGetLastError();
+}
+
+bool split_gemm_fits(int64_t M, int64_t K, int64_t x_rows, int64_t ld_x, int items) {
+    const int64_t lim = (int64_t) 1 << 31;
+    return M % 4 == 0 && K % BK == 0 && M * K * 4 < lim && (x_rows * ld_x * 4 < lim || items == 1);
+}
+
+hipError_t launch_gemm_split(SplitGemm &p, hipStream_t s) {
+    if (p.M < 4 || p.M % 4 || p.N < 1 || p.K < BK || p.K % BK || p.splits < 1 || p.splits > p.K / BK || !p.x || !p.w ||
+        !p.we || !p.xe || p.ld_y % 4 || (int64_t) p.M * p.ld_w * 4 >= ((int64_t) 1 << 31))
+        return hipErrorInvalidValue;
+    if (p.ea && (p.period < 4 || p.period % 4 || p.M % p.period || p.splits != 1 || p.y_bf16 || (!p.yp && !p.y2) ||
+                 (p.yp && (p.ld_y % 32 || p.period % 32 || !p.amax_x || !p.e_out))))
+        return hipErrorInvalidValue;
+    if (!p.ea && (!p.y || !p.xf || !p.wf || p.accumulate || (p.splits > 1 && (p.bias || p.y_bf16))))
+        return hipErrorInvalidValue;
+    if (p.conv_ic && (p.conv_ic % BK || p.K % p.conv_ic || p.conv_ow < 1 || p.conv_iw < 1 || p.conv_s < 1 ||
+                      p.conv_d < 1 || p.conv_p < 0 || p.N % p.conv_ow))
+        return hipErrorInvalidValue;
+    p.x_rows = p.conv_ic ? (int64_t) (p.N / p.conv_ow) * p.conv_iw : p.N;
+    const int64_t tiles44 = (int64_t) ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.splits;
+    const bool big = tiles44 >= 256;
+    p.tiles_m = (p.M + 127) / 128;
+    p.tiles_n = big ? (p.N + 127) / 128 : (p.N + 63) / 64;
+    // Which operand an XCD's L2 should fetch once: the larger one. Dealing
+    // whole token tiles (or (m tile, slice) pairs) over the 8 XCDs needs
+    // enough of them that the last round of 8 is a small part.
+    const int64_t tn = (int64_t) p.tiles_n * p.splits, tm = (int64_t) p.tiles_m * p.splits;
+    const bool can1 = tn >= 64 || tn % 8 == 0, can2 = tm >= 64 || tm % 8 == 0;
+    const bool x_larger = p.x_rows * p.ld_x > (int64_t) p.M * p.K;
+    p.deal = can1 && (x_larger || !can2) ? 1 : can2 ? 2 : 0;
+    const int64_t grid = p.deal == 1 ? (tn + 7) / 8 * 8 * p.tiles_m
+                       : p.deal == 2 ? (tm + 7) / 8 * 8 * p.tiles_n : tm * p.tiles_n;
+    if (big) launch_split_tiles<4, 4>(p, (int) grid, s);
+    else launch_split_tiles<4, 2>(p, (int) grid, s);
+    return hipGetLastError();
+}
+
+hipError_t launch_split_begin(const float *x, int64_t n, float *slot, int nslot, int *e, hipStream_t s) {
+    launch_kernel(split_begin_kernel, dim3(1), dim3(1024), 0, s, x, n, slot, nslot, e);
+    return hipGetLastError();
+}
+
+hipError_t launch_split_transpose(const float *x, int C, int T, const int *e, uint32_t *y, hipStream_t s) {
+    if (C % 32) return hipErrorInvalidValue;
+    const int64_t n = (int64_t) (C / 4) * T;
+    launch_kernel(split_transpose_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, x, C, T, e, y);
+    return hipGetLastError();
+}
+
+}  // namespace tsk

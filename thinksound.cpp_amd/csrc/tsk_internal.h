@@ -191,8 +191,7 @@ enum GroupEpi : int {
     // SwiGLU over two weights sharing X: y[n, m] = silu(X W[m]) * (X W3[m]),
     // no bias (convmlp / mlp, src/mmdit.cpp:39-52)
     EPI_SWIGLU_F32 = 15,
-    EPI_SWIGLU_BF16 = 16,
-    EPI_F32X = 17         // y f32 = acc + bias (+ y), SnakeBeta into y / y2 / split planes (see GemmProblem)
+    EPI_SWIGLU_BF16 = 16
 };
 enum GemmFlags : int { GEMM_X_F32 = 1 };
 
@@ -226,16 +225,6 @@ struct GemmProblem {
     float theta_scale, freq_scale, eps;
     float q_scale;                 // q is multiplied by this before its fp16 cast
     const float *rope_cs;          // launch_gemm_ks: (cos, sin) of pair i at position s: [s * 64 + 2 i]
-    // EPI_F32X (split products of F32 weights): y f32 = acc + bias, plus the
-    // old y with accumulate (y nullable: not written), then optionally a
-    // SnakeBeta (snk_ea non-null; channel m % snk_period, ea = exp(alpha),
-    // eb = exp(-beta)) into y2 (f32, row stride ld_y) or yp (bf16 split
-    // planes, rows of 3 ld_y: period group g of a row at 3 g snk_period holds
-    // hi | hi | lo of its channels), else in place of y
-    const float *snk_ea, *snk_eb;
-    int snk_period;
-    float *y2;
-    uint16_t *yp;
     // filled by the launchers
     int tiles_m, tiles_n, block_begin;
     int kt_split;                  // 32-wide k tiles per split (launch_gemm_ks)
@@ -418,6 +407,51 @@ struct F32Snake {
 // (plain rows or implicit im2col), y f32 or bf16 (+bias), optionally followed
 // by a SnakeBeta (f32 y only)
 hipError_t launch_gemm_f32(const GemmProblem &p, int y_bf16, hipStream_t s, const F32Snake *snake = nullptr);
+// F32 products on the fp16 matrix cores (gemm_split.hip): operands as split
+// rows (32 hi, 32 lo fp16 per group of 32 values, of the value times
+// 2^(15 - e); one 4-byte word per value, strides in words)
+struct SplitGemm {
+    const uint32_t *x, *w;         // split activation rows, split weight rows [M][K] (ld_w)
+    int64_t ld_x, ld_w;
+    const int *we;                 // [M] exponents of the weight rows
+    const int *xe;                 // exponent of x, or with xe_per_row one per row
+    int xe_per_row;
+    const float *bias;             // [M], nullable
+    void *y;                       // f32 (or y_bf16) rows; with a SnakeBeta nullable
+    int64_t ld_y;                  // also the row stride of y2 and yp
+    int y_bf16, accumulate;        // accumulate: y += (SnakeBeta form only)
+    int M, N, K;
+    int splits;                    // K slices: slice z into y + z * part_stride, no bias (1: none)
+    int64_t part_stride;
+    // implicit im2col as GemmProblem's, over contiguous batch items of conv_iw rows
+    int conv_ic, conv_iw, conv_ow, conv_s, conv_p, conv_d;
+    // without a SnakeBeta: the f32 operands (results of infinities and NaN)
+    const float *xf, *wf;
+    int64_t ld_xf, xf_batch, ld_wf;
+    // SnakeBeta of y (ea non-null; F32Snake's parameters): split rows yp, or f32 rows y2
+    const float *ea, *eb;
+    int period;
+    float *y2;
+    uint32_t *yp;
+    // yp's exponent, from a bound: l1 * *amax_x + badd (+ 1.01 * *amax_old), written to *e_out;
+    // slots raised to max |y| / max |snake| (nullable)
+    float l1, badd;
+    const float *amax_x, *amax_old;
+    int *e_out;
+    float *amax_y, *amax_s;
+    // set by the launcher
+    int tiles_m, tiles_n, deal;
+    int64_t x_rows;
+};
+// M % 4, K (and conv_ic) % 32, 16-byte aligned rows (strides % 4)
+hipError_t launch_gemm_split(SplitGemm &p, hipStream_t s);
+bool split_gemm_fits(int64_t M, int64_t K, int64_t x_rows, int64_t ld_x, int items);
+// f32 rows (stride ld_x) -> split rows [rows][cols] and their exponents; in place with y == x, ld_x == cols
+hipError_t launch_split_rows(const float *x, int64_t ld_x, int64_t rows, int cols, uint32_t *y, int *e, hipStream_t s);
+// slot[0] = max |x| of the finite values, *e its exponent, slot[1 .. nslot) = 0
+hipError_t launch_split_begin(const float *x, int64_t n, float *slot, int nslot, int *e, hipStream_t s);
+// x [C][T] f32 -> split rows [T][C] at exponent *e (C % 32 == 0)
+hipError_t launch_split_transpose(const float *x, int C, int T, const int *e, uint32_t *y, hipStream_t s);
 // y = silu(a) * b, f32, n elements
 hipError_t launch_silu_mul(const float *a, const float *b, float *y, int64_t n, hipStream_t s);
 // y[n][m] = sum of S K-split slices p[z][n][m] (rows of M, slices `stride` apart, summed in order)

@@ -2,8 +2,10 @@
 // 62-124) on gfx950, F32 throughout (the converter keeps the VAE F32).
 //
 // Activations are token-major rows [T][C] (channels fastest), so every
-// convolution is one F32 GEMM over implicit im2col rows (launch_gemm_f32,
-// fp32 MFMA): y[t][oc] = sum_{kw, ic} W[oc][kw][ic] x[t + kw d - p][ic].
+// convolution is one F32 GEMM over implicit im2col rows:
+// y[t][oc] = sum_{kw, ic} W[oc][kw][ic] x[t + kw d - p][ic], its products on the
+// fp16 matrix cores from split operands (gemm_split.hip) where the channel
+// counts allow, else fp32 MFMAs (gemm_f32.hip).
 // The reference keeps [T, C] with time fastest and runs im2col + mul_mat; the
 // sums are the same products in another order.
 //
@@ -46,7 +48,8 @@ struct VW {
     int stride;             // ct: the stride s
     size_t offset;          // device float offset of the prepared layout
     size_t count;           // floats stored
-    size_t offset16;        // split products: bf16 offset of the planes (3 count: [hi | lo | hi] per IC group)
+    size_t woffset;         // split products: int offset of the rows' exponents
+    float l1, amax;         // split products: max over the rows of sum |w|, max |w| (biases, exp(-beta): max)
 };
 
 }  // namespace
@@ -60,14 +63,13 @@ struct tsk_vae {
     float *lat = nullptr;                          // latent rows [T][latent_dim]
     size_t act_cap = 0;
     int hop = 1;
-    // F32 products as three bf16 ones (opt-in, TSK_VAE_SPLIT=1 when the model
-    // is created; every channel count a multiple of 64): the kernels' split
-    // planes, and the activations the convolutions read as split planes
-    // [T][3 C] (two buffers and the latent)
+    // split products (every channel count a multiple of 32): the kernels in
+    // the blob and the snakes in act[1], act[2], lat are split rows
+    // (gemm_split.hip); the residual stream act[0] stays f32
     bool split = false;
-    uint16_t *blob16 = nullptr;
-    uint16_t *ap[2] = {nullptr, nullptr};
-    uint16_t *latp = nullptr;
+    int *wexp = nullptr;                           // exponents of the kernels' rows
+    float *slots = nullptr;                        // max |snake| and max |residual| per convolution
+    int *exps = nullptr;                           // exponent of each split tensor
 };
 
 namespace {
@@ -82,7 +84,8 @@ void addv(tsk_vae *v, const std::string &name, int64_t a, int64_t b, int64_t c, 
     x.conv = conv;
     x.ct = ct;
     x.stride = stride;
-    x.offset = x.offset16 = 0;
+    x.offset = x.woffset = 0;
+    x.l1 = x.amax = 0.0f;
     // prepared layouts: conv kw-major [OC][K * IC]; transposed conv the merged
     // 3-tap kernel [s * OC][3 * IC] and its bias replicated [s * OC]
     x.count = ct ? (size_t) stride * c * 3 * b : (size_t) (a * b * c);
@@ -183,89 +186,85 @@ int conv_t(const tsk_vae *v, const std::string &p, const float *x, int IC, int T
     return TSK_OK;
 }
 
-// ---- split products: the cooperative bf16 GEMM over 3 IC (weight planes
-// [hi | lo | hi] against input planes [hi | hi | lo]: x w up to x_lo w_lo and
-// the lo roundings, ~2^-17 of |x w| per term) with the EPI_F32X epilogue:
-// bias, the residual update, and the SnakeBeta `snake` (parameters of
-// period C) into the split planes yp the next convolution reads, or into an
-// f32 y2 (the final snake, for the fp32 output convolution)
-struct SplitOut {
-    float *y;           // f32 output rows (nullable: not written)
-    bool accumulate;    // y += conv
-    const char *snake;  // SnakeBeta parameters' prefix, or null
-    int C;              // its period (channels)
-    float *y2;          // the snake as f32 rows
-    uint16_t *yp;       // the snake as split planes
+// ---- split products. Convolution number i of the decode reads the split
+// tensor i (exponent exps[i], max |value| slots[2 i]) and writes tensor i + 1
+// (slots[2 i + 2]) as the SnakeBeta of its output; the residual stream it
+// leaves has max |value| slots[2 i + 3].
+constexpr int VAE_CONVS = 1 + 5 * 7;
+constexpr int VAE_SLOTS = 2 * (VAE_CONVS + 1);
+
+struct SplitStep {
+    int i;                 // convolution number
+    const float *x;        // split rows in
+    float *y;              // f32 output rows (nullable: not written)
+    int old;               // >= 0: y += conv, the old y left by convolution `old`
+    std::string snake;     // SnakeBeta parameters' prefix
+    int C;                 // its period (channels)
+    float *out;            // the snake: split rows, or f32 rows (last)
+    bool last;
 };
 
-void set_out(const tsk_vae *v, GemmProblem &q, const SplitOut &o) {
-    q.y = o.y;
-    q.accumulate = o.accumulate ? 1 : 0;
-    if (o.snake) {
-        q.snk_ea = wp(v, std::string(o.snake) + ".alpha");
-        q.snk_eb = wp(v, std::string(o.snake) + ".beta");
-        q.snk_period = o.C;
-        q.y2 = o.y2;
-        q.yp = o.yp;
-    }
+SplitGemm split_gemm(const tsk_vae *v, const std::string &p, const SplitStep &t, int IC) {
+    const VW &w = wi(v, p + ".weight"), &b = wi(v, p + ".bias"), &sb = wi(v, t.snake + ".beta");
+    SplitGemm q;
+    memset(&q, 0, sizeof(q));
+    q.x = (const uint32_t *) t.x; q.ld_x = IC;
+    q.w = (const uint32_t *) (v->blob + w.offset);
+    q.we = v->wexp + w.woffset;
+    q.xe = v->exps + t.i;
+    q.bias = v->blob + b.offset;
+    q.y = t.y; q.accumulate = t.old >= 0;
+    q.splits = 1;
+    q.conv_s = q.conv_d = 1;
+    q.ea = wp(v, t.snake + ".alpha"); q.eb = v->blob + sb.offset; q.period = t.C;
+    if (t.last) q.y2 = t.out;
+    else q.yp = (uint32_t *) t.out;
+    q.l1 = 1.01f * w.l1; q.badd = 1.01f * (b.amax + sb.amax);
+    q.amax_x = v->slots + 2 * t.i;
+    q.amax_old = t.old >= 0 ? v->slots + 2 * t.old + 3 : nullptr;
+    q.e_out = v->exps + t.i + 1;
+    q.amax_s = v->slots + 2 * t.i + 2;
+    q.amax_y = t.y ? v->slots + 2 * t.i + 3 : nullptr;
+    return q;
 }
 
-int conv_split(const tsk_vae *v, const std::string &p, const uint16_t *xp, int IC, int T_in, int pad, int dil,
-               const SplitOut &o, hipStream_t s) {
+int conv_split(const tsk_vae *v, const std::string &p, int IC, int T_in, int pad, int dil, const SplitStep &t,
+               hipStream_t s) {
     const VW &w = wi(v, p + ".weight");
     const int KW = (int) w.ne[0], OC = (int) w.ne[2];
-    GemmGroup g;
-    memset(&g, 0, sizeof(g));
-    g.nprob = 1;
-    GemmProblem &q = g.p[0];
-    q.x = xp; q.ld_x = 3 * IC;
-    q.w = v->blob16 + w.offset16; q.ld_w = (int64_t) KW * 3 * IC;
-    q.bias = wp(v, p + ".bias");
+    SplitGemm q = split_gemm(v, p, t, IC);
+    q.ld_w = (int64_t) KW * IC;
     q.ld_y = OC;
     const int T_out = T_in + 2 * pad - dil * (KW - 1);
-    q.M = OC; q.N = T_out; q.K = KW * 3 * IC; q.splits = 1;
+    q.M = OC; q.N = T_out; q.K = KW * IC;
     if (KW > 1 || pad) {
-        q.conv_ic = 3 * IC; q.conv_iw = T_in; q.conv_ow = T_out; q.conv_s = 1; q.conv_p = pad; q.conv_d = dil;
+        q.conv_ic = IC; q.conv_iw = T_in; q.conv_ow = T_out; q.conv_p = pad; q.conv_d = dil;
     }
-    set_out(v, q, o);
-    return hipcheck(launch_gemm_coop(g, EPI_F32X, s), "vae split conv");
+    return hipcheck(launch_gemm_split(q, s), "vae split conv");
 }
 
-// the transposed convolution of conv_t over the split planes: the merged
-// kernel's planes [s OC][3 taps][3 IC], its two-tap phase groups
-int conv_t_split(const tsk_vae *v, const std::string &p, const uint16_t *xp, int IC, int T_in, const SplitOut &o,
-                 hipStream_t s) {
+// the transposed convolution of conv_t: the merged kernel's two-tap phase groups
+int conv_t_split(const tsk_vae *v, const std::string &p, int IC, int T_in, const SplitStep &t, hipStream_t s) {
     const VW &w = wi(v, p + ".weight");
     const int OC = (int) w.ne[2], st = w.stride;
-    const uint16_t *wq = v->blob16 + w.offset16;
-    const float *bias = wp(v, p + ".bias");
     const int ra = ct_split_phase(w.ne[0], st);
-    GemmGroup g;
-    memset(&g, 0, sizeof(g));
-    g.nprob = 1;
-    GemmProblem &q = g.p[0];
-    q.x = xp; q.ld_x = 3 * IC;
-    q.ld_w = (int64_t) 9 * IC;
-    q.ld_y = (int64_t) st * OC;
-    q.N = T_in; q.splits = 1;
-    q.conv_ic = 3 * IC; q.conv_iw = T_in; q.conv_ow = T_in; q.conv_s = 1; q.conv_d = 1;
-    set_out(v, q, o);
-    if (ra < 0) {
-        q.w = wq; q.bias = bias;
-        q.M = st * OC; q.K = 9 * IC; q.conv_p = 1;
-        return hipcheck(launch_gemm_coop(g, EPI_F32X, s), "vae split transposed conv");
-    }
-    for (int gi = 0; gi < 2; ++gi) {
-        const int r0 = gi ? ra : 0, r1 = gi ? st : ra;
-        if (r1 <= r0) continue;
+    const SplitGemm q0 = split_gemm(v, p, t, IC);
+    for (int g = 0; g < 2; ++g) {
+        const int r0 = ra < 0 ? 0 : g ? ra : 0, r1 = ra < 0 || g ? st : ra;
+        if (r1 <= r0 || (ra < 0 && g)) continue;
         const int64_t row0 = (int64_t) r0 * OC;
-        q.w = wq + row0 * 9 * IC + (gi ? 3 * IC : 0);   // taps 1, 2 for the second group
-        q.bias = bias + row0;
-        q.y = o.y ? o.y + row0 : nullptr;
-        q.y2 = o.y2 ? o.y2 + row0 : nullptr;
-        q.yp = o.yp ? o.yp + 3 * row0 : nullptr;          // row0 is a multiple of the period OC
-        q.M = (r1 - r0) * OC; q.K = 6 * IC; q.conv_p = gi ? 0 : 1;
-        const int rc = hipcheck(launch_gemm_coop(g, EPI_F32X, s), "vae split transposed conv");
+        SplitGemm q = q0;
+        q.w += row0 * 3 * IC + (ra >= 0 && g ? IC : 0);     // taps 1, 2 for the second group
+        q.ld_w = (int64_t) 3 * IC;
+        q.we += row0;
+        q.bias += row0;
+        q.y = (float *) q.y + row0;
+        q.ld_y = (int64_t) st * OC;
+        if (q.yp) q.yp += row0;                              // row0 is a multiple of the period OC
+        if (q.y2) q.y2 += row0;
+        q.M = (r1 - r0) * OC; q.N = T_in; q.K = (ra < 0 ? 3 : 2) * IC;
+        q.conv_ic = IC; q.conv_iw = T_in; q.conv_ow = T_in; q.conv_p = ra < 0 || !g ? 1 : 0;
+        const int rc = hipcheck(launch_gemm_split(q, s), "vae split transposed conv");
         if (rc) return rc;
     }
     return TSK_OK;
@@ -303,10 +302,9 @@ extern "C" void tsk_vae_destroy(tsk_vae *v) {
     for (float *a : v->act)
         if (a) (void) hipFree(a);
     if (v->lat) (void) hipFree(v->lat);
-    if (v->blob16) (void) hipFree(v->blob16);
-    for (uint16_t *a : v->ap)
-        if (a) (void) hipFree(a);
-    if (v->latp) (void) hipFree(v->latp);
+    if (v->wexp) (void) hipFree(v->wexp);
+    if (v->slots) (void) hipFree(v->slots);
+    if (v->exps) (void) hipFree(v->exps);
     delete v;
 }
 
@@ -362,25 +360,21 @@ extern "C" int tsk_vae_create(const tsk_vae_config *cfg, tsk_vae **out) {
         off += (x.count + 63) & ~(size_t) 63;
     }
     v->act_cap = (size_t) c.max_latent * (size_t) max_ch_t;
-    // split products (opt-in) when every convolution's channels fit the
-    // cooperative bf16 GEMM's 64-wide stages over 3 IC (the final k7 stays
-    // fp32 products). The decoder amplifies a product's relative error about
-    // 50-100 times on its way to the audio: split products (~2^-17 per term)
-    // leave the audio ~5e-4 rel-L2 from fp32 products (fp32 ones: ~6e-5 from
-    // an fp64 decode), 1.6-1.7 times faster
-    v->split = tuning().vae_split && c.latent_dim % 64 == 0;
+    // split products need whole 32-channel groups in every tensor a convolution
+    // reads or writes but the final k7's, and 31-bit byte offsets into a kernel
+    v->split = c.latent_dim % 32 == 0;
     for (int n = 0; n < 5; ++n) {
         int ci, co, st;
         block_dims(c, n, &ci, &co, &st);
-        v->split = v->split && ci % 64 == 0 && co % 64 == 0;
+        v->split = v->split && ci % 32 == 0 && co % 32 == 0;
     }
-    size_t off16 = 0;
-    if (v->split)
-        for (auto &x : v->w)
-            if ((x.conv || x.ct) && x.name != "decoder.layers.7.weight") {
-                x.offset16 = off16;
-                off16 += (3 * x.count + 127) & ~(size_t) 127;
-            }
+    size_t nexp = 0;
+    for (auto &x : v->w)
+        if ((x.conv || x.ct) && x.name != "decoder.layers.7.weight") {
+            v->split = v->split && sizeof(float) * x.count < ((size_t) 1 << 31);
+            x.woffset = nexp;
+            nexp += (size_t) (x.ct ? x.stride : 1) * x.ne[2];
+        }
     auto alloc = [&](void **p, size_t bytes) -> int {
         hipError_t e = hipMalloc(p, bytes);
         if (e != hipSuccess) return fail(TSK_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
@@ -391,14 +385,14 @@ extern "C" int tsk_vae_create(const tsk_vae_config *cfg, tsk_vae **out) {
         (rc = alloc((void **) &v->act[1], sizeof(float) * v->act_cap)) ||
         (rc = alloc((void **) &v->act[2], sizeof(float) * v->act_cap)) ||
         (rc = alloc((void **) &v->lat, sizeof(float) * (size_t) c.max_latent * c.latent_dim)) ||
-        (v->split && ((rc = alloc((void **) &v->blob16, 2 * off16)) ||
-                      (rc = alloc((void **) &v->ap[0], 6 * v->act_cap)) ||
-                      (rc = alloc((void **) &v->ap[1], 6 * v->act_cap)) ||
-                      (rc = alloc((void **) &v->latp, 6 * (size_t) c.max_latent * c.latent_dim))))) {
+        (v->split && ((rc = alloc((void **) &v->wexp, sizeof(int) * nexp)) ||
+                      (rc = alloc((void **) &v->slots, sizeof(float) * VAE_SLOTS)) ||
+                      (rc = alloc((void **) &v->exps, sizeof(int) * (VAE_CONVS + 1)))))) {
         tsk_vae_destroy(v);
         return rc;
     }
     hipError_t e = hipMemset(v->blob, 0, sizeof(float) * off);
+    if (e == hipSuccess && v->split) e = hipMemset(v->wexp, 0, sizeof(int) * nexp);
     if (e != hipSuccess) { tsk_vae_destroy(v); return hip_fail(e, "vae init"); }
     *out = v;
     return TSK_OK;
@@ -421,13 +415,14 @@ extern "C" int tsk_vae_set_tensor(tsk_vae *v, const char *name, const float *src
     if (!v || !name || !src) return fail(TSK_ERR_INVALID_ARG, "NULL argument");
     auto it = v->idx.find(name);
     if (it == v->idx.end()) return fail(TSK_ERR_INVALID_ARG, "unknown tensor '%s'", name);
-    const VW &x = v->w[it->second];
+    VW &x = v->w[it->second];
     const int64_t N = x.ne[0] * x.ne[1] * x.ne[2];
     if (n != N) return fail(TSK_ERR_SHAPE, "'%s' has %lld elements, got %lld", name, (long long) N, (long long) n);
     std::vector<float> t(x.count, 0.0f);
     const std::string nm = name;
     const bool is_alpha = nm.size() > 6 && nm.compare(nm.size() - 6, 6, ".alpha") == 0;
     const bool is_beta = nm.size() > 5 && nm.compare(nm.size() - 5, 5, ".beta") == 0;
+    x.amax = x.l1 = 0.0f;
     if (x.ct) {
         // merged 3-tap kernel: row r * OC + oc, tap j (input frame q - 1 + j),
         // channel ic = W'[oc][ic][k] for the phase's two taps k
@@ -454,35 +449,45 @@ extern "C" int tsk_vae_set_tensor(tsk_vae *v, const char *name, const float *src
         for (int64_t i = 0; i < n; ++i) t[i] = is_alpha ? expf(src[i]) : is_beta ? expf(-src[i]) : src[i];
     }
     hipError_t e = hipMemcpy(v->blob + x.offset, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess && v->split && (x.conv || x.ct) && x.name != "decoder.layers.7.weight") {
-        // the prepared rows in groups of IC -> [hi | lo | hi] per group,
-        // hi = bf16(w), lo = bf16(w - hi)
-        const size_t G = (size_t) x.ne[1];
-        std::vector<uint16_t> sp(3 * x.count);
-        for (size_t g0 = 0; g0 < x.count; g0 += G)
-            for (size_t i = 0; i < G; ++i) {
-                const float w = t[g0 + i];
-                const uint16_t hi = host_bf16_bits(w);
-                const uint32_t hb = (uint32_t) hi << 16;
-                float hf;
-                memcpy(&hf, &hb, 4);
-                uint16_t *d = &sp[3 * g0 + i];
-                d[0] = hi;
-                d[G] = std::isfinite(hf) ? host_bf16_bits(w - hf) : (uint16_t) 0;
-                d[2 * G] = hi;
+    if (v->split) {
+        for (float a : t) x.amax = std::max(x.amax, std::isfinite(a) ? std::fabs(a) : 0.0f);
+        if ((x.conv || x.ct) && nm != "decoder.layers.7.weight") {
+            // the row bounds, and the rows split in place
+            const size_t rows = (size_t) (x.ct ? x.stride : 1) * x.ne[2], K = t.size() / rows;
+            for (size_t r = 0; r < rows; ++r) {
+                float l1 = 0.0f;
+                for (size_t k = 0; k < K; ++k) l1 += std::isfinite(t[r * K + k]) ? std::fabs(t[r * K + k]) : 0.0f;
+                x.l1 = std::max(x.l1, l1);
             }
-        e = hipMemcpy(v->blob16 + x.offset16, sp.data(), 2 * sp.size(), hipMemcpyHostToDevice);
+            if (e == hipSuccess)
+                e = launch_split_rows(v->blob + x.offset, (int64_t) K, (int64_t) rows, (int) K,
+                                      (uint32_t *) (v->blob + x.offset), v->wexp + x.woffset, nullptr);
+            if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+        }
     }
     return hipcheck(e, "vae set_tensor copy");
 }
 
 namespace {
 
+// conv k7 (no bias) of the final snake sx [frames][C] -> planar audio
+// [out_channels][frames]: the stream-per-wave kernel for 128 -> 2 channels, else
+// the GEMM's rows [frames][out_channels] (t) and a transpose
+int decode_out(const tsk_vae *v, const float *sx, float *t, int C, int64_t frames, float *audio_d, hipStream_t st) {
+    const tsk_vae_config &c = v->cfg;
+    const VW &wf = wi(v, "decoder.layers.7.weight");
+    if (C == 128 && wf.ne[0] == 7 && c.out_channels == 2)
+        return hipcheck(launch_conv_small_oc(sx, (int) frames, C, 7, 2, wp(v, "decoder.layers.7.weight"), nullptr, 3,
+                                             audio_d, frames, st),
+                        "vae final convolution");
+    const int rc = conv(v, "decoder.layers.7", false, sx, C, (int) frames, 3, 1, t, false, st);
+    if (rc) return rc;
+    return hipcheck(launch_transpose_ct(t, 1, (int) frames, c.out_channels, audio_d, st), "vae audio");
+}
+
 int decode_impl(tsk_vae *v, int T, const float *latent_d, float *audio_d, hipStream_t st) {
     const tsk_vae_config &c = v->cfg;
     int rc;
-    // latent ne = [T, latent_dim] (time fastest) -> rows [T][latent_dim]
-    if ((rc = hipcheck(launch_transpose_ct(latent_d, 1, c.latent_dim, T, v->lat, st), "vae latent"))) return rc;
     // Every SnakeBeta runs in the epilogue of the convolution that produces
     // its input: x (buffer 0) holds the residual stream, sx (buffer 1 or 2)
     // the snake of x that the next convolution reads, t the other one. A
@@ -490,52 +495,49 @@ int decode_impl(tsk_vae *v, int T, const float *latent_d, float *audio_d, hipStr
     float *x = v->act[0], *sx = v->act[1], *t = v->act[2];
     int in0, out0, s0;
     block_dims(c, 0, &in0, &out0, &s0);
-    if (v->split && tuning().vae_split) {
-        // the same chain on split products: each snake written as the split
-        // planes the next convolution reads (sp, then tp), the residual
-        // stream x f32, the final snake f32 (sx) for the output convolution
-        uint16_t *sp = v->ap[0], *tp = v->ap[1];
-        if ((rc = hipcheck(launch_cast_rows_split3(v->lat, c.latent_dim, 0, T, T, c.latent_dim, v->latp, st),
-                           "vae latent planes")) ||
-            (rc = conv_split(v, "decoder.layers.0", v->latp, c.latent_dim, T, 3, 1,
-                             SplitOut{nullptr, false, "decoder.layers.1.layers.0", in0, nullptr, sp}, st)))
+    if (v->split) {
+        // the latent's exponent and rows, then the chain on split rows (the
+        // residual stream x f32, the final snake f32 in sx)
+        if ((rc = hipcheck(launch_split_begin(latent_d, (int64_t) T * c.latent_dim, v->slots, VAE_SLOTS, v->exps, st),
+                           "vae latent")) ||
+            (rc = hipcheck(launch_split_transpose(latent_d, c.latent_dim, T, v->exps, (uint32_t *) v->lat, st),
+                           "vae latent")) ||
+            (rc = conv_split(v, "decoder.layers.0", c.latent_dim, T, 3, 1,
+                             SplitStep{0, v->lat, nullptr, -1, "decoder.layers.1.layers.0", in0, sx, false}, st)))
             return rc;
         int64_t fr = T;
-        int Cs = in0;
+        int i = 1, res = 0, Cs = in0;                        // next convolution; the one that wrote x last
         const int dl[3] = {1, 3, 9};
         for (int n = 0; n < 5; ++n) {
             int ci, co, s;
             block_dims(c, n, &ci, &co, &s);
             const std::string bp = "decoder.layers." + std::to_string(n + 1);
-            const std::string sn0 = bp + ".layers.2.layers.0";
-            if ((rc = conv_t_split(v, bp + ".layers.1", sp, ci, (int) fr,
-                                   SplitOut{x, false, sn0.c_str(), co, nullptr, tp}, st)))
+            if ((rc = conv_t_split(v, bp + ".layers.1", ci, (int) fr,
+                                   SplitStep{i, sx, x, -1, bp + ".layers.2.layers.0", co, t, false}, st)))
                 return rc;
-            std::swap(sp, tp);
+            std::swap(sx, t);
+            res = i++;
             fr *= s;
             Cs = co;
             for (int r = 0; r < 3; ++r) {
-                const std::string rp = bp + ".layers." + std::to_string(r + 2), sn = rp + ".layers.2";
-                if ((rc = conv_split(v, rp + ".layers.1", sp, Cs, (int) fr, 3 * dl[r], dl[r],
-                                     SplitOut{nullptr, false, sn.c_str(), Cs, nullptr, tp}, st)))
-                    return rc;
+                const std::string rp = bp + ".layers." + std::to_string(r + 2);
                 const bool last = n == 4 && r == 2;
                 const std::string np = r < 2 ? bp + ".layers." + std::to_string(r + 3) + ".layers.0"
                                      : n < 4 ? "decoder.layers." + std::to_string(n + 2) + ".layers.0"
                                              : std::string("decoder.layers.6");
-                if ((rc = conv_split(v, rp + ".layers.3", tp, Cs, (int) fr, 0, 1,
-                                     SplitOut{x, true, np.c_str(), Cs, last ? sx : nullptr, last ? nullptr : sp}, st)))
+                if ((rc = conv_split(v, rp + ".layers.1", Cs, (int) fr, 3 * dl[r], dl[r],
+                                     SplitStep{i, sx, nullptr, -1, rp + ".layers.2", Cs, t, false}, st)) ||
+                    (rc = conv_split(v, rp + ".layers.3", Cs, (int) fr, 0, 1,
+                                     SplitStep{i + 1, t, x, res, np, Cs, sx, last}, st)))
                     return rc;
+                res = i + 1;
+                i += 2;
             }
         }
-        const VW &wf7 = wi(v, "decoder.layers.7.weight");
-        if (Cs == 128 && wf7.ne[0] == 7 && c.out_channels == 2)
-            return hipcheck(launch_conv_small_oc(sx, (int) fr, Cs, 7, 2, wp(v, "decoder.layers.7.weight"), nullptr, 3,
-                                                 audio_d, fr, st),
-                            "vae final convolution");
-        if ((rc = conv(v, "decoder.layers.7", false, sx, Cs, (int) fr, 3, 1, t, false, st))) return rc;
-        return hipcheck(launch_transpose_ct(t, 1, (int) fr, c.out_channels, audio_d, st), "vae audio");
+        return decode_out(v, sx, t, Cs, fr, audio_d, st);
     }
+    // latent ne = [T, latent_dim] (time fastest) -> rows [T][latent_dim]
+    if ((rc = hipcheck(launch_transpose_ct(latent_d, 1, c.latent_dim, T, v->lat, st), "vae latent"))) return rc;
     // conv k7 -> snake of block 1 (the conv's own output is not used again)
     F32Snake sk = snake_epi(v, "decoder.layers.1.layers.0", in0, nullptr);
     if ((rc = conv(v, "decoder.layers.0", true, v->lat, c.latent_dim, T, 3, 1, sx, false, st, &sk))) return rc;
@@ -566,16 +568,7 @@ int decode_impl(tsk_vae *v, int T, const float *latent_d, float *audio_d, hipStr
             if ((rc = conv(v, rp + ".layers.3", true, t, C, (int) frames, 0, 1, x, true, st, &sk))) return rc;
         }
     }
-    // conv k7 (no bias) of the final snake -> planar audio [out_channels][T_audio]:
-    // the stream-per-wave kernel for 128 -> 2 channels, else the GEMM's rows
-    // [T_audio][out_channels] and a transpose
-    const VW &wf = wi(v, "decoder.layers.7.weight");
-    if (C == 128 && wf.ne[0] == 7 && c.out_channels == 2)
-        return hipcheck(launch_conv_small_oc(sx, (int) frames, C, 7, 2, wp(v, "decoder.layers.7.weight"), nullptr, 3,
-                                             audio_d, frames, st),
-                        "vae final convolution");
-    if ((rc = conv(v, "decoder.layers.7", false, sx, C, (int) frames, 3, 1, t, false, st))) return rc;
-    return hipcheck(launch_transpose_ct(t, 1, (int) frames, c.out_channels, audio_d, st), "vae audio");
+    return decode_out(v, sx, t, C, frames, audio_d, st);
 }
 
 }  // namespace
