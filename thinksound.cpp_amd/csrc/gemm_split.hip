@@ -113,12 +113,21 @@ __device__ __forceinline__ float f32_dot(const SplitGemm &p, int m, int n, int k
     return s;
 }
 
+// UNIT: a residual unit of the VAE in one launch where its channels fit one
+// tile (M <= 128, M % 32 == 0): the tile's convolution, bias and SnakeBeta stay in
+// the workgroup (split at the tile's own exponent into the ring's LDS, in the
+// layout of M / 32 activation steps) and are the operand of the k1 convolution
+// (w2, its fragments straight from L2 into registers). As two launches the
+// k1's was bound by its four passes over the activations (30 s, 128 channels,
+// 1.3 M frames: 980 + 790 us); one launch reads the snake once and writes the
+// residual and the next snake.
+//
 // Workgroup = 2 x 2 waves of TM x TN 16x16 tiles; operand lines by direct
 // global -> LDS loads into a two-stage ring of 32-wide K steps (line chunk c of
 // a row at slot c ^ ((row / 2) % 8): the 16 rows of a fragment read hit
 // distinct banks). Per step and 64 x 64 wave tile: 16 16-byte LDS reads for 48
 // MFMAs of 16 cycles; two workgroups per CU.
-template <int TM, int TN, bool SNAKE>
+template <int TM, int TN, bool SNAKE, bool UNIT>
 __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int ROWS = BM + BN, STAGE = ROWS * BK;          // words per stage
@@ -278,8 +287,120 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
             for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
     }
 
+    int mid_e = 0;
+    if constexpr (UNIT) {
+        __shared__ float red[4];
+        const int ns = p.M / BK;
+        // second weights, row m's step s: hi at chunk lg, lo at chunk 4 + lg (rows past M: the last one)
+        f16x8 ah[2][TM], al[2][TM];
+        const uint32_t *wr[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            wr[i] = p.w2 + (int64_t) min((wm * TM + i) * 16 + lr, p.M - 1) * p.M + 4 * lg;
+            ah[0][i] = *(const f16x8 *) wr[i];
+            al[0][i] = *(const f16x8 *) (wr[i] + 16);
+        }
+        // this lane's four channels of a token: bias, SnakeBeta
+        float tm_ = 0.0f;
+        const int xe = *p.xe - 30;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int mc = min((wm * TM + i) * 16 + 4 * lg, p.M - 4);
+            const i32x4 we = *(const i32x4 *) (p.we + mc);
+            const f32x4 mb = *(const f32x4 *) (p.mid_bias + mc), me = *(const f32x4 *) (p.mid_ea + mc),
+                        mf = *(const f32x4 *) (p.mid_eb + mc);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                float v[4], ar[4], s2[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    v[r] = __builtin_ldexpf(acc[i][j][r], xe + we[r]) + mb[r];
+                    ar[r] = v[r] * me[r];
+                }
+                sin2_x4(ar, s2);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    acc[i][j][r] = v[r] + s2[r] * mf[r];
+                    if (finite_f(acc[i][j][r])) tm_ = fmaxf(tm_, fabsf(acc[i][j][r]));
+                }
+            }
+        }
+        tm_ = wave_max(tm_);
+        if (lane == 0) red[wave] = tm_;
+        __syncthreads();                                      // also: the ring's last reads are done
+        mid_e = bound_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+        const float scale = exp2_int(15 - mid_e);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int mc = (wm * TM + i) * 16 + 4 * lg, c = (mc & 31) >> 3;
+            float *st = smem + (mc >> 5) * (BN * BK) + ((mc & 7) >> 1);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int row = (wn * TN + j) * 16 + lr;
+                const float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+                f16x4 hi, lo;
+                split4(v, scale, hi, lo);
+                if (mc < p.M) {
+                    *(f16x4 *) &st[at(row, c)] = hi;
+                    *(f16x4 *) &st[at(row, 4 + c)] = lo;
+                }
+                acc[i][j] = f32x4{0, 0, 0, 0};
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < BM / BK; ++t) {
+            if (t >= ns) break;
+            if (t + 1 < ns) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    ah[(t + 1) & 1][i] = *(const f16x8 *) (wr[i] + 32 * (t + 1));
+                    al[(t + 1) & 1][i] = *(const f16x8 *) (wr[i] + 32 * (t + 1) + 16);
+                }
+            }
+            const float *st = smem + t * (BN * BK);
+            f16x8 bh[TN], bl[TN];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                bh[j] = *(const f16x8 *) &st[at((wn * TN + j) * 16 + lr, lg)];
+                bl[j] = *(const f16x8 *) &st[at((wn * TN + j) * 16 + lr, 4 + lg)];
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t & 1][i], bh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t & 1][i], bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t & 1][i], bh[j], acc[i][j], 0, 0, 0);
+        }
+    }
+
     // ---- epilogue: the accumulators as the workgroup's [BN][BM] tile in LDS,
     // then four consecutive outputs of one token per thread
+    constexpr int G = BM / 4;
+    static_assert(NT % G == 0, "fixed channel group per thread");
+    const int ml = (tid % G) * 4, m0 = bm0 + ml;
+    const bool mok = m0 < p.M;                                // M % 4 == 0: all four or none
+    // the old rows of a residual update, eight at a time and the first ones
+    // before the tile is staged: read one by one, each waits for memory
+    constexpr int STEP = NT / G, ITER = BN / STEP, NB = 8;
+    static_assert(ITER % NB == 0, "whole batches of rows");
+    f32x4 old[NB];
+    auto load_old = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            const int n = bn0 + tid / G + (b * NB + u) * STEP;
+            old[u] = f32x4{0, 0, 0, 0};
+            if (n < p.N && mok) old[u] = *(const f32x4 *) ((const float *) p.y + (int64_t) n * p.ld_y + m0);
+        }
+    };
+    if constexpr (SNAKE)
+        if (p.accumulate) load_old(0);
     __syncthreads();                                          // the ring's last reads are done
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -287,10 +408,6 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
         for (int j = 0; j < TN; ++j)
             *(f32x4 *) &smem[((wn * TN + j) * 16 + lr) * LDT + (wm * TM + i) * 16 + 4 * lg] = acc[i][j];
     __syncthreads();
-    constexpr int G = BM / 4;
-    static_assert(NT % G == 0, "fixed channel group per thread");
-    const int ml = (tid % G) * 4, m0 = bm0 + ml;
-    const bool mok = m0 < p.M;                                // M % 4 == 0: all four or none
     float bv[4] = {0, 0, 0, 0}, ea[4], eb[4];
     int we[4] = {0, 0, 0, 0};
     float oscale = 0.0f, ym = 0.0f, sm = 0.0f;
@@ -298,7 +415,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if (p.bias) bv[r] = p.bias[m0 + r];
-            we[r] = p.we[m0 + r] - 30;
+            we[r] = (UNIT ? p.we2 : p.we)[m0 + r] - 30;
         }
         if constexpr (SNAKE) {
             const int c0 = m0 % p.period;                     // period % 4 == 0: c0 + 3 < period
@@ -313,7 +430,9 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
         if (p.yp) {
             // |y| <= sum |w| max |x| + max |bias| (+ max |old y|), |snake(y)| <= |y| + max eb
             // (l1 and badd hold these maxima and 1 % for the roundings)
-            float bound = p.l1 * *p.amax_x + p.badd;
+            float bound = *p.amax_x;
+            if constexpr (UNIT) bound = p.mid_l1 * bound + p.mid_badd;
+            bound = p.l1 * bound + p.badd;
             if (p.amax_old) bound += 1.01f * *p.amax_old;
             const int eo = bound_exp(bound);
             oscale = exp2_int(15 - eo);
@@ -321,11 +440,16 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
         }
     }
     const int k_lo = kt0 * BK, k_hi = (kt0 + nk) * BK;
-    for (int nl = tid / G; nl < BN; nl += NT / G) {
-        const int n = bn0 + nl;
-        if (n >= p.N || !mok) break;
+#pragma unroll 1
+    for (int b = 0; b < ITER / NB; ++b) {
+    if constexpr (SNAKE)
+        if (p.accumulate && b) load_old(b);
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int nl = tid / G + (b * NB + u) * STEP, n = bn0 + nl;
+        if (n >= p.N || !mok) continue;
         const f32x4 a4 = *(const f32x4 *) &smem[nl * LDT + ml];
-        const int xe = p.xe[p.xe_per_row ? n : 0];
+        const int xe = UNIT ? mid_e : p.xe[p.xe_per_row ? n : 0];
         float o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -346,9 +470,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
             if (p.y) {
                 float *yr = (float *) p.y + (int64_t) n * p.ld_y + m0;
                 if (p.accumulate) {
-                    const f32x4 old = *(const f32x4 *) yr;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) o[r] = old[r] + o[r];
+                    for (int r = 0; r < 4; ++r) o[r] = old[u][r] + o[r];
                 }
                 *(f32x4 *) yr = f32x4{o[0], o[1], o[2], o[3]};
 #pragma unroll
@@ -373,6 +496,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
             }
         }
     }
+    }
     if constexpr (SNAKE) {
         ym = wave_max(ym);
         sm = wave_max(sm);
@@ -385,8 +509,9 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
 
 template <int TM, int TN>
 void launch_split_tiles(const SplitGemm &p, int grid, hipStream_t s) {
-    if (p.ea) launch_kernel((gemm_split_kernel<TM, TN, true>), dim3(grid), dim3(NT), 0, s, p);
-    else launch_kernel((gemm_split_kernel<TM, TN, false>), dim3(grid), dim3(NT), 0, s, p);
+    if (p.w2) launch_kernel((gemm_split_kernel<TM, TN, true, true>), dim3(grid), dim3(NT), 0, s, p);
+    else if (p.ea) launch_kernel((gemm_split_kernel<TM, TN, true, false>), dim3(grid), dim3(NT), 0, s, p);
+    else launch_kernel((gemm_split_kernel<TM, TN, false, false>), dim3(grid), dim3(NT), 0, s, p);
 }
 
 // one workgroup: max |x| over n values into slot[0] and its exponent into
@@ -474,6 +599,8 @@ hipError_t launch_gemm_split(SplitGemm &p, hipStream_t s) {
         return hipErrorInvalidValue;
     if (p.ea && (p.period < 4 || p.period % 4 || p.M % p.period || p.splits != 1 || p.y_bf16 || (!p.yp && !p.y2) ||
                  (p.yp && (p.ld_y % 32 || p.period % 32 || !p.amax_x || !p.e_out))))
+        return hipErrorInvalidValue;
+    if (p.w2 && (!p.ea || !p.y || p.M % 32 || p.M > 128 || !p.we2 || !p.mid_bias || !p.mid_ea || !p.mid_eb || p.xe_per_row))
         return hipErrorInvalidValue;
     if (!p.ea && (!p.y || !p.xf || !p.wf || p.accumulate || (p.splits > 1 && (p.bias || p.y_bf16))))
         return hipErrorInvalidValue;

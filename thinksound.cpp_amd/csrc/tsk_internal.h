@@ -439,6 +439,13 @@ struct SplitGemm {
     const float *amax_x, *amax_old;
     int *e_out;
     float *amax_y, *amax_s;
+    // residual unit (w2 non-null; M <= 128, M % 32): a second, k1 convolution of the
+    // SnakeBeta (mid_*) of the first one; bias, ea, eb, y, l1, badd are the second's.
+    // The first's output is bounded by mid_l1 * *amax_x + mid_badd
+    const uint32_t *w2;            // [M][M] split rows
+    const int *we2;
+    const float *mid_bias, *mid_ea, *mid_eb;   // [M]
+    float mid_l1, mid_badd;
     // set by the launcher
     int tiles_m, tiles_n, deal;
     int64_t x_rows;

@@ -243,6 +243,30 @@ int conv_split(const tsk_vae *v, const std::string &p, int IC, int T_in, int pad
     return hipcheck(launch_gemm_split(q, s), "vae split conv");
 }
 
+// a residual unit of at most 128 channels (convolutions i and i + 1 of t) in one launch
+int unit_split(const tsk_vae *v, const std::string &rp, int C, int T, int dil, const SplitStep &t, hipStream_t s) {
+    const VW &w1 = wi(v, rp + ".layers.1.weight"), &w2 = wi(v, rp + ".layers.3.weight");
+    const VW &b1 = wi(v, rp + ".layers.1.bias"), &eb1 = wi(v, rp + ".layers.2.beta");
+    const int KW = (int) w1.ne[0];
+    SplitStep last = t;
+    last.i = t.i + 1;
+    SplitGemm q = split_gemm(v, rp + ".layers.3", last, C);
+    q.w2 = q.w; q.we2 = q.we;
+    q.w = (const uint32_t *) (v->blob + w1.offset);
+    q.we = v->wexp + w1.woffset;
+    q.xe = v->exps + t.i;
+    q.amax_x = v->slots + 2 * t.i;
+    q.mid_bias = v->blob + b1.offset;
+    q.mid_ea = wp(v, rp + ".layers.2.alpha"); q.mid_eb = v->blob + eb1.offset;
+    q.mid_l1 = 1.01f * w1.l1; q.mid_badd = 1.01f * (b1.amax + eb1.amax);
+    q.l1 = 1.01f * w2.l1;
+    q.ld_w = (int64_t) KW * C;
+    q.ld_y = C;
+    q.M = C; q.N = T; q.K = KW * C;
+    q.conv_ic = C; q.conv_iw = T; q.conv_ow = T; q.conv_p = dil * (KW / 2); q.conv_d = dil;
+    return hipcheck(launch_gemm_split(q, s), "vae residual unit");
+}
+
 // the transposed convolution of conv_t: the merged kernel's two-tap phase groups
 int conv_t_split(const tsk_vae *v, const std::string &p, int IC, int T_in, const SplitStep &t, hipStream_t s) {
     const VW &w = wi(v, p + ".weight");
@@ -525,11 +549,16 @@ int decode_impl(tsk_vae *v, int T, const float *latent_d, float *audio_d, hipStr
                 const std::string np = r < 2 ? bp + ".layers." + std::to_string(r + 3) + ".layers.0"
                                      : n < 4 ? "decoder.layers." + std::to_string(n + 2) + ".layers.0"
                                              : std::string("decoder.layers.6");
-                if ((rc = conv_split(v, rp + ".layers.1", Cs, (int) fr, 3 * dl[r], dl[r],
+                if (Cs <= 128) {
+                    if ((rc = unit_split(v, rp, Cs, (int) fr, dl[r], SplitStep{i, sx, x, res, np, Cs, t, last}, st)))
+                        return rc;
+                    std::swap(sx, t);
+                } else if ((rc = conv_split(v, rp + ".layers.1", Cs, (int) fr, 3 * dl[r], dl[r],
                                      SplitStep{i, sx, nullptr, -1, rp + ".layers.2", Cs, t, false}, st)) ||
-                    (rc = conv_split(v, rp + ".layers.3", Cs, (int) fr, 0, 1,
-                                     SplitStep{i + 1, t, x, res, np, Cs, sx, last}, st)))
+                           (rc = conv_split(v, rp + ".layers.3", Cs, (int) fr, 0, 1,
+                                            SplitStep{i + 1, t, x, res, np, Cs, sx, last}, st))) {
                     return rc;
+                }
                 res = i + 1;
                 i += 2;
             }
