@@ -57,3 +57,89 @@ def test_vae_split_nan_stays_local(vae):
     assert np.isnan(a[:, :2048]).all()
     far = slice(20 * 2048, None)
     assert np.isfinite(a[:, far]).all() and rel_l2(a[:, far], ref[:, far]) <= 2e-4
+
+
+# ---------------------------------------------------------------- F32 nodes
+def rows_close(got, w, x, bound):
+    """every output row against 64-bit products, relative to |w| |x| of its own row (its sum's condition):
+    operands to 2^-23, the products left out 2^-22, both with random signs, and sums of K terms in fp32"""
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = np.sqrt(((np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T) ** 2).sum(-1))
+    err = np.sqrt(((got - ref) ** 2).sum(-1)) / np.maximum(scale, 1e-300)
+    print(f"rows: max error / |x||w| {err.max():.2e}", flush=True)
+    return err.max() <= bound
+
+
+@pytest.mark.parametrize("N,K,M", [(1, 448, 4), (63, 480, 132), (65, 1024, 128), (129, 2080, 64), (388, 4096, 96),
+                                   (600, 512, 1028)])
+def test_mul_mat_split(env, N, K, M):
+    """remainders of every tile and of the K slices; rows and weights of very different size keep their own precision"""
+    tsk, _ = env
+    rng = np.random.default_rng(N + K)
+    x = (rng.standard_normal((N, K)) * 2.0 ** rng.integers(-40, 40, (N, 1))).astype(np.float32)
+    w = (rng.standard_normal((M, K)) * 2.0 ** rng.integers(-20, 20, (M, 1))).astype(np.float32)
+    y = tsk.mul_mat(tsk.to_device(w), tsk.to_device(x)).numpy()
+    scale = 2.0 ** np.floor(np.log2(np.abs(w).max(-1)))           # columns to one size: an error of a small one shows
+    assert rows_close(y / scale, w / scale[:, None], x, 2.0 ** -22)
+
+
+@pytest.mark.parametrize("B,IW,IC,OC,KW,s0,p0,d0", [(2, 65, 160, 36, 3, 1, 1, 1), (3, 31, 96, 128, 7, 2, 3, 2),
+                                                    (1, 130, 512, 64, 1, 1, 0, 1), (2, 40, 256, 8, 3, 1, 4, 1)])
+def test_conv1d_split(env, B, IW, IC, OC, KW, s0, p0, d0):
+    """one output sums input rows of different exponents: steps of 2^30 and more between neighbours, zero rows
+    between them, batch items that must not see each other, padding wider than the kernel"""
+    tsk, _ = env
+    rng = np.random.default_rng(IW + OC)
+    e = rng.integers(-35, 35, (B, IW, 1))
+    x = (rng.standard_normal((B, IW, IC)) * 2.0 ** e).astype(np.float32)
+    x[:, 5:8] = 0
+    x[0, 20] *= 2.0 ** -60
+    w = (rng.standard_normal((OC, IC, KW)) * 0.05).astype(np.float32)
+    y = tsk.conv1d(tsk.to_device(w), tsk.to_device(x), None, s0, p0, d0).numpy().reshape(B, -1, OC)
+    xp = np.zeros((B, IW + 2 * p0, IC), np.float32)
+    xp[:, p0:p0 + IW] = x
+    OW = (IW + 2 * p0 - d0 * (KW - 1) - 1) // s0 + 1
+    cols = np.stack([xp[:, k * d0:k * d0 + (OW - 1) * s0 + 1:s0] for k in range(KW)], 2).reshape(B * OW, KW * IC)
+    assert rows_close(y.reshape(B * OW, OC), w.transpose(0, 2, 1).reshape(OC, -1), cols, 2.0 ** -22)
+
+
+def test_split_infinities(env):
+    """infinities and NaN give what fp32 products give, and only in the rows and columns that hold them"""
+    tsk, _ = env
+    rng = np.random.default_rng(2)
+    x, w = rng.standard_normal((70, 512)).astype(np.float32), rng.standard_normal((64, 512)).astype(np.float32)
+    clean = tsk.mul_mat(tsk.to_device(w), tsk.to_device(x)).numpy()
+    # 1e37: its products (|w| < 6) and their sums stay below fp32's 3.4e38, so that
+    # only the infinities make infinities, in fp32 as in 64 bits
+    x[3, 7], x[4, 9], w[5, 11], x[6, 0] = np.inf, np.nan, -np.inf, 1e37
+    y = tsk.mul_mat(tsk.to_device(w), tsk.to_device(x)).numpy()
+    with np.errstate(all="ignore"):
+        ref = (x[:, None, :].astype(np.float64) * w[None]).sum(-1)
+    assert np.array_equal(np.isnan(y), np.isnan(ref))
+    odd = ~np.isfinite(ref)
+    assert np.array_equal(y[odd & ~np.isnan(ref)], ref[odd & ~np.isnan(ref)].astype(np.float32))
+    same = np.ones_like(odd)
+    same[[3, 4, 6]] = False
+    same[:, 5] = False
+    assert np.array_equal(y[same], clean[same])
+
+
+def test_split_without_scratch(env):
+    """a bound workspace too small for the split products: fp32 products, as before"""
+    tsk, orc = env
+    rng = np.random.default_rng(3)
+    x, w = rng.standard_normal((100, 512)).astype(np.float32), rng.standard_normal((64, 512)).astype(np.float32)
+    xd, wd, y = tsk.to_device(x), tsk.to_device(w), tsk.empty((100, 64))
+    n = tsk.workspace_size(tsk.OP_MUL_MAT, [wd, xd], y)
+    s = tsk.Stream()
+    outs = []
+    for size in (n, n - 256):
+        buf = tsk.empty((size,), "u8")
+        tsk.set_workspace(buf, stream=s)
+        tsk.mul_mat(wd, xd, out=y, stream=s)
+        s.synchronize()
+        outs.append(y.numpy())
+        assert rel_l2(outs[-1], orc.mul_mat(w, x)) <= 1e-5
+    assert not np.array_equal(*outs)                              # two sets of products
+    tsk.set_workspace(None, stream=s)
+    s.destroy()

@@ -19,6 +19,8 @@
 // Layout: a row of C values (C % 32 == 0) is C 4-byte words in groups of 32 values, one
 // 128-byte line each: [32 hi][32 lo]. So rows, strides and bytes are those of
 // the f32 rows, and a 32-wide K step of a row is one line.
+#include <algorithm>
+
 #include "tsk_common.h"
 #include "tsk_internal.h"
 #include "tsk_runtime.h"
@@ -99,7 +101,7 @@ __device__ __forceinline__ void raise_slot(float *slot, float m) {
 // |s| < 2^15). The f32 operands give what fp32 products give.
 __device__ __forceinline__ float f32_dot(const SplitGemm &p, int m, int n, int k0, int k1) {
     float s = 0.0f;
-    const float *w = p.wf + (int64_t) m * p.ld_wf;
+    const float *w = m < p.wf_rows ? p.wf + (int64_t) m * p.ld_wf : p.wf2 + (int64_t) (m - p.wf_rows) * p.ld_wf;
     if (p.conv_ic) {
         const int b = n / p.conv_ow, o = n - b * p.conv_ow;
         for (int k = k0; k < k1; ++k) {
@@ -127,8 +129,8 @@ __device__ __forceinline__ float f32_dot(const SplitGemm &p, int m, int n, int k
 // a row at slot c ^ ((row / 2) % 8): the 16 rows of a fragment read hit
 // distinct banks). Per step and 64 x 64 wave tile: 16 16-byte LDS reads for 48
 // MFMAs of 16 cycles; two workgroups per CU.
-template <int TM, int TN, bool SNAKE, bool UNIT>
-__global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
+template <int TM, int TN, int WPC, bool SNAKE, bool UNIT>
+__global__ __launch_bounds__(NT, WPC) void gemm_split_kernel(const SplitGemm p) {
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int ROWS = BM + BN, STAGE = ROWS * BK;          // words per stage
     constexpr int NWL = ROWS / 8, WLW = NWL / 4;             // wave-loads (8 rows) per stage, per wave
@@ -137,29 +139,19 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
     constexpr int RING = 2 * STAGE, EPI_F = BN * LDT;
     __shared__ __attribute__((aligned(16))) float smem[RING > EPI_F ? RING : EPI_F];
 
-    // workgroup -> tile. L % 8 is the XCD: with deal 1 every m tile of a token
-    // tile runs on one XCD (its L2 fetches the activation rows once), with
-    // deal 2 every token tile of an (m tile, slice) pair (the weights once)
+    // workgroup -> tile. L % 8 is the XCD: each takes a consecutive eighth of
+    // the tiles in (slice, larger operand, smaller operand) order, so that the
+    // tiles it runs at one time share one K slice and a block of both operands
+    // in its L2
     int tm, tn, z;
     {
-        const int L = (int) blockIdx.x, q = L >> 3, S = p.splits;
-        if (p.deal == 1) {
-            const int t = (q / p.tiles_m) * 8 + (L & 7);
-            if (t >= p.tiles_n * S) return;
-            tm = q % p.tiles_m;
-            tn = t % p.tiles_n;
-            z = t / p.tiles_n;
-        } else if (p.deal == 2) {
-            const int t = (q / p.tiles_n) * 8 + (L & 7);
-            if (t >= p.tiles_m * S) return;
-            tn = q % p.tiles_n;
-            tm = t / S;
-            z = t % S;
-        } else {
-            tm = L % p.tiles_m;
-            tn = L / p.tiles_m % p.tiles_n;
-            z = L / (p.tiles_m * p.tiles_n);
-        }
+        const int L = (int) blockIdx.x, T = p.tiles_m * p.tiles_n;
+        const int u = (L & 7) * p.per_xcd + (L >> 3);
+        if (u >= T * p.splits) return;
+        z = u / T;
+        const int t = u - z * T;
+        tm = p.m_inner ? t % p.tiles_m : t / p.tiles_n;
+        tn = p.m_inner ? t / p.tiles_m : t % p.tiles_n;
     }
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -254,12 +246,54 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
     auto at = [](int row, int c) { return row * BK + ((c ^ ((row >> 1) & 7)) << 2); };
+    // Row exponents (xe_per_row): the accumulators are in units of the row that
+    // the current tap reads; a tap whose row has another exponent rescales them
+    // by a power of two (at most 2^60 either way, see split_rows_kernel). Rows
+    // in the padding change nothing.
+    constexpr int UNSET = -100000;
+    int ecur[TN], xrow[TN], xpos[TN], etap = 0, eleft = 0;
+    auto tap_exps = [&]() {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int iw = xpos[j] + etap * p.conv_d;
+            const bool in = !p.conv_ic || (iw >= 0 && iw < p.conv_iw);
+            const int e = in ? p.xe[p.conv_ic ? xrow[j] + iw : xrow[j]] : UNSET;
+            if (e == UNSET || e == ecur[j]) continue;
+            const float f = ecur[j] == UNSET ? 1.0f : exp2_int(ecur[j] - e);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][j][r] *= f;
+            ecur[j] = e;
+        }
+    };
+    if constexpr (!SNAKE) {
+        if (p.xe_per_row) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int n = min(bn0 + (wn * TN + j) * 16 + lr, p.N - 1);
+                const int b = p.conv_ic ? n / p.conv_ow : 0;
+                ecur[j] = UNSET;
+                xrow[j] = p.conv_ic ? b * p.conv_iw : n;
+                xpos[j] = p.conv_ic ? (n - b * p.conv_ow) * p.conv_s - p.conv_p : 0;
+            }
+            etap = p.conv_ic ? kw : 0;
+            eleft = p.conv_ic ? ic_left : nk;
+            tap_exps();
+        }
+    }
     if (nk > 0) issue(0);
     for (int it = 0; it < nk; ++it) {
+        if constexpr (!SNAKE) {
+            if (p.xe_per_row && eleft-- == 0) {
+                ++etap;
+                eleft = p.conv_ic / BK - 1;
+                tap_exps();
+            }
+        }
         // this wave's loads of the step have landed, then every wave's; the
         // barrier also ends every wave's reads of the other slot
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         if (it + 1 < nk) issue((it + 1) & 1);
         const float *st = smem + (it & 1) * STAGE;
         f16x8 ah[TM], al[TM], bh[TN], bl[TN];
@@ -401,6 +435,13 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
     };
     if constexpr (SNAKE)
         if (p.accumulate) load_old(0);
+    __shared__ int row_e[SNAKE ? 1 : BN];
+    if constexpr (!SNAKE) {
+        if (p.xe_per_row && wm == 0 && lg == 0) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) row_e[(wn * TN + j) * 16 + lr] = ecur[j] == UNSET ? 0 : ecur[j];
+        }
+    }
     __syncthreads();                                          // the ring's last reads are done
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -449,7 +490,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
         const int nl = tid / G + (b * NB + u) * STEP, n = bn0 + nl;
         if (n >= p.N || !mok) continue;
         const f32x4 a4 = *(const f32x4 *) &smem[nl * LDT + ml];
-        const int xe = UNIT ? mid_e : p.xe[p.xe_per_row ? n : 0];
+        const int xe = UNIT ? mid_e : !SNAKE && p.xe_per_row ? row_e[SNAKE ? 0 : nl] : p.xe[0];
         float o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -507,11 +548,15 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const SplitGemm p) {
     }
 }
 
-template <int TM, int TN>
-void launch_split_tiles(const SplitGemm &p, int grid, hipStream_t s) {
-    if (p.w2) launch_kernel((gemm_split_kernel<TM, TN, true, true>), dim3(grid), dim3(NT), 0, s, p);
-    else if (p.ea) launch_kernel((gemm_split_kernel<TM, TN, true, false>), dim3(grid), dim3(NT), 0, s, p);
-    else launch_kernel((gemm_split_kernel<TM, TN, false, false>), dim3(grid), dim3(NT), 0, s, p);
+template <int TM, int TN, int WPC>
+void launch_split_tiles(SplitGemm &p, hipStream_t s) {
+    p.tiles_m = (p.M + 32 * TM - 1) / (32 * TM);
+    p.tiles_n = (p.N + 32 * TN - 1) / (32 * TN);
+    p.per_xcd = (int) (((int64_t) p.tiles_m * p.tiles_n * p.splits + 7) / 8);
+    const int grid = 8 * p.per_xcd;
+    if (p.w2) launch_kernel((gemm_split_kernel<TM, TN, WPC, true, true>), dim3(grid), dim3(NT), 0, s, p);
+    else if (p.ea) launch_kernel((gemm_split_kernel<TM, TN, WPC, true, false>), dim3(grid), dim3(NT), 0, s, p);
+    else launch_kernel((gemm_split_kernel<TM, TN, WPC, false, false>), dim3(grid), dim3(NT), 0, s, p);
 }
 
 // one workgroup: max |x| over n values into slot[0] and its exponent into
@@ -549,48 +594,133 @@ __global__ __launch_bounds__(256) void split_transpose_kernel(const float *x, in
     store_split4(y + (int64_t) t * C, c, hi, lo);
 }
 
-// f32 rows -> split rows at their own exponents, one wave per row: the row's
-// maximum, then its groups (8 lanes each). In place works: a wave has loaded
-// all of a group before it writes it, and no other wave reads the row.
-__device__ __forceinline__ void split_row(const float *x, int cols, uint32_t *y, int *e) {
-    const int lane = threadIdx.x & 63;
+// f32 rows -> split rows at their own exponents: the row's maximum, then its
+// groups (8 lanes each). In place works: a wave has loaded all of a group
+// before it writes it, and no other wave reads or writes the group.
+template <int T>
+__device__ __forceinline__ float row_max(const float *x, int cols, int t) {
     float m = 0.0f;
-    for (int c = 4 * lane; c < cols; c += 256) {
+#pragma unroll 4
+    for (int c = 4 * t; c < cols; c += 4 * T) {
         const f32x4 v = *(const f32x4 *) (x + c);
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (finite_f(v[r])) m = fmaxf(m, fabsf(v[r]));
+        for (int r = 0; r < 4; ++r) m = fmaxf(m, finite_f(v[r]) ? fabsf(v[r]) : 0.0f);
     }
-    const int ex = bound_exp(wave_max(m));
-    if (lane == 0) *e = ex;
-    const float scale = exp2_int(15 - ex);
-    for (int c = 4 * lane; c < cols; c += 256) {
+    return wave_max(m);
+}
+template <int T>
+__device__ __forceinline__ void split_row(const float *x, int cols, int t, int e, uint32_t *y) {
+    const float scale = exp2_int(15 - e);
+#pragma unroll 4
+    for (int c = 4 * t; c < cols; c += 4 * T) {
         const f32x4 v = *(const f32x4 *) (x + c);
         const float a[4] = {v[0], v[1], v[2], v[3]};
         f16x4 hi, lo;
         split4(a, scale, hi, lo);
-        store_split4(y, c, hi, lo);
+        store_split4(y + (c & ~31), c & 31, hi, lo);
     }
 }
 
-__global__ __launch_bounds__(NT) void split_rows_kernel(const float *x, int64_t ld_x, int64_t rows, int cols,
-                                                        uint32_t *y, int *e) {
-    const int64_t row = (int64_t) blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    if (row < rows) split_row(x + row * ld_x, cols, y + row * cols, e + row);
+// Up to four sets of rows in one launch (a product's weights and activations:
+// two memory-bound passes of a few microseconds that overlap). A workgroup
+// takes one row of a set with rows of 2048 values and more (a wave would walk
+// them alone), else eight.
+// Rows a convolution reads (halo = (KW - 1) * dilation > 0): one output sums
+// rows of different exponents, so a row's exponent is raised to 60 below the
+// largest among the rows up to `halo` away in its batch item; what that drops
+// is 2^-100 of such a neighbour.
+__global__ __launch_bounds__(NT) void split_rows_kernel(const SplitRowsGroup g) {
+    __shared__ int es[SPLIT_RB + 2 * SPLIT_HALO];
+    __shared__ float red[NT / 64];
+    int k = 0;
+    while (k + 1 < g.n && (int) blockIdx.x >= g.j[k + 1].begin) ++k;
+    const SplitRows &p = g.j[k];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto row_at = [&](int64_t r) { return p.x + (p.rows_b ? (r / p.rows_b) * p.ld_b + (r % p.rows_b) * p.ld_x : r * p.ld_x); };
+    if (p.wide) {
+        const int64_t r = (int) blockIdx.x - p.begin;
+        const float *x = row_at(r);
+        const float m = row_max<NT>(x, p.cols, threadIdx.x);
+        if (lane == 0) red[wave] = m;
+        __syncthreads();
+        const int e = bound_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+        if (threadIdx.x == 0) p.e[r] = e;
+        split_row<NT>(x, p.cols, threadIdx.x, e, p.y + r * p.cols);
+        return;
+    }
+    const int64_t r0 = (int64_t) ((int) blockIdx.x - p.begin) * SPLIT_RB;
+    for (int i = wave; i < SPLIT_RB + 2 * p.halo; i += NT / 64) {
+        const int64_t r = r0 - p.halo + i;
+        const bool in = r >= 0 && r < p.rows;
+        const float m = in ? row_max<64>(row_at(r), p.cols, lane) : 0.0f;
+        if (lane == 0) es[i] = bound_exp(m);
+    }
+    __syncthreads();
+    for (int i = wave; i < SPLIT_RB && r0 + i < p.rows; i += NT / 64) {
+        const int64_t r = r0 + i;
+        int e = es[p.halo + i];
+        if (p.halo) {
+            const int pos = (int) (p.rows_b ? r % p.rows_b : r), last = (int) (p.rows_b ? p.rows_b : p.rows) - 1;
+            for (int d = 1; d <= p.halo; ++d) {
+                if (pos - d >= 0) e = max(e, es[p.halo + i - d] - 60);
+                if (pos + d <= last) e = max(e, es[p.halo + i + d] - 60);
+            }
+        }
+        if (lane == 0) p.e[r] = e;
+        split_row<64>(row_at(r), p.cols, lane, e, p.y + r * p.cols);
+    }
 }
 
 }  // namespace
 
-hipError_t launch_split_rows(const float *x, int64_t ld_x, int64_t rows, int cols, uint32_t *y, int *e, hipStream_t s) {
-    if (cols % BK || ld_x % 4 || rows < 1) return hipErrorInvalidValue;
-    launch_kernel(split_rows_kernel, dim3((unsigned) ((rows + NT / 64 - 1) / (NT / 64))), dim3(NT), 0, s, x, ld_x, rows,
-                  cols, y, e);
+hipError_t launch_split_rows(SplitRowsGroup &g, hipStream_t s) {
+    if (g.n < 1 || g.n > 4) return hipErrorInvalidValue;
+    int64_t blocks = 0;
+    for (int k = 0; k < g.n; ++k) {
+        SplitRows &p = g.j[k];
+        if (p.cols % BK || p.ld_x % 4 || p.ld_b % 4 || ((uintptr_t) p.x & 15) || p.rows < 1 || p.rows > INT32_MAX ||
+            p.halo < 0 || p.halo > SPLIT_HALO)
+            return hipErrorInvalidValue;
+        p.wide = p.cols >= 2048 && p.halo == 0;
+        p.begin = (int) blocks;
+        blocks += p.wide ? p.rows : (p.rows + SPLIT_RB - 1) / SPLIT_RB;
+        if (blocks > INT32_MAX) return hipErrorInvalidValue;
+    }
+    launch_kernel(split_rows_kernel, dim3((unsigned) blocks), dim3(NT), 0, s, g);
     return hipGetLastError();
 }
 
 bool split_gemm_fits(int64_t M, int64_t K, int64_t x_rows, int64_t ld_x, int items) {
     const int64_t lim = (int64_t) 1 << 31;
     return M % 4 == 0 && K % BK == 0 && M * K * 4 < lim && (x_rows * ld_x * 4 < lim || items == 1);
+}
+
+namespace {
+// estimated microseconds of a launch on 128 x 128 tiles (wide; two workgroups
+// per CU) or 128 x 64 (three): a K step of all of a CU's workgroups takes
+// 1.2, 1.65 or 0.6, 0.9, 1.35 us with one, two or three of them (measured on
+// 1292 rows of K = 1024 and 3072), and K slices cost the pass that sums them
+double split_cost(int64_t M, int64_t N, int64_t K, int S, bool wide) {
+    static const double step[2][4] = {{0, 0.6, 0.9, 1.35}, {0, 1.2, 1.65, 0}};
+    const int per_cu = wide ? 2 : 3, cus = device_info().cus;
+    const int64_t units = ((M + 127) / 128) * (wide ? (N + 127) / 128 : (N + 63) / 64) * S;
+    const int64_t full = units / (per_cu * cus), rest = units % (per_cu * cus);
+    const double round = full * step[wide][per_cu] + step[wide][(rest + cus - 1) / cus];
+    return (double) ((K / BK + S - 1) / S) * round + (S > 1 ? 3.5 + 1.3e-6 * S * N * M : 0.0);
+}
+}  // namespace
+
+int split_gemm_slices(int64_t M, int64_t N, int64_t K, int most) {
+    int sp = 1;
+    double best = 1e30;
+    for (int c = 1; c <= most && (c == 1 || K / BK / c >= 8); ++c) {
+        const double t = std::min(split_cost(M, N, K, c, false), split_cost(M, N, K, c, true));
+        if (t < best) {
+            best = t;
+            sp = c;
+        }
+    }
+    return sp;
 }
 
 hipError_t launch_gemm_split(SplitGemm &p, hipStream_t s) {
@@ -602,27 +732,17 @@ hipError_t launch_gemm_split(SplitGemm &p, hipStream_t s) {
         return hipErrorInvalidValue;
     if (p.w2 && (!p.ea || !p.y || p.M % 32 || p.M > 128 || !p.we2 || !p.mid_bias || !p.mid_ea || !p.mid_eb || p.xe_per_row))
         return hipErrorInvalidValue;
-    if (!p.ea && (!p.y || !p.xf || !p.wf || p.accumulate || (p.splits > 1 && (p.bias || p.y_bf16))))
+    if (!p.ea && (!p.y || !p.xf || !p.wf || (p.M > p.wf_rows && !p.wf2) || p.accumulate || (p.splits > 1 && (p.bias || p.y_bf16))))
         return hipErrorInvalidValue;
     if (p.conv_ic && (p.conv_ic % BK || p.K % p.conv_ic || p.conv_ow < 1 || p.conv_iw < 1 || p.conv_s < 1 ||
                       p.conv_d < 1 || p.conv_p < 0 || p.N % p.conv_ow))
         return hipErrorInvalidValue;
     p.x_rows = p.conv_ic ? (int64_t) (p.N / p.conv_ow) * p.conv_iw : p.N;
-    const int64_t tiles44 = (int64_t) ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.splits;
-    const bool big = tiles44 >= 256;
-    p.tiles_m = (p.M + 127) / 128;
-    p.tiles_n = big ? (p.N + 127) / 128 : (p.N + 63) / 64;
-    // Which operand an XCD's L2 should fetch once: the larger one. Dealing
-    // whole token tiles (or (m tile, slice) pairs) over the 8 XCDs needs
-    // enough of them that the last round of 8 is a small part.
-    const int64_t tn = (int64_t) p.tiles_n * p.splits, tm = (int64_t) p.tiles_m * p.splits;
-    const bool can1 = tn >= 64 || tn % 8 == 0, can2 = tm >= 64 || tm % 8 == 0;
-    const bool x_larger = p.x_rows * p.ld_x > (int64_t) p.M * p.K;
-    p.deal = can1 && (x_larger || !can2) ? 1 : can2 ? 2 : 0;
-    const int64_t grid = p.deal == 1 ? (tn + 7) / 8 * 8 * p.tiles_m
-                       : p.deal == 2 ? (tm + 7) / 8 * 8 * p.tiles_n : tm * p.tiles_n;
-    if (big) launch_split_tiles<4, 4>(p, (int) grid, s);
-    else launch_split_tiles<4, 2>(p, (int) grid, s);
+    p.m_inner = p.x_rows * p.ld_x > (int64_t) p.M * p.K;
+    const int64_t tiles42 = (int64_t) ((p.M + 127) / 128) * ((p.N + 63) / 64) * p.splits;
+    if (tiles42 > INT32_MAX / 16) return hipErrorInvalidValue;
+    if (split_cost(p.M, p.N, p.K, p.splits, true) <= split_cost(p.M, p.N, p.K, p.splits, false)) launch_split_tiles<4, 4, 2>(p, s);
+    else launch_split_tiles<4, 2, 3>(p, s);
     return hipGetLastError();
 }
 

@@ -772,6 +772,27 @@ __global__ void silu_mul_slices_kernel(const float *a, const float *b, int S, in
     y[i] = v / (1.0f + expf(-v)) * g;
 }
 
+// the same for rows of 2 F: a = p[n][f], b = p[n][F + f]
+__global__ void silu_mul_rows_kernel(const float *p, int S, int64_t stride, int64_t N, int F, float *y) {
+    const int64_t q = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    const int fq = F / 4;
+    if (q >= N * fq) return;
+    const int64_t n = q / fq;
+    const float *src = p + n * 2 * F + (q - n * fq) * 4;
+    f32x4 v = *(const f32x4 *) src, g = *(const f32x4 *) (src + F), o;
+    for (int z = 1; z < S; ++z) {
+        const f32x4 a = *(const f32x4 *) (src + z * stride), b = *(const f32x4 *) (src + z * stride + F);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] += a[e];
+            g[e] += b[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = v[e] / (1.0f + expf(-v[e])) * g[e];
+    *(f32x4 *) (y + q * 4) = o;
+}
+
 // y[n][m] = (sum of S K-split slices p[z][n][m], slice stride `stride`,
 // rows of M, summed in slice order) + bias[m] (nullable), rows of ld_y
 __global__ void sum_slices_kernel(const float *p, int S, int64_t stride, const float *bias, int64_t N, int M, float *y,
@@ -1346,6 +1367,14 @@ hipError_t launch_silu_mul_slices(const float *a, const float *b, int S, int64_t
                                   hipStream_t s) {
     if (S < 1 || (S > 1 && stride < n)) return hipErrorInvalidValue;
     launch_kernel(silu_mul_slices_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, a, b, S, stride, y, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_silu_mul_rows(const float *p, int S, int64_t stride, int64_t N, int F, float *y, hipStream_t s) {
+    if (S < 1 || N < 1 || F < 4 || F % 4 || stride % 4 || (S > 1 && stride < N * 2 * F) || ((uintptr_t) p & 15) ||
+        ((uintptr_t) y & 15))
+        return hipErrorInvalidValue;
+    launch_kernel(silu_mul_rows_kernel, dim3(blocks_for(N * (F / 4), 256)), dim3(256), 0, s, p, S, stride, N, F, y);
     return hipGetLastError();
 }
 

@@ -414,7 +414,7 @@ struct SplitGemm {
     const uint32_t *x, *w;         // split activation rows, split weight rows [M][K] (ld_w)
     int64_t ld_x, ld_w;
     const int *we;                 // [M] exponents of the weight rows
-    const int *xe;                 // exponent of x, or with xe_per_row one per row
+    const int *xe;                 // exponent of x, or with xe_per_row (no SnakeBeta) one per row of x
     int xe_per_row;
     const float *bias;             // [M], nullable
     void *y;                       // f32 (or y_bf16) rows; with a SnakeBeta nullable
@@ -425,9 +425,11 @@ struct SplitGemm {
     int64_t part_stride;
     // implicit im2col as GemmProblem's, over contiguous batch items of conv_iw rows
     int conv_ic, conv_iw, conv_ow, conv_s, conv_p, conv_d;
-    // without a SnakeBeta: the f32 operands (results of infinities and NaN)
-    const float *xf, *wf;
+    // without a SnakeBeta: the f32 operands (results of infinities and NaN);
+    // rows from wf_rows on are wf2's (two kernels of one input side by side)
+    const float *xf, *wf, *wf2;
     int64_t ld_xf, xf_batch, ld_wf;
+    int wf_rows;
     // SnakeBeta of y (ea non-null; F32Snake's parameters): split rows yp, or f32 rows y2
     const float *ea, *eb;
     int period;
@@ -447,20 +449,45 @@ struct SplitGemm {
     const float *mid_bias, *mid_ea, *mid_eb;   // [M]
     float mid_l1, mid_badd;
     // set by the launcher
-    int tiles_m, tiles_n, deal;
+    int tiles_m, tiles_n, m_inner, per_xcd;
     int64_t x_rows;
 };
 // M % 4, K (and conv_ic) % 32, 16-byte aligned rows (strides % 4)
 hipError_t launch_gemm_split(SplitGemm &p, hipStream_t s);
 bool split_gemm_fits(int64_t M, int64_t K, int64_t x_rows, int64_t ld_x, int items);
-// f32 rows (stride ld_x) -> split rows [rows][cols] and their exponents; in place with y == x, ld_x == cols
-hipError_t launch_split_rows(const float *x, int64_t ld_x, int64_t rows, int cols, uint32_t *y, int *e, hipStream_t s);
+// K slices that fill the chip with the tiles of an M x N x K split product
+int split_gemm_slices(int64_t M, int64_t N, int64_t K, int most);
+// f32 rows -> split rows [rows][cols] (cols % 32) and their exponents, up to
+// four sets in one launch; in place with y == x, ld_x == cols. Row r is at x +
+// r * ld_x, or with rows_b (rows per batch item) at x + r / rows_b * ld_b + r %
+// rows_b * ld_x. halo (<= SPLIT_HALO): (KW - 1) * dilation of the convolution
+// that reads the rows
+constexpr int SPLIT_RB = 8, SPLIT_HALO = 12;
+struct SplitRows {
+    const float *x;
+    int64_t ld_x, ld_b;
+    int rows_b;
+    int64_t rows;
+    int cols, halo;
+    uint32_t *y;
+    int *e;
+    // set by the launcher
+    int wide, begin;
+};
+struct SplitRowsGroup {
+    SplitRows j[4];
+    int n;
+};
+hipError_t launch_split_rows(SplitRowsGroup &g, hipStream_t s);
 // slot[0] = max |x| of the finite values, *e its exponent, slot[1 .. nslot) = 0
 hipError_t launch_split_begin(const float *x, int64_t n, float *slot, int nslot, int *e, hipStream_t s);
 // x [C][T] f32 -> split rows [T][C] at exponent *e (C % 32 == 0)
 hipError_t launch_split_transpose(const float *x, int C, int T, const int *e, uint32_t *y, hipStream_t s);
 // y = silu(a) * b, f32, n elements
 hipError_t launch_silu_mul(const float *a, const float *b, float *y, int64_t n, hipStream_t s);
+// y[n][f] = silu(a) * b for rows of 2 F: a = p[n][f], b = p[n][F + f], each the
+// sum of S slices `stride` apart in slice order (F % 4 == 0, 16-byte aligned)
+hipError_t launch_silu_mul_rows(const float *p, int S, int64_t stride, int64_t N, int F, float *y, hipStream_t s);
 // y[n][m] = sum of S K-split slices p[z][n][m] (rows of M, slices `stride` apart, summed in order)
 // + bias[m] (nullable), into rows of ld_y; M, ld_y, stride multiples of 4, 16-byte aligned
 hipError_t launch_sum_slices(const float *p, int S, int64_t stride, const float *bias, int64_t N, int M, float *y,

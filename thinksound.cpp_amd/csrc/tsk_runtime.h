@@ -20,6 +20,9 @@ int require_init();
 // buffer can only be read by work queued on s) and reallocates; a caller that
 // cannot allow that binds its own buffer, sized by tsk_workspace_size.
 int workspace(hipStream_t s, size_t bytes, void **out);
+// whether it can be had: the bound buffer is large enough, or the library's
+// own is or may grow (it may not while s is captured)
+bool workspace_can(hipStream_t s, size_t bytes);
 
 // Launch-shape overrides for tuning sweeps and A/B tests, read from the
 // environment by tsk_init (every call re-reads them) and never on a launch:
@@ -40,8 +43,9 @@ int workspace(hipStream_t s, size_t bytes, void **out);
 //   TSK_ATTN_Q8   Q8_0 driver: the attention writes linear1's Q8_0 activations itself (1), or f32 + quantize (0)
 //   TSK_F32_DL / TSK_F32_DL_NS  F32 GEMM with direct global -> LDS loads (1, default; 0 = register staged)
 //                 and its ring depth (2, default; 3)
-//   TSK_F32_SPLIT reference graph: F32 matrices as three bf16 products (1, default; read when a model is
-//                 created, which then holds the split copies) or fp32 MFMA products (0, read on every call)
+//   TSK_F32_SPLIT F32 weights of the C-ABI nodes as three fp16 products of scaled halves (1, default) or fp32 MFMA
+//                 products (0); reference graph: F32 matrices as three bf16 products (1, default; read when a
+//                 model is created, which then holds the split copies) or fp32 ones (0, read on every call)
 //   TSK_SPLIT_WG  most 128 x 128 tiles times K slices of a split product's launch (512)
 struct Tuning {
     int q8_cfg = 0;

@@ -483,9 +483,13 @@ extern "C" int tsk_vae_set_tensor(tsk_vae *v, const char *name, const float *src
                 for (size_t k = 0; k < K; ++k) l1 += std::isfinite(t[r * K + k]) ? std::fabs(t[r * K + k]) : 0.0f;
                 x.l1 = std::max(x.l1, l1);
             }
-            if (e == hipSuccess)
-                e = launch_split_rows(v->blob + x.offset, (int64_t) K, (int64_t) rows, (int) K,
-                                      (uint32_t *) (v->blob + x.offset), v->wexp + x.woffset, nullptr);
+            SplitRowsGroup sg;
+            memset(&sg, 0, sizeof(sg));
+            sg.n = 1;
+            sg.j[0].x = v->blob + x.offset; sg.j[0].ld_x = (int64_t) K;
+            sg.j[0].rows = (int64_t) rows; sg.j[0].cols = (int) K;
+            sg.j[0].y = (uint32_t *) (v->blob + x.offset); sg.j[0].e = v->wexp + x.woffset;
+            if (e == hipSuccess) e = launch_split_rows(sg, nullptr);
             if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         }
     }
