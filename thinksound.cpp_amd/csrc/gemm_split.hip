@@ -622,41 +622,47 @@ __device__ __forceinline__ void split_row(const float *x, int cols, int t, int e
 }
 
 // Up to four sets of rows in one launch (a product's weights and activations:
-// two memory-bound passes of a few microseconds that overlap). A workgroup
-// takes one row of a set with rows of 2048 values and more (a wave would walk
-// them alone), else eight.
+// two memory-bound passes of a few microseconds that overlap). A workgroup of
+// eight waves takes rows_wg rows: a wave walks a row's maximum alone, then the
+// whole workgroup splits the rows. One row where there are few (388 rows of
+// 2816 values: 15 us with eight rows and four waves), since then the chip is
+// idle and every step waits for memory; four from 2048 rows on, where the
+// maxima of the rows beside them would be read once more for each row.
 // Rows a convolution reads (halo = (KW - 1) * dilation > 0): one output sums
 // rows of different exponents, so a row's exponent is raised to 60 below the
 // largest among the rows up to `halo` away in its batch item; what that drops
 // is 2^-100 of such a neighbour.
-__global__ __launch_bounds__(NT) void split_rows_kernel(const SplitRowsGroup g) {
+constexpr int ST = 512;
+__global__ __launch_bounds__(ST) void split_rows_kernel(const SplitRowsGroup g) {
     __shared__ int es[SPLIT_RB + 2 * SPLIT_HALO];
-    __shared__ float red[NT / 64];
+    __shared__ float red[ST / 64];
     int k = 0;
     while (k + 1 < g.n && (int) blockIdx.x >= g.j[k + 1].begin) ++k;
     const SplitRows &p = g.j[k];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     auto row_at = [&](int64_t r) { return p.x + (p.rows_b ? (r / p.rows_b) * p.ld_b + (r % p.rows_b) * p.ld_x : r * p.ld_x); };
-    if (p.wide) {
-        const int64_t r = (int) blockIdx.x - p.begin;
-        const float *x = row_at(r);
-        const float m = row_max<NT>(x, p.cols, threadIdx.x);
+    const int64_t r0 = (int64_t) ((int) blockIdx.x - p.begin) * p.rows_wg;
+    if (p.rows_wg == 1 && p.halo == 0) {
+        // one row for all waves
+        const float *x = row_at(r0);
+        const float m = row_max<ST>(x, p.cols, threadIdx.x);
         if (lane == 0) red[wave] = m;
         __syncthreads();
-        const int e = bound_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-        if (threadIdx.x == 0) p.e[r] = e;
-        split_row<NT>(x, p.cols, threadIdx.x, e, p.y + r * p.cols);
+        float t = red[0];
+        for (int i = 1; i < ST / 64; ++i) t = fmaxf(t, red[i]);
+        const int e = bound_exp(t);
+        if (threadIdx.x == 0) p.e[r0] = e;
+        split_row<ST>(x, p.cols, threadIdx.x, e, p.y + r0 * p.cols);
         return;
     }
-    const int64_t r0 = (int64_t) ((int) blockIdx.x - p.begin) * SPLIT_RB;
-    for (int i = wave; i < SPLIT_RB + 2 * p.halo; i += NT / 64) {
+    for (int i = wave; i < p.rows_wg + 2 * p.halo; i += ST / 64) {
         const int64_t r = r0 - p.halo + i;
         const bool in = r >= 0 && r < p.rows;
         const float m = in ? row_max<64>(row_at(r), p.cols, lane) : 0.0f;
         if (lane == 0) es[i] = bound_exp(m);
     }
     __syncthreads();
-    for (int i = wave; i < SPLIT_RB && r0 + i < p.rows; i += NT / 64) {
+    for (int i = 0; i < p.rows_wg && r0 + i < p.rows; ++i) {
         const int64_t r = r0 + i;
         int e = es[p.halo + i];
         if (p.halo) {
@@ -666,8 +672,8 @@ __global__ __launch_bounds__(NT) void split_rows_kernel(const SplitRowsGroup g) 
                 if (pos + d <= last) e = max(e, es[p.halo + i + d] - 60);
             }
         }
-        if (lane == 0) p.e[r] = e;
-        split_row<64>(row_at(r), p.cols, lane, e, p.y + r * p.cols);
+        if (threadIdx.x == 0) p.e[r] = e;
+        split_row<ST>(row_at(r), p.cols, threadIdx.x, e, p.y + r * p.cols);
     }
 }
 
@@ -681,12 +687,12 @@ hipError_t launch_split_rows(SplitRowsGroup &g, hipStream_t s) {
         if (p.cols % BK || p.ld_x % 4 || p.ld_b % 4 || ((uintptr_t) p.x & 15) || p.rows < 1 || p.rows > INT32_MAX ||
             p.halo < 0 || p.halo > SPLIT_HALO)
             return hipErrorInvalidValue;
-        p.wide = p.cols >= 2048 && p.halo == 0;
+        p.rows_wg = p.halo == 0 ? (p.cols >= 2048 ? 1 : SPLIT_RB) : p.rows < 2048 ? 1 : SPLIT_RB / 2;
         p.begin = (int) blocks;
-        blocks += p.wide ? p.rows : (p.rows + SPLIT_RB - 1) / SPLIT_RB;
+        blocks += (p.rows + p.rows_wg - 1) / p.rows_wg;
         if (blocks > INT32_MAX) return hipErrorInvalidValue;
     }
-    launch_kernel(split_rows_kernel, dim3((unsigned) blocks), dim3(NT), 0, s, g);
+    launch_kernel(split_rows_kernel, dim3((unsigned) blocks), dim3(ST), 0, s, g);
     return hipGetLastError();
 }
 

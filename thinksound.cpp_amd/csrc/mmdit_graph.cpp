@@ -62,8 +62,9 @@ struct MW {
     bool qkv_perm;          // rows (or entries) of a qkv projection: (h d j) -> [q | k | v]
     size_t offset;          // F32 / BF16 values, or the Q8_0 int8 plane [M][K]
     size_t offset_d;        // Q8_0: the fp16 block-scale plane [M][K / 32]
-    size_t offset_s;        // split F32 matrix: bf16 planes, rows [hi | lo | hi] per K (per kw for a conv)
-    bool split;             // F32 matrix also held as split planes (products as three bf16 ones)
+    size_t offset_s;        // split F32 matrix: its split rows (gemm_split.hip) and their exponents
+    size_t offset_e;
+    bool split;             // F32 matrix also held as split rows (products on the fp16 matrix cores)
     float amax;             // max |value| of a vector as last set
 };
 
@@ -74,7 +75,8 @@ struct Lin {
     const float *wf;        // F32
     const int8_t *qw;       // Q8_0 planes
     const uint16_t *dw;
-    const uint16_t *ws;     // F32 held split: bf16 rows [M][3 K], [hi | lo | hi]
+    const uint32_t *ws;     // F32 held split: split rows and their exponents
+    const int *we;
     const float *b;
     int K, M;
 };
@@ -83,7 +85,8 @@ struct Conv {
     int type;
     const uint16_t *w;
     const float *wf;
-    const uint16_t *ws;     // F32 held split: bf16 rows [OC][KW * 3 IC], [hi | lo | hi] per kw
+    const uint32_t *ws;     // F32 held split: split rows and their exponents
+    const int *we;
     const float *b;
     int KW, IC, OC;
 };
@@ -139,6 +142,10 @@ struct tsk_mmdit {
     // SwiGLU hidden state and its halves, and the conversion scratch of the
     // BF16 / Q8_0 products
     float *xn32 = nullptr, *o32 = nullptr, *qkv32 = nullptr, *hid32 = nullptr, *h1 = nullptr, *h3 = nullptr;
+    uint32_t *xsplit = nullptr;           // split products: the activations' split rows and exponents
+    int *xexp = nullptr;
+    size_t xsplit_cap = 0;                // values of xsplit, rows of xexp
+    int xexp_cap = 0;
     uint16_t *cvt16 = nullptr;
     int8_t *qx = nullptr;
     float *dx = nullptr;
@@ -175,7 +182,7 @@ void addw(tsk_mmdit *m, const std::string &name, int64_t a, int64_t b, int64_t c
     x.kind = kind;
     x.type = TSK_TYPE_F32;
     x.qkv_perm = perm;
-    x.offset = x.offset_d = x.offset_s = 0;
+    x.offset = x.offset_d = x.offset_s = x.offset_e = 0;
     x.split = false;
     x.amax = 0.0f;
     m->idx[name] = (int) m->w.size();
@@ -245,7 +252,7 @@ Lin lin_of(const tsk_mmdit *m, const std::string &p, bool bias) {
     if (x.type == TSK_TYPE_F32) L.wf = (const float *) base;
     else if (x.type == TSK_TYPE_BF16) L.w = (const uint16_t *) base;
     else { L.qw = (const int8_t *) base; L.dw = (const uint16_t *) (m->blob + x.offset_d); }
-    if (x.split) L.ws = (const uint16_t *) (m->blob + x.offset_s);
+    if (x.split) { L.ws = (const uint32_t *) (m->blob + x.offset_s); L.we = (const int *) (m->blob + x.offset_e); }
     L.b = bias ? wp<float>(m, p + ".bias") : nullptr;
     return L;
 }
@@ -257,7 +264,7 @@ Conv conv_of(const tsk_mmdit *m, const std::string &p, bool bias) {
     C.type = x.type;
     if (x.type == TSK_TYPE_F32) C.wf = wp<float>(m, p + ".weight");
     else C.w = wp<uint16_t>(m, p + ".weight");
-    if (x.split) C.ws = (const uint16_t *) (m->blob + x.offset_s);
+    if (x.split) { C.ws = (const uint32_t *) (m->blob + x.offset_s); C.we = (const int *) (m->blob + x.offset_e); }
     C.b = bias ? wp<float>(m, p + ".bias") : nullptr;
     C.KW = (int) x.ne[0];
     C.IC = (int) x.ne[1];
@@ -461,37 +468,70 @@ int rows_bf16(tsk_mmdit *m, const Rows &src, int N, int K, hipStream_t s) {
                     "mmdit bf16 rows");
 }
 
-// F32 products as three bf16 ones (TSK_F32_SPLIT, for a model created with
-// it): the weight's planes [hi | lo | hi] against the rows' [hi | hi | lo]
-// sum x_hi w_hi + x_hi w_lo + x_lo w_hi over 3 K, which leaves out x_lo w_lo
-// and the roundings of the lo parts, about 2^-17 of |x w| per term (fp32
-// MFMA products: 157 TFLOP/s at most; three bf16 ones: 2.5 PFLOP/s / 3)
-bool split_on(const uint16_t *ws) { return ws && tuning().f32_split; }
-Lin split_lin(const Lin &L) {
-    Lin S = L;
-    S.type = TSK_TYPE_BF16; S.w = L.ws; S.K = 3 * L.K;
-    return S;
+// F32 products on the fp16 matrix cores (TSK_F32_SPLIT, for a model created
+// with it): split rows of the weight, held since it was set, and of the
+// activations, written to m->xsplit before each product
+bool split_on(const uint32_t *ws) { return ws && tuning().f32_split; }
+struct SplitW {
+    const uint32_t *ws;
+    const int *we;
+    const float *wf, *wf2;   // the f32 rows; from wf_rows on wf2's (w1 | w3 side by side)
+    int wf_rows, M, K;
+};
+SplitW split_w(const Lin &L) { return SplitW{L.ws, L.we, L.wf, nullptr, L.M, L.M, L.K}; }
+SplitW split_w(const Conv &C) { return SplitW{C.ws, C.we, C.wf, nullptr, C.OC, C.OC, C.KW * C.IC}; }
+// w1 | w3 as one weight of twice the rows (their split rows and exponents are placed back to back)
+SplitW split_pair(SplitW a, const SplitW &b) {
+    a.wf2 = b.wf;
+    a.M *= 2;
+    return a;
 }
-Conv split_conv(const Conv &C) {
-    Conv S = C;
-    S.type = TSK_TYPE_BF16; S.w = C.ws; S.IC = 3 * C.IC;
-    return S;
+bool adjacent(const SplitW &a, const SplitW &b) {
+    return b.ws == a.ws + (size_t) a.M * a.K && b.we == a.we + a.M && a.M == b.M && a.K == b.K;
 }
-// the rows as the split operand [N][3 K] in m->cvt16
-int rows_split3(tsk_mmdit *m, const Rows &src, int N, int K, hipStream_t s) {
-    if ((size_t) N * 3 * K > m->cvt_cap) return fail(TSK_ERR_SHAPE, "split rows of %d x %d exceed the scratch", N, K);
-    const int rpb = src.grp ? src.grp : N;
-    return hipcheck(launch_cast_rows_split3(src.x, src.ld, src.grp ? src.gstride : 0, rpb, N, K, m->cvt16, s),
-                    "mmdit split rows");
+// y [N][ld_y] = rows . w (+ bias), the rows [N][cols] or the convolution of KW
+// = K / cols taps over items of IW = src.grp of them (padding pad), or with
+// splits > 1 (no bias) K-split slices `stride` apart
+int split_product(tsk_mmdit *m, const SplitW &w, const Rows &src, int rows, int cols, int pad, const float *bias, float *y,
+                  int64_t ld_y, int splits, int64_t stride, hipStream_t s) {
+    if ((size_t) rows * cols > m->xsplit_cap || rows > m->xexp_cap)
+        return fail(TSK_ERR_SHAPE, "split rows of %d x %d exceed the scratch", rows, cols);
+    const int KW = w.K / cols, IW = src.grp, OW = IW + 2 * pad - (KW - 1);
+    SplitRowsGroup g;
+    memset(&g, 0, sizeof(g));
+    g.n = 1;
+    g.j[0].x = src.x; g.j[0].ld_x = src.ld; g.j[0].rows_b = src.grp; g.j[0].ld_b = src.grp ? src.gstride : 0;
+    g.j[0].rows = rows; g.j[0].cols = cols; g.j[0].halo = KW - 1;
+    g.j[0].y = m->xsplit; g.j[0].e = m->xexp;
+    int rc = hipcheck(launch_split_rows(g, s), "mmdit split rows");
+    if (rc) return rc;
+    SplitGemm q;
+    memset(&q, 0, sizeof(q));
+    q.x = m->xsplit; q.ld_x = cols;
+    q.xe = m->xexp; q.xe_per_row = 1;
+    q.w = w.ws; q.ld_w = w.K; q.we = w.we;
+    q.bias = bias;
+    q.y = y; q.ld_y = ld_y;
+    q.M = w.M; q.K = w.K;
+    q.N = src.grp ? rows / IW * OW : rows;
+    q.splits = splits; q.part_stride = stride;
+    if (src.grp) { q.conv_ic = cols; q.conv_iw = IW; q.conv_ow = OW; q.conv_s = q.conv_d = 1; q.conv_p = pad; }
+    q.xf = src.x; q.ld_xf = src.ld; q.xf_batch = src.gstride;
+    q.wf = w.wf; q.wf2 = w.wf2; q.wf_rows = w.wf_rows; q.ld_wf = w.K;
+    return hipcheck(launch_gemm_split(q, s), "mmdit split product");
 }
-// K slices of a split product (K three times the F32 one, 9216-25344 for
-// the graph's convolutions): the most, up to `most`, that keep the 128 x 128
-// tiles times slices within TSK_SPLIT_WG (512; swept 256-1536 on the Q8_0
-// graph: 384-512 best, 9 s 7.26 against 7.57-7.80 ms per forward, 30 s
-// 12.24 against 13.05-13.12); every slice an even number of 32-k tiles.
-// Counted from the rows per batch item times the batch capacity, so that a
-// batch row is summed in the same order whatever the call's batch.
-int split_slices(const tsk_mmdit *m, int M, int K, int S, int most = PART_SLICES) {
+// K slices of a split product of S rows per batch item: counted with the
+// batch capacity, so that a batch row is summed in the same order whatever the
+// call's batch (the tile shape changes no sum)
+int split_slices_f32(const tsk_mmdit *m, int M, int K, int S, int most) {
+    return split_gemm_slices(M, (int64_t) S * m->cfg.max_batch, K, most);
+}
+// K slices of a bf16 convolution into plain rows: the most, up to `most`,
+// that keep the 128 x 128 tiles times slices within TSK_SPLIT_WG (512); every
+// slice an even number of 32-k tiles. Counted from the rows per batch item
+// times the batch capacity, so that a batch row is summed in the same order
+// whatever the call's batch.
+int split_slices(const tsk_mmdit *m, int M, int K, int S, int most) {
     const int64_t t = (int64_t) ((M + 127) / 128) * ((S * m->cfg.max_batch + 127) / 128);
     const int kt = K / 32;
     int sp = 1;
@@ -499,7 +539,7 @@ int split_slices(const tsk_mmdit *m, int M, int K, int S, int most = PART_SLICES
         if (kt % c == 0 && (kt / c) % 2 == 0 && t * c <= tuning().split_wg) sp = c;
     return sp;
 }
-constexpr int SPLIT_SUM_MAX = 16;   // slices of a split convolution summed into a plain output
+constexpr int SPLIT_SUM_MAX = 16;   // slices of a convolution summed into a plain output
 // A BF16 convolution into plain f32 rows (y = conv(x) + b): over few tiles
 // with a long K (the input projections' convMLP w2, K = 8448 over 112
 // workgroups at 9 s; the final k7 convolution, 64 outputs, 7 workgroups) as
@@ -522,10 +562,10 @@ int conv_plain(tsk_mmdit *m, const Conv &C, const uint16_t *x, int64_t ld_x, int
 
 // K slices of a residual-branch convolution on the f32 path (summed by the
 // next LayerNorm): F32 kernels as fp32 products by f32_splits, as split
-// products by split_slices; BF16 kernels unsplit
+// products by split_slices_f32; BF16 kernels unsplit
 int res_splits(const tsk_mmdit *m, const Conv &C, int S) {
     if (C.type != TSK_TYPE_F32) return 1;
-    return split_on(C.ws) ? split_slices(m, C.OC, 3 * C.KW * C.IC, S) : f32_splits(m, C.OC, C.KW * C.IC, S);
+    return split_on(C.ws) ? split_slices_f32(m, C.OC, C.KW * C.IC, S, PART_SLICES) : f32_splits(m, C.OC, C.KW * C.IC, S);
 }
 
 // y[n][m] = x[n] . W[m] (+ b), any storage type
@@ -534,11 +574,8 @@ int res_splits(const tsk_mmdit *m, const Conv &C, int S) {
 int g_lin(tsk_mmdit *m, const Lin &L, const Rows &src, int N, float *y, int64_t ld_y, bool bias, hipStream_t s,
           const QkvScatter *qs = nullptr) {
     const float *b = bias ? L.b : nullptr;
-    if (L.type == TSK_TYPE_F32 && split_on(L.ws)) {
-        int rc = rows_split3(m, src, N, L.K, s);
-        if (rc) return rc;
-        return lin(split_lin(L), m->cvt16, 3 * L.K, N, y, ld_y, false, s, nullptr, !bias);
-    }
+    if (L.type == TSK_TYPE_F32 && split_on(L.ws))
+        return split_product(m, split_w(L), src, N, L.K, 0, b, y, ld_y, 1, 0, s);
     if (L.type == TSK_TYPE_F32) {
         GemmProblem q;
         memset(&q, 0, sizeof(q));
@@ -587,24 +624,22 @@ int g_conv(tsk_mmdit *m, const Conv &C, const float *x, int64_t ld_x, int64_t xb
            int64_t ld_y, bool bias, hipStream_t s, int splits = 1) {
     if (splits > 1 && bias) return fail(TSK_ERR_INVALID_ARG, "K-split slices carry no bias");
     if (C.type == TSK_TYPE_F32 && split_on(C.ws)) {
-        int rc = rows_split3(m, Rows{x, ld_x, IW, xb}, B * IW, C.IC, s);
-        if (rc) return rc;
-        const Conv S = split_conv(C);
         // a plain output over few tiles (the input projections' and the final
-        // layer's convolutions, up to K = 25344): K-split slices into m->h3
+        // layer's convolutions, up to K = 8448): K-split slices into m->h1
         // (free outside the SwiGLU halves), summed with the bias
+        const Rows src{x, ld_x, IW, xb};
         const int OW = IW + 2 * pad - (C.KW - 1), N = B * OW;
-        const size_t cap = (size_t) F32_KSPLIT_MAX * m->Rmax * m->cfg.mlp_hidden;   // floats of m->h3
+        const size_t cap = (size_t) 2 * F32_KSPLIT_MAX * m->Rmax * m->cfg.mlp_hidden;   // floats of m->h1
         const int most = (int) std::min<size_t>(SPLIT_SUM_MAX, cap / ((size_t) m->cfg.max_batch * OW * C.OC));
         const int sp = splits == 1 && C.OC % 4 == 0 && ld_y % 4 == 0 && ((uintptr_t) y & 15) == 0
-                           ? split_slices(m, C.OC, S.KW * S.IC, OW, most) : 1;
+                           ? split_slices_f32(m, C.OC, C.KW * C.IC, OW, most) : 1;
         if (sp > 1) {
-            if ((rc = conv(S, m->cvt16, S.IC, (int64_t) IW * S.IC, IW, B, pad, m->h3, C.OC, false, s, true, sp)))
-                return rc;
-            return hipcheck(launch_sum_slices(m->h3, sp, (int64_t) N * C.OC, bias ? C.b : nullptr, N, C.OC, y, ld_y, s),
+            int rc = split_product(m, split_w(C), src, B * IW, C.IC, pad, nullptr, m->h1, C.OC, sp, (int64_t) N * C.OC, s);
+            if (rc) return rc;
+            return hipcheck(launch_sum_slices(m->h1, sp, (int64_t) N * C.OC, bias ? C.b : nullptr, N, C.OC, y, ld_y, s),
                             "mmdit split slices");
         }
-        return conv(S, m->cvt16, S.IC, (int64_t) IW * S.IC, IW, B, pad, y, ld_y, false, s, !bias, splits);
+        return split_product(m, split_w(C), src, B * IW, C.IC, pad, bias ? C.b : nullptr, y, ld_y, splits, N * ld_y, s);
     }
     if (C.type == TSK_TYPE_F32) {
         GemmProblem q;
@@ -635,36 +670,29 @@ int g_swiglu(tsk_mmdit *m, bool is_conv, const Conv &c1, const Conv &c3, const C
     const int N = B * S;
     const int F = is_conv ? c1.OC : l1.M;
     const int t1 = is_conv ? c1.type : l1.type, t3 = is_conv ? c3.type : l3.type;
-    const bool split = t1 == TSK_TYPE_F32 && t3 == TSK_TYPE_F32 && split_on(is_conv ? c1.ws : l1.ws) &&
-                       split_on(is_conv ? c3.ws : l3.ws);
-    // split convolution halves over few rows (the 9 s shapes: 176 tiles of
-    // 128 x 128 where the fused GEMM would take 64 x 64 ones streaming all of
-    // K = 9216): each half as K-split slices of 128-row tiles, summed by the
-    // SiLU * gate kernel
-    const bool split_sliced = split && is_conv && (int64_t) ((F + 63) / 64) * ((N + 127) / 128) < 400;
+    const SplitW s1 = is_conv ? split_w(c1) : split_w(l1), s3 = is_conv ? split_w(c3) : split_w(l3);
+    const bool split = t1 == TSK_TYPE_F32 && t3 == TSK_TYPE_F32 && split_on(s1.ws) && split_on(s3.ws) && adjacent(s1, s3);
     int rc;
-    if (split_sliced) {
-        const int IC = 3 * c1.IC;
-        const int sp = split_slices(m, F, c1.KW * IC, S);
-        if ((rc = rows_split3(m, Rows{x, ld_x, S, xb}, N, c1.IC, s))) return rc;
-        if ((rc = conv(split_conv(c1), m->cvt16, IC, (int64_t) S * IC, S, B, 1, m->h1, F, false, s, true, sp)) ||
-            (rc = conv(split_conv(c3), m->cvt16, IC, (int64_t) S * IC, S, B, 1, m->h3, F, false, s, true, sp)) ||
-            (rc = hipcheck(launch_silu_mul_slices(m->h1, m->h3, sp, (int64_t) N * F, m->hid32, (int64_t) N * F, s),
-                           "mmdit silu * gate")))
-            return rc;
-    } else if ((t1 == TSK_TYPE_BF16 && t3 == TSK_TYPE_BF16) || split) {
-        // both halves in one cooperative GEMM with the SwiGLU epilogue, f32
-        // out; split F32 halves over their planes and the rows' split operand
-        const int f = split ? 3 : 1, IC = f * (is_conv ? c1.IC : l1.K);
+    if (split) {
+        // both halves as one product of 2 F outputs, its K slices summed by the SiLU * gate kernel
+        const int sp = split_slices_f32(m, 2 * F, s1.K, S, F32_KSPLIT_MAX);
         const Rows src = is_conv ? Rows{x, ld_x, S, xb} : Rows{x, ld_x, 0, 0};
-        if ((rc = split ? rows_split3(m, src, N, IC / 3, s) : rows_bf16(m, src, N, IC, s))) return rc;
+        if ((rc = split_product(m, split_pair(s1, s3), src, N, is_conv ? c1.IC : l1.K, is_conv ? 1 : 0, nullptr, m->h1,
+                                2 * F, sp, (int64_t) N * 2 * F, s)) ||
+            (rc = hipcheck(launch_silu_mul_rows(m->h1, sp, (int64_t) N * 2 * F, N, F, m->hid32, s), "mmdit silu * gate")))
+            return rc;
+    } else if (t1 == TSK_TYPE_BF16 && t3 == TSK_TYPE_BF16) {
+        // both halves in one cooperative GEMM with the SwiGLU epilogue, f32 out
+        const int IC = is_conv ? c1.IC : l1.K;
+        const Rows src = is_conv ? Rows{x, ld_x, S, xb} : Rows{x, ld_x, 0, 0};
+        if ((rc = rows_bf16(m, src, N, IC, s))) return rc;
         GemmGroup g;
         memset(&g, 0, sizeof(g));
         g.nprob = 1;
         GemmProblem &q = g.p[0];
         q.x = m->cvt16; q.ld_x = IC;
-        q.w = split ? (is_conv ? c1.ws : l1.ws) : is_conv ? c1.w : l1.w;
-        q.w3 = split ? (is_conv ? c3.ws : l3.ws) : is_conv ? c3.w : l3.w;
+        q.w = is_conv ? c1.w : l1.w;
+        q.w3 = is_conv ? c3.w : l3.w;
         q.ld_w = is_conv ? (int64_t) c1.KW * IC : IC;
         q.y = m->hid32; q.ld_y = F;
         q.M = F; q.N = N; q.K = (int) q.ld_w; q.splits = 1;
@@ -691,6 +719,26 @@ int g_swiglu(tsk_mmdit *m, bool is_conv, const Conv &c1, const Conv &c3, const C
     }
     if (is_conv) return g_conv(m, c2, m->hid32, F, (int64_t) S * F, S, B, 1, y, ld_y, false, s, y2_splits);
     return g_lin(m, l2, Rows{m->hid32, F, 0, 0}, N, y, ld_y, false, s);
+}
+
+// ---- products over the conditioning vectors (one row per batch item), every
+// storage type: launch_gemv_rows where the batch capacity allows (by the
+// capacity, so that a row's bits do not depend on the call's batch)
+bool vec_rows(const tsk_mmdit *m) { return m->cfg.max_batch <= 4; }
+int vec_lin(const Lin &L, const void *x, bool x_bf16, int B, float *y, int64_t ld_y, bool bias, hipStream_t s) {
+    GemvRows q;
+    memset(&q, 0, sizeof(q));
+    q.x = x; q.x_bf16 = x_bf16; q.ld_x = L.K;
+    if (L.type == TSK_TYPE_Q8_0) {
+        q.qw = L.qw; q.dw = L.dw;
+    } else {
+        q.w = L.type == TSK_TYPE_F32 ? (const void *) L.wf : (const void *) L.w;
+        q.w_f32 = L.type == TSK_TYPE_F32; q.ld_w = L.K;
+    }
+    q.bias = bias ? L.b : nullptr;
+    q.y = y; q.ld_y = ld_y;
+    q.N = B; q.M = L.M; q.K = L.K;
+    return hipcheck(launch_gemv_rows(q, s), "mmdit vector product");
 }
 
 int g_conv_mlp(tsk_mmdit *m, const std::string &p, const float *x, int64_t ld_x, int64_t xb, int S, int B, float *y,
@@ -1013,7 +1061,7 @@ extern "C" void tsk_mmdit_destroy(tsk_mmdit *m) {
     void *bufs[] = {m->blob, m->lat, m->clip, m->txt, m->sync, m->ext, m->clip0, m->txt0, m->silu_ext, m->silu_gc,
                     m->vec, m->vec16, m->mods_lat, m->mods_gc, m->xn, m->hid, m->o, m->q, m->k, m->vt, m->part,
                     m->tmp32, m->rope_l, m->rope_c, m->in16, m->in32, m->act16, m->freq, m->temb, m->xn32, m->o32,
-                    m->qkv32, m->hid32, m->h1, m->h3, m->cvt16, m->qx, m->dx, m->xs, m->f0, m->flow2};
+                    m->qkv32, m->hid32, m->h1, m->xsplit, m->xexp, m->cvt16, m->qx, m->dx, m->xs, m->f0, m->flow2};
     for (void *b : bufs)
         if (b) (void) hipFree(b);
     delete m;
@@ -1086,13 +1134,16 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
         any_q8 = any_q8 || t == TSK_TYPE_Q8_0;
         m->fast = m->fast && t == rule_type(TSK_TYPE_BF16, x);
     }
-    // F32 matrices also held as split bf16 planes (TSK_F32_SPLIT): every
+    // F32 matrices also held as split rows (TSK_F32_SPLIT): every
     // linear and convolution of the f32 path but the adaLN sets (one GEMM
     // over a whole set) and the t_embed MLP (B rows, fp32 products)
     bool any_split = false;
     if (!m->fast && tuning().f32_split)
         for (MW &x : m->w) {
-            x.split = x.type == TSK_TYPE_F32 && x.kind != K_VEC && x.name.find("adaLN_modulation") == std::string::npos &&
+            x.split = x.type == TSK_TYPE_F32 && x.kind != K_VEC &&
+                      split_gemm_fits(x.kind == K_CONV ? x.ne[2] : x.ne[1], x.kind == K_CONV ? x.ne[0] * x.ne[1] : x.ne[0],
+                                      (int64_t) c.max_batch * (c.max_latent + c.max_clip + c.max_sync + X),
+                                      x.kind == K_CONV ? x.ne[1] : x.ne[0], 2) && x.name.find("adaLN_modulation") == std::string::npos &&
                       x.name.find("t_embed") == std::string::npos;
             any_split = any_split || x.split;
         }
@@ -1113,9 +1164,10 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
         const int i = m->idx.at(name);
         MW &x = m->w[i];
         const int64_t n = x.ne[0] * x.ne[1] * x.ne[2];
-        const size_t bytes = plane == 2 ? (x.split ? 6 * (size_t) n : 0) : type_bytes(x.type, n, plane);
+        const size_t rows = (size_t) (x.kind == K_CONV ? x.ne[2] : x.ne[1]);
+        const size_t bytes = plane >= 2 ? (x.split ? 4 * (plane == 2 ? (size_t) n : rows) : 0) : type_bytes(x.type, n, plane);
         if (!bytes) return;
-        (plane == 2 ? x.offset_s : plane ? x.offset_d : x.offset) = off;
+        (plane == 3 ? x.offset_e : plane == 2 ? x.offset_s : plane ? x.offset_d : x.offset) = off;
         off += (bytes + 255) & ~(size_t) 255;
         placed[i] |= 1 << plane;
     };
@@ -1125,8 +1177,11 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
         for (const auto &p : *set) place(p + ".adaLN_modulation.1.bias", 0);
     }
     for (size_t i = 0; i < m->w.size(); ++i)
-        for (int plane = 0; plane < 3; ++plane)
+        for (int plane = 0; plane < 2; ++plane)
             if (!(placed[i] & (1 << plane))) place(m->w[i].name, plane);
+    // split rows, then exponents: a w1 and its w3 follow one another (mlp_hidden % 64: no gaps)
+    for (int plane = 2; plane < 4; ++plane)
+        for (size_t i = 0; i < m->w.size(); ++i) place(m->w[i].name, plane);
     const int B = c.max_batch, T = c.max_latent, C = c.max_clip, S = c.max_sync;
     const int64_t Ml = (int64_t) (nj + c.fused_depth) * 6 * H + 2 * H;          // latent blocks + final layer
     const int64_t Mg = (int64_t) 2 * (nj - 1) * 6 * H + 2 * 2 * H;             // clip + text (last pre_only)
@@ -1188,14 +1243,19 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
         a(&m->o32, sizeof(float) * B * m->Nmax * H);
         a(&m->qkv32, sizeof(float) * R * 3 * H);
         a(&m->hid32, sizeof(float) * R * F);
-        a(&m->h1, sizeof(float) * F32_KSPLIT_MAX * R * F);   // K-split slices of the F32 convMLP halves
-        a(&m->h3, sizeof(float) * F32_KSPLIT_MAX * R * F);
-        // conversions: at most R rows (B * T for the per-token adaLN) of the
-        // widest input, three times as wide as split operands
+        a(&m->h1, sizeof(float) * 2 * F32_KSPLIT_MAX * R * F);   // K-split slices of the F32 convMLP halves
+        m->h3 = m->h1 ? m->h1 + (size_t) F32_KSPLIT_MAX * R * F : nullptr;
+        // conversions: at most R rows (B * T for the per-token adaLN) of the widest input
         const size_t conv_rows = (size_t) std::max(R, (int64_t) B * T);
-        if (any_bf16 || any_split) {
-            m->cvt_cap = conv_rows * Wcv * (any_split ? 3 : 1);
+        if (any_bf16) {
+            m->cvt_cap = conv_rows * Wcv;
             a(&m->cvt16, 2 * m->cvt_cap);
+        }
+        if (any_split) {
+            m->xsplit_cap = conv_rows * Wcv;
+            m->xexp_cap = (int) conv_rows;
+            a(&m->xsplit, 4 * m->xsplit_cap);
+            a(&m->xexp, sizeof(int) * conv_rows);
         }
         if (any_q8) {
             m->q_cap = conv_rows * Wcv;
@@ -1341,24 +1401,15 @@ extern "C" int tsk_mmdit_set_tensor(tsk_mmdit *m, const char *name, const float 
     if (x.type == TSK_TYPE_F32) {
         e = hipMemcpy(m->blob + x.offset, v.data(), 4 * (size_t) n, hipMemcpyHostToDevice);
         if (e == hipSuccess && x.split) {
-            // rows of K (a conv: KW groups of IC per output row) -> [hi | lo | hi]
-            // per group, hi = bf16(w), lo = bf16(w - hi)
-            const int64_t G = x.kind == K_CONV ? x.ne[1] : x.ne[0];
-            std::vector<uint16_t> sp((size_t) (3 * n));
-            for (int64_t g0 = 0; g0 < n; g0 += G)
-                for (int64_t i = 0; i < G; ++i) {
-                    const float w = v[(size_t) (g0 + i)];
-                    const uint16_t hi = host_bf16_bits(w);
-                    uint32_t hb = (uint32_t) hi << 16;
-                    float hf;
-                    memcpy(&hf, &hb, 4);
-                    const uint16_t lo = std::isfinite(hf) ? host_bf16_bits(w - hf) : (uint16_t) 0;
-                    uint16_t *d = &sp[(size_t) (3 * g0 + i)];
-                    d[0] = hi;
-                    d[G] = lo;
-                    d[2 * G] = hi;
-                }
-            e = hipMemcpy(m->blob + x.offset_s, sp.data(), 2 * sp.size(), hipMemcpyHostToDevice);
+            SplitRowsGroup g;
+            memset(&g, 0, sizeof(g));
+            g.n = 1;
+            g.j[0].rows = x.kind == K_CONV ? x.ne[2] : x.ne[1];
+            g.j[0].cols = (int) (n / g.j[0].rows);
+            g.j[0].x = (const float *) (m->blob + x.offset); g.j[0].ld_x = g.j[0].cols;
+            g.j[0].y = (uint32_t *) (m->blob + x.offset_s); g.j[0].e = (int *) (m->blob + x.offset_e);
+            e = launch_split_rows(g, nullptr);
+            if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         }
     } else if (x.type == TSK_TYPE_BF16) {
         std::vector<uint16_t> bf((size_t) n);
@@ -1512,6 +1563,8 @@ int prep_cond(tsk_mmdit *m, const Call &k, hipStream_t st) {
     const int H = c.hidden, X = 2 * c.text_seq, B = k.B;
     float *tfc = vslot(m, B, V_TFC), *cmean = vslot(m, B, V_CMEAN), *cfc = vslot(m, B, V_CFC),
           *gsum = vslot(m, B, V_GSUM), *gcm = vslot(m, B, V_GCM);
+    // (tmp32 holds the two hidden vectors of each item)
+    const bool vec = vec_rows(m) && 2 * (int64_t) c.max_batch * c.mlp_hidden <= (int64_t) m->Rmax * H;
     int rc;
     if (m->fast) {
         // bf16 copies of the staged conditioning inputs (the BF16 mul_mats round their src1)
@@ -1540,14 +1593,15 @@ int prep_cond(tsk_mmdit *m, const Call &k, hipStream_t st) {
                           lin_of(m, "text_input_proj.2.w2", false), a16, H, B * X, m->txt0, H, st)))
             return rc;
         // conditioning vectors (:184-193)
-        if ((rc = lin(lin_of(m, "text_cond_proj", true), k.g16, c.clip_dim, B, tfc, H, false, st)) ||
+        if (!vec &&
+            ((rc = lin(lin_of(m, "text_cond_proj", true), k.g16, c.clip_dim, B, tfc, H, false, st)) ||
             (rc = hipcheck(launch_row_mean(m->clip0, B, k.clip_S, H, cmean, st), "clip mean")) ||
             (rc = hipcheck(launch_f32_to_bf16(cmean, v16, (int64_t) B * H, st), "bf16")) ||
             (rc = lin(lin_of(m, "clip_cond_proj", true), v16, H, B, cfc, H, false, st)) ||
             (rc = hipcheck(launch_add_f32(cfc, tfc, gsum, (int64_t) B * H, st), "add")) ||
             (rc = hipcheck(launch_f32_to_bf16(gsum, v16, (int64_t) B * H, st), "bf16")) ||
             (rc = lin_mlp(m, lin_of(m, "global_cond_mlp.w1", false), lin_of(m, "global_cond_mlp.w3", false),
-                          lin_of(m, "global_cond_mlp.w2", false), v16, H, B, gcm, H, st)))
+                          lin_of(m, "global_cond_mlp.w2", false), v16, H, B, gcm, H, st))))
             return rc;
     } else {
         float *t32 = m->tmp32;
@@ -1566,11 +1620,25 @@ int prep_cond(tsk_mmdit *m, const Call &k, hipStream_t st) {
             (rc = hipcheck(launch_silu_inplace(t32, (int64_t) B * X * H, st), "silu")) ||
             (rc = g_lin_mlp(m, "text_input_proj.2", t32, H, B * X, m->txt0, H, st)))
             return rc;
-        if ((rc = g_lin(m, lin_of(m, "text_cond_proj", true), Rows{k.g, c.clip_dim, 0, 0}, B, tfc, H, true, st)) ||
+        if (!vec &&
+            ((rc = g_lin(m, lin_of(m, "text_cond_proj", true), Rows{k.g, c.clip_dim, 0, 0}, B, tfc, H, true, st)) ||
             (rc = hipcheck(launch_row_mean(m->clip0, B, k.clip_S, H, cmean, st), "clip mean")) ||
             (rc = g_lin(m, lin_of(m, "clip_cond_proj", true), Rows{cmean, H, 0, 0}, B, cfc, H, true, st)) ||
             (rc = hipcheck(launch_add_f32(cfc, tfc, gsum, (int64_t) B * H, st), "add")) ||
-            (rc = g_lin_mlp(m, "global_cond_mlp", gsum, H, B, gcm, H, st)))
+            (rc = g_lin_mlp(m, "global_cond_mlp", gsum, H, B, gcm, H, st))))
+            return rc;
+    }
+    if (vec) {
+        const Lin w1 = lin_of(m, "global_cond_mlp.w1", false), w3 = lin_of(m, "global_cond_mlp.w3", false);
+        float *h1 = m->tmp32, *h3 = h1 + (size_t) B * w1.M;
+        if ((rc = vec_lin(lin_of(m, "text_cond_proj", true), k.g, false, B, tfc, H, true, st)) ||
+            (rc = hipcheck(launch_row_mean(m->clip0, B, k.clip_S, H, cmean, st), "clip mean")) ||
+            (rc = vec_lin(lin_of(m, "clip_cond_proj", true), cmean, false, B, cfc, H, true, st)) ||
+            (rc = hipcheck(launch_add_f32(cfc, tfc, gsum, (int64_t) B * H, st), "add")) ||
+            (rc = vec_lin(w1, gsum, false, B, h1, w1.M, false, st)) ||
+            (rc = vec_lin(w3, gsum, false, B, h3, w1.M, false, st)) ||
+            (rc = hipcheck(launch_silu_mul(h1, h3, h1, (int64_t) B * w1.M, st), "silu * gate")) ||
+            (rc = vec_lin(lin_of(m, "global_cond_mlp.w2", false), h1, false, B, gcm, H, false, st)))
             return rc;
     }
     if ((rc = grab(m, "clip_pp", m->clip0, (size_t) B * k.clip_S * H, st)) ||
@@ -1618,10 +1686,13 @@ int step(tsk_mmdit *m, const Call &k, const float *t, float *flow, hipStream_t s
     for (int b = 0; b < B; ++b) tv.t[b] = t[b];
     if ((rc = hipcheck(launch_timestep_embed(m->freq, tv, B, H, m->temb, st), "timestep embedding"))) return rc;
     const Lin te_a = lin_of(m, "t_embed.mlp.0", true), te_b = lin_of(m, "t_embed.mlp.2", true);
-    if (te_a.type == TSK_TYPE_F32) rc = lin_f32(te_a, m->temb, B, te0, st);
+    const bool vec = vec_rows(m);
+    if (vec) rc = vec_lin(te_a, m->temb, false, B, te0, H, true, st);
+    else if (te_a.type == TSK_TYPE_F32) rc = lin_f32(te_a, m->temb, B, te0, st);
     else rc = g_lin(m, te_a, Rows{m->temb, H, 0, 0}, B, te0, H, true, st);
     if (rc || (rc = hipcheck(launch_silu_inplace(te0, (int64_t) B * H, st), "silu"))) return rc;
-    if (te_b.type == TSK_TYPE_F32) rc = lin_f32(te_b, te0, B, te, st);
+    if (vec) rc = vec_lin(te_b, te0, false, B, te, H, true, st);
+    else if (te_b.type == TSK_TYPE_F32) rc = lin_f32(te_b, te0, B, te, st);
     else rc = g_lin(m, te_b, Rows{te0, H, 0, 0}, B, te, H, true, st);
     if (rc || (rc = grab(m, "t_emb", te, (size_t) B * H, st))) return rc;
     // ---- global_c = gcmlp + t_emb, extended_c (:194-196)
@@ -1639,14 +1710,16 @@ int step(tsk_mmdit *m, const Call &k, const float *t, float *flow, hipStream_t s
         if ((rc = hipcheck(launch_silu_bf16(m->ext, m->silu_ext, (int64_t) B * T * H, st), "silu")) ||
             (rc = hipcheck(launch_silu_bf16(gc, m->silu_gc, (int64_t) B * H, st), "silu")) ||
             (rc = lin(m->ada_lat, m->silu_ext, H, B * T, m->mods_lat, Ml, false, st)) ||
-            (rc = lin(m->ada_gc, m->silu_gc, H, B, m->mods_gc, Mg, false, st)))
+            (rc = vec ? vec_lin(m->ada_gc, m->silu_gc, true, B, m->mods_gc, Mg, true, st)
+                      : lin(m->ada_gc, m->silu_gc, H, B, m->mods_gc, Mg, false, st)))
             return rc;
     } else {
         // silu in place: extended_c and global_c are not read again this step
         if ((rc = hipcheck(launch_silu_inplace(m->ext, (int64_t) B * T * H, st), "silu")) ||
             (rc = hipcheck(launch_silu_inplace(gc, (int64_t) B * H, st), "silu")) ||
             (rc = g_lin(m, m->ada_lat, Rows{m->ext, H, 0, 0}, B * T, m->mods_lat, Ml, true, st)) ||
-            (rc = g_lin(m, m->ada_gc, Rows{gc, H, 0, 0}, B, m->mods_gc, Mg, true, st)))
+            (rc = vec ? vec_lin(m->ada_gc, gc, false, B, m->mods_gc, Mg, true, st)
+                      : g_lin(m, m->ada_gc, Rows{gc, H, 0, 0}, B, m->mods_gc, Mg, true, st)))
             return rc;
     }
     // the clip and text streams start from their input projections

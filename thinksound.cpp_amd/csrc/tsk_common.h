@@ -23,10 +23,10 @@ constexpr int kWave = 64;
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t h) {
     return __uint_as_float((uint32_t) h << 16);
 }
+// v_cvt_pk_bf16_f32: for all 2^32 values the bits of the integer rounding (x + 0x7fff + (x >> 16 & 1)) >> 16, NaN quieted
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-    uint32_t x = __float_as_uint(f);
-    if ((x & 0x7fffffffu) > 0x7f800000u) return (uint16_t) ((x >> 16) | 64u);
-    return (uint16_t) ((x + (0x7fffu + ((x >> 16) & 1u))) >> 16);
+    const __bf16 h = (__bf16) f;
+    return __builtin_bit_cast(uint16_t, h);
 }
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float f) {
     _Float16 h = (_Float16) f;              // v_cvt_f16_f32: RNE

@@ -247,6 +247,13 @@ int gemm_ks_bm(int cfg);
 // and the SwiGLU epilogue: EPI_STORE_F32 / _BF16, EPI_SWIGLU_F32 / _BF16.
 // M % 16 == 0, K % 32 == 0, 16-byte aligned rows.
 hipError_t launch_gemm_coop(GemmGroup &g, int epi, hipStream_t s);
+// the same over f32 activation rows, rounded to bf16 in the kernel (64 x 64
+// tiles; one problem, row-major weights, K and conv_ic % 64, ld_x and
+// x_group_stride % 4, no SwiGLU): the bits of a bf16 copy of the rows
+hipError_t launch_gemm_coop_xf32(GemmGroup &g, int epi, hipStream_t s);
+// K slices (EPI_PARTIAL) that make an M x N x K product with an f32 result
+// fastest, the pass that sums them included; ic: a convolution's channels, or 0
+int gemm_coop_slices(int64_t M, int64_t N, int64_t K, int64_t ic);
 // RoPE (cos, sin) table for positions 0 .. npos-1 and n_dims / 2 pairs, the
 // angle freq_scale * p * theta_scale^i evaluated as rope_theta() does:
 // cs[p * n_dims + 2 i] = cos, [.. + 1] = sin
@@ -284,6 +291,28 @@ hipError_t launch_quantize_rows_q8_pair(const QuantRows &r0, const QuantRows &r1
 hipError_t launch_qkv_scatter(const QkvScatter &p, hipStream_t s);
 // two streams' scatters in one launch
 hipError_t launch_qkv_scatter2(const QkvScatter &p0, const QkvScatter &p1, hipStream_t s);
+
+// y[n][m] = sum_k x[n][k] w[m][k] + bias[m] for a few rows (gemv.hip): BF16 or
+// F32 weights w (16-byte aligned rows, ld_w elements apart, K % 8), or Q8_0
+// planes qw / dw (K % 32); x f32 (BF16, Q8_0: or bf16) 16-byte aligned rows,
+// converted as ggml_mul_mat converts its src1
+constexpr int GEMV_MAX_ROWS = 8;
+struct GemvRows {
+    const void *x;
+    int x_bf16;
+    int64_t ld_x;
+    const void *w;
+    int w_f32;
+    int64_t ld_w;
+    const int8_t *qw;
+    const uint16_t *dw;
+    const float *bias;     // [M], nullable
+    void *y;
+    int y_bf16;
+    int64_t ld_y;
+    int N, M, K;
+};
+hipError_t launch_gemv_rows(const GemvRows &p, hipStream_t s);
 
 // ---------------------------------------------------------------- small ops
 // generic 4-D strided views used by the C-ABI element-wise entry points
@@ -386,9 +415,6 @@ hipError_t launch_im2col_1d(const float *x, int64_t sp, int64_t sc, int64_t sn, 
 // x + b * ld_b + i * ld_x (element strides, multiples of 4; cols % 4 == 0)
 hipError_t launch_cast_rows_bf16(const float *x, int64_t ld_x, int64_t ld_b, int rows_per_b, int64_t rows, int cols,
                                  uint16_t *y, hipStream_t s);
-// f32 rows as [hi | hi | lo] bf16 planes, 3 cols per row (split products of F32 weights)
-hipError_t launch_cast_rows_split3(const float *x, int64_t ld_x, int64_t ld_b, int rows_per_b, int64_t rows, int cols,
-                                   uint16_t *y, hipStream_t s);
 // conv kernel [KW, IC, OC] of es-byte elements (element strides s0..s2) ->
 // kw-major rows dst[oc][kw * IC + ic]
 hipError_t launch_conv_pack(const void *w, int es, int64_t s0, int64_t s1, int64_t s2, int KW, int IC, int OC, void *dst,
@@ -472,7 +498,7 @@ struct SplitRows {
     uint32_t *y;
     int *e;
     // set by the launcher
-    int wide, begin;
+    int rows_wg, begin;
 };
 struct SplitRowsGroup {
     SplitRows j[4];

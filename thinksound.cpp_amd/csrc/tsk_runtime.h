@@ -43,10 +43,10 @@ bool workspace_can(hipStream_t s, size_t bytes);
 //   TSK_ATTN_Q8   Q8_0 driver: the attention writes linear1's Q8_0 activations itself (1), or f32 + quantize (0)
 //   TSK_F32_DL / TSK_F32_DL_NS  F32 GEMM with direct global -> LDS loads (1, default; 0 = register staged)
 //                 and its ring depth (2, default; 3)
-//   TSK_F32_SPLIT F32 weights of the C-ABI nodes as three fp16 products of scaled halves (1, default) or fp32 MFMA
-//                 products (0); reference graph: F32 matrices as three bf16 products (1, default; read when a
-//                 model is created, which then holds the split copies) or fp32 ones (0, read on every call)
-//   TSK_SPLIT_WG  most 128 x 128 tiles times K slices of a split product's launch (512)
+//   TSK_F32_SPLIT F32 weights of the C-ABI nodes and of the reference graph as three fp16 products of scaled halves
+//                 (1, default) or fp32 MFMA products (0); the graph reads it when a model is created, which then
+//                 holds split copies, and on every call
+//   TSK_SPLIT_WG  most 128 x 128 tiles times K slices of the graph's bf16 convolutions into plain rows (512)
 struct Tuning {
     int q8_cfg = 0;
     bool q8_old = false;
