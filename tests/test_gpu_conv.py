@@ -238,3 +238,18 @@ def test_mlp_swiglu(env, bf16):
     got = tsk.mlp_swiglu(dev(w1), dev(w3), dev(w2), tsk.to_device(x)).numpy()
     assert got.shape == (2, 77, OC)
     assert rel_l2(got, ref) <= (3e-4 if bf16 else 1e-5)
+
+
+@pytest.mark.parametrize("B,IW,IC,OC,KW,s0,p0,d0", [(2, 33, 64, 1024, 3, 1, 1, 1), (1, 100, 1024, 64, 7, 1, 3, 1),
+                                                    (3, 41, 512, 48, 7, 2, 5, 2)])
+def test_conv1d_bf16_f32_rows_and_slices(env, B, IW, IC, OC, KW, s0, p0, d0):
+    """BF16 kernels over f32 rows rounded inside the kernel (padding, strides, several items) and in K slices: the
+    result of bf16 rows, and the oracle's up to the order of exact products (2^-24 sqrt(K))"""
+    tsk, orc = env
+    rng = np.random.default_rng(IW + OC)
+    w = kernel(orc, rng, OC, IC, KW)
+    x, bias = rng.standard_normal((B, IW, IC)).astype(np.float32), rng.standard_normal(OC).astype(np.float32)
+    wd, bd = tsk.bf16_to_device(w), tsk.to_device(bias)
+    got = tsk.conv1d(wd, tsk.to_device(x), bd, s0, p0, d0).numpy()
+    assert rel_l2(got, orc.conv1d(w, x, bias, s0, p0, d0, w_type=orc.BF16)) <= 2e-6
+    assert np.array_equal(got, tsk.conv1d(wd, tsk.bf16_to_device(orc.f32_to_bf16_bits(x)), bd, s0, p0, d0).numpy())

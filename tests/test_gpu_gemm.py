@@ -146,3 +146,52 @@ def test_q8_0_cooperative_matches_2x2_wave_kernel(env, N, K, M, cfg, monkeypatch
         monkeypatch.delenv("TSK_Q8_CFG", raising=False)
         tsk.init(0, reread=True)
     assert np.array_equal(y, y_old)
+
+
+@pytest.mark.parametrize("typ", ["bf16", "f32", "q8_0"])
+@pytest.mark.parametrize("N,K,M", [(1, 32, 1), (2, 1024, 6144), (3, 544, 36), (4, 2816, 1028), (8, 1056, 104), (9, 1024, 64)])
+def test_mul_mat_few_rows(env, typ, N, K, M):
+    """1 to 8 rows run on waves that own weight rows, more on tiles: K past a whole 512-value step, M past a
+    workgroup's rows, f32 and bf16 results. Against the oracle on the same converted operands: sums of K products in
+    another order (2^-24 sqrt(K) of the terms), 2^-9 where the result is rounded to bf16"""
+    tsk, orc = env
+    rng = np.random.default_rng(N + K)
+    w = (rng.standard_normal((M, K)) * 0.05).astype(np.float32)
+    x = rng.standard_normal((N, K)).astype(np.float32)
+    bias = rng.standard_normal(M).astype(np.float32)
+    if typ == "q8_0":
+        blocks = orc.quantize_q8_0(w)
+        wd = tsk.q8_0_repack(tsk.to_device(blocks))
+        ref = refmath.q8_0_matmul_exact(blocks, orc.quantize_q8_0(x, orc.Q8_CPU_SIMD)) + bias
+    elif typ == "bf16":
+        wb = orc.f32_to_bf16_bits(w)
+        wd, ref = tsk.bf16_to_device(wb), orc.mul_mat(wb, x, a_type=orc.BF16) + bias
+    else:
+        wd, ref = tsk.to_device(w), orc.mul_mat(w, x) + bias
+    xd, bd = tsk.to_device(x), tsk.to_device(bias)
+    at = tsk.Q8_0_SPLIT if typ == "q8_0" else None
+    y = tsk.mul_mat(wd, xd, bias=bd, a_type=at).numpy()
+    assert rel_l2(y, ref) <= 2e-6
+    if M % 8 == 0:
+        y16 = tsk.mul_mat(wd, xd, bias=bd, a_type=at, out_dtype="bf16").numpy()
+        assert rel_l2(orc.bf16_bits_to_f32(y16), ref) <= 2.0 ** -8
+    if typ == "bf16":
+        xb = orc.f32_to_bf16_bits(x)
+        assert np.array_equal(tsk.mul_mat(wd, tsk.bf16_to_device(xb), bias=bd).numpy(), y)
+
+
+@pytest.mark.parametrize("N,K,M", [(9, 64, 16), (65, 192, 1024), (388, 1024, 3072), (70, 4096, 80), (200, 2816, 1024),
+                                   (646, 2560, 1040)])
+def test_bf16_gemm_f32_rows_and_slices(env, N, K, M):
+    """f32 activations rounded inside the kernel are a bf16 copy of them (same bits with bf16 activations where the
+    product runs whole); long K over few tiles in slices, the bias added by their sum. Against the oracle: sums of K
+    exact products in another order (2^-24 sqrt(K) of the terms)"""
+    tsk, orc = env
+    rng = np.random.default_rng(N + K)
+    wb = orc.f32_to_bf16_bits((rng.standard_normal((M, K)) * 0.05).astype(np.float32))
+    x, bias = rng.standard_normal((N, K)).astype(np.float32), rng.standard_normal(M).astype(np.float32)
+    wd, bd = tsk.bf16_to_device(wb), tsk.to_device(bias)
+    y = tsk.mul_mat(wd, tsk.to_device(x), bias=bd).numpy()
+    assert rel_l2(y, orc.mul_mat(wb, x, a_type=orc.BF16) + bias) <= 2e-6
+    y16 = tsk.mul_mat(wd, tsk.bf16_to_device(orc.f32_to_bf16_bits(x)), bias=bd).numpy()
+    assert np.array_equal(y, y16)

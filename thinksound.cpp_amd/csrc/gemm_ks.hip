@@ -138,15 +138,18 @@ enum : int {
     MODE_COOP = 2,     // 2 x 2 waves over the tile, one shared LDS ring
     MODE_COOP_PIPE = 3,// MODE_COOP with the next stage's fragments read from LDS during this stage's MFMAs
     MODE_COOP64 = 4,   // MODE_COOP with 64-wide k stages of whole 128-byte rows (swizzled in LDS)
+    MODE_COOP64F = 6,  // MODE_COOP64 over f32 activation rows, rounded to bf16 as they are read from LDS
     MODE_PF = 5        // MODE_COOP64's LDS layout, double-buffered, fed from R stages of register prefetch
 };
 
 template <int TM, int TN, int R, int MODE, int KH = 1>
 constexpr size_t lds_bytes() {
-    constexpr bool coop = MODE == MODE_COOP || MODE == MODE_COOP_PIPE || MODE == MODE_COOP64 || MODE == MODE_PF;
+    constexpr bool coop = MODE == MODE_COOP || MODE == MODE_COOP_PIPE || MODE == MODE_COOP64 || MODE == MODE_COOP64F ||
+                          MODE == MODE_PF;
     constexpr size_t ring = MODE == MODE_DIRECT ? 0
                           : MODE == MODE_PF     ? (size_t) 2 * 2 * (TM + TN) * 1024
                           : MODE == MODE_COOP64 ? (size_t) R * 2 * (TM + TN) * 1024
+                          : MODE == MODE_COOP64F ? (size_t) R * (2 * TM + 4 * TN) * 1024
                           : coop                ? (size_t) R * KH * (TM + TN) * 1024
                                                 : (size_t) 4 * R * (TM + TN) * 1024;
     constexpr size_t red = coop ? (size_t) (16 * TN) * (16 * TM + 4) * 4
@@ -165,7 +168,8 @@ constexpr bool epi_swiglu(int epi) { return epi == EPI_SWIGLU_F32 || epi == EPI_
 template <int TM, int TN, int R, int MODE, int EPI, int KH, bool CONV>
 __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord tc, uint8_t *lds) {
     constexpr int BM = 16 * TM, BN = 16 * TN, L = TM + TN, STAGE = KH * L * 1024;
-    constexpr bool PIPE = MODE == MODE_COOP_PIPE, PF = MODE == MODE_PF, C64 = MODE == MODE_COOP64 || PF;
+    constexpr bool XF = MODE == MODE_COOP64F;
+    constexpr bool PIPE = MODE == MODE_COOP_PIPE, PF = MODE == MODE_PF, C64 = MODE == MODE_COOP64 || XF || PF;
     constexpr bool COOP = MODE == MODE_COOP || PIPE || C64, DIRECT = MODE == MODE_DIRECT;
     static_assert(!COOP || (TM % 2 == 0 && TN % 2 == 0 && (C64 ? L % 2 : L % 4) == 0), "cooperative tile shape");
     static_assert((COOP && !PIPE && !C64) || KH == 1, "KH: 32-wide k tiles per cooperative stage");
@@ -253,8 +257,14 @@ __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord t
         // row is one whole 128-byte line, and the MFMA read of chunk c of
         // row t at block t / 8, row t % 8, slot c ^ key hits 16 distinct
         // 16-byte bank groups over the 16 rows.
-        constexpr int U = TM + TN, LW = 2 * U / 4;
-        constexpr int USZ = 2048, STG = U * USZ;
+        // MODE_COOP64F: an activation unit is 16 rows x 256 bytes of f32, two
+        // such 2 KiB halves of 32 k each (BE halves of 16-bit units per unit,
+        // XE halfwords per value); the bf16 rounding is the one a conversion
+        // launch would apply, without its launch and its pass over memory.
+        constexpr int BE = XF ? 4 : 2, XE = XF ? 2 : 1;
+        constexpr int LW = (2 * TM + BE * TN) / 4;
+        static_assert((2 * TM + BE * TN) % 4 == 0, "whole loads per wave");
+        constexpr int USZ = 2048, STG = TM * USZ + TN * BE * 1024;
         const int ns = my_n;
         const int r8 = lane >> 3;
         // MFMA read offsets of this lane (token / row t = lane % 16, chunk 4 kh + lane / 16)
@@ -276,9 +286,10 @@ __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord t
         int qlds[LW], qstep[LW], qconv[CONV ? LW : 1], qchk[CONV ? LW : 1];
 #pragma unroll
         for (int q = 0; q < LW; ++q) {
-            const int f = wave + 4 * q, u = f >> 1, h = f & 1;
-            const int chk = ((lane & 7) ^ r8 ^ (4 * h)) * 8;            // bf16 elements
-            qlds[q] = u * USZ + h * 1024;
+            const int f = wave + 4 * q, fb = f - 2 * TM, h = f & 1;
+            const int u = f < 2 * TM ? f >> 1 : TM + fb / BE, kx = XF && f >= 2 * TM ? fb >> 1 & 1 : 0;
+            const int chk = ((lane & 7) ^ r8 ^ (4 * h)) * 8;            // halfwords
+            qlds[q] = f * 1024;
             if constexpr (CONV) {
                 qconv[q] = 0;
                 qchk[q] = chk;
@@ -298,12 +309,12 @@ __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord t
                 if constexpr (CONV) {
                     // implicit im2col: the row base (batch item) and first input position
                     const int b = n / p.conv_ow, ow = n - b * p.conv_ow;
-                    qsrc[q] = (const uint16_t *) p.x + (int64_t) b * p.x_group_stride + chk;
+                    qsrc[q] = (const uint16_t *) p.x + XE * (int64_t) b * p.x_group_stride + chk + 64 * kx;
                     qconv[q] = ow * p.conv_s - p.conv_p;
                     qstep[q] = 0;
                 } else {
-                    qsrc[q] = (const uint16_t *) p.x + x_row(p, n) + chk + kt0 * 32;
-                    qstep[q] = 64;
+                    qsrc[q] = (const uint16_t *) p.x + XE * (x_row(p, n) + kt0 * 32) + chk + 64 * kx;
+                    qstep[q] = 64 * XE;
                 }
             }
         }
@@ -317,7 +328,7 @@ __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord t
                     if (isb) {
                         const int k = (kt0 + 2 * t) * 32, kw = k / p.conv_ic, ic0 = k - kw * p.conv_ic;
                         const int iw = qconv[q] + kw * p.conv_d;
-                        g2l16(iw >= 0 && iw < p.conv_iw ? qsrc[q] + (int64_t) iw * p.ld_x + ic0 : g_zero_row + qchk[q],
+                        g2l16(iw >= 0 && iw < p.conv_iw ? qsrc[q] + XE * ((int64_t) iw * p.ld_x + ic0) : g_zero_row + qchk[q],
                               dst + qlds[q]);
                         continue;
                     }
@@ -333,7 +344,44 @@ __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord t
         // scheduling barrier keeps the compiler from interleaving reads and
         // MFMAs, which serialises on the LDS latency): the second half's reads
         // are in flight during the first half's MFMAs
+        int xoff[2];
+        {
+            const int tq = lane & 15, kc = lane >> 4;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                xoff[e] = (tq >> 3) * 1024 + (tq & 7) * 128 + (((2 * kc + e) ^ (tq & 7) ^ (4 * (tq >> 3))) * 16);
+        }
+        auto compute_f = [&](const uint8_t *src) {
+            bf16x8 a[2][TMW];
+            f32x4 x[2][TNW][2];
+#pragma unroll
+            for (int kh = 0; kh < 2; ++kh) {
+#pragma unroll
+                for (int i = 0; i < TMW; ++i) a[kh][i] = *(const bf16x8 *) (src + (wm * TMW + i) * USZ + aro[kh]);
+#pragma unroll
+                for (int j = 0; j < TNW; ++j)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        x[kh][j][e] = *(const f32x4 *) (src + TM * USZ + (wn * TNW + j) * 4096 + kh * 2048 + xoff[e]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+                for (int j = 0; j < TNW; ++j) {
+                    bf16x8 b;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) b[e] = (__bf16) x[kh][j][e >> 2][e & 3];
+#pragma unroll
+                    for (int i = 0; i < TMW; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kh][i], b, acc[i][j], 0, 0, 0);
+                }
+        };
         auto compute = [&](const uint8_t *src) {
+            if constexpr (XF) {
+                compute_f(src);
+                return;
+            }
             bf16x8 a[2][TMW], b[2][TNW];
 #pragma unroll
             for (int kh = 0; kh < 2; ++kh) {
@@ -857,7 +905,7 @@ hipError_t ks_launch(GemmGroup &g, hipStream_t s) {
         p.tiles_n = (p.N + BN - 1) / BN;
         p.kt_split = (p.K / 32 + p.splits - 1) / p.splits;
         if (KH > 1 && ((p.K / 32) % p.splits || p.kt_split % KH)) return hipErrorInvalidValue;
-        if ((MODE == MODE_COOP64 || MODE == MODE_PF) &&
+        if ((MODE == MODE_COOP64 || MODE == MODE_COOP64F || MODE == MODE_PF) &&
             ((p.K / 32) % p.splits || p.kt_split % 2 || (CONV && p.conv_ic % 64)))
             return hipErrorInvalidValue;
         p.block_begin = (nblocks + 7) & ~7;
@@ -897,6 +945,31 @@ hipError_t conv_epi(GemmGroup &g, int epi, hipStream_t s) {
 }
 
 }  // namespace
+
+hipError_t launch_gemm_coop_xf32(GemmGroup &g, int epi, hipStream_t s) {
+    const GemmProblem &p = g.p[0];
+    const bool conv = p.conv_ic != 0;
+    if (g.nprob != 1 || p.M < 16 || p.M % 16 || p.N < 1 || p.K < 64 || p.K % 64 || p.splits < 1 || p.w_tiled || p.ld_w % 8 ||
+        ((uintptr_t) p.w & 15) || ((uintptr_t) p.x & 15) || p.ld_x % 4 || (p.splits != 1 && epi != EPI_PARTIAL))
+        return hipErrorInvalidValue;
+    if (conv && (p.conv_ic % 64 || p.K % p.conv_ic || p.x_group_rows || p.conv_ow < 1 || p.conv_iw < 1 || p.conv_s < 1 ||
+                 p.conv_d < 1 || p.conv_p < 0 || p.N % p.conv_ow || p.x_group_stride % 4))
+        return hipErrorInvalidValue;
+    // a two-stage ring: three workgroups per CU (three stages, two: 388 x 1024
+    // -> 3072 11.9 / 12.3 us, 2080 rows 40 / 51)
+    switch (epi) {
+        case EPI_STORE_F32:
+            return conv ? ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_F32, 1, true>(g, s)
+                        : ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_F32, 1, false>(g, s);
+        case EPI_STORE_BF16:
+            return conv ? ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_BF16, 1, true>(g, s)
+                        : ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_BF16, 1, false>(g, s);
+        case EPI_PARTIAL:
+            return conv ? ks_launch<4, 4, 2, MODE_COOP64F, EPI_PARTIAL, 1, true>(g, s)
+                        : ks_launch<4, 4, 2, MODE_COOP64F, EPI_PARTIAL, 1, false>(g, s);
+        default: return hipErrorInvalidValue;
+    }
+}
 
 hipError_t launch_gemm_coop(GemmGroup &g, int epi, hipStream_t s) {
     if (g.nprob < 1 || g.nprob > 2) return hipErrorInvalidValue;
@@ -944,6 +1017,34 @@ hipError_t launch_gemm_coop(GemmGroup &g, int epi, hipStream_t s) {
         case 32: return conv ? conv_epi<8, 8, 2, true, MODE_COOP64>(g, epi, s) : conv_epi<8, 8, 2, false, MODE_COOP64>(g, epi, s);
         default: return hipErrorInvalidValue;
     }
+}
+
+int gemm_coop_slices(int64_t M, int64_t N, int64_t K, int64_t ic) {
+    // A tile walks its slice of K alone: 0.33 us per 64 k while the chip is not
+    // full, 0.40 and 0.50 with two and three 64 x 64 tiles on a CU (128 x 64,
+    // from 400 of them: 0.4, 0.55, 0.8); the pass that sums the slices costs
+    // 3.3 us and 2.4e-6 us per value of them. Measured, us without / with, the
+    // cast of the rows included: K = 4096, M = 1024, N = 64 25 / 13, N = 388
+    // 29 / 18; K = 7168, M = 64, 388 rows 56 / 15; convMLP of 1292 rows 128 /
+    // 97. From K = 2560: K = 1024, N = 388 11.4 / 12.6
+    const int64_t kt = K / 64, t64 = ((M + 63) / 64) * ((N + 63) / 64), t128 = ((M + 127) / 128) * ((N + 63) / 64);
+    if (K % 64 || ic % 64 || M % 16 || M < 16 || kt < 40) return 1;
+    static const double step[2][4] = {{0, 0.33, 0.40, 0.50}, {0, 0.40, 0.55, 0.80}};
+    const int cus = device_info().cus;
+    int sp = 1;
+    double best = 1e30;
+    for (int c = 1; c <= 16; ++c) {
+        if (kt % c || (c > 1 && kt / c < 6)) continue;
+        const int wide = t128 * c >= 400;
+        const int64_t u = (wide ? t128 : t64) * c, full = u / (3 * cus), rest = u % (3 * cus);
+        const double us = (double) (kt / c) * (full * step[wide][3] + step[wide][(rest + cus - 1) / cus]) +
+                          (c > 1 ? 3.3 + 2.4e-6 * c * N * M : 0.0);
+        if (us < best) {
+            best = us;
+            sp = c;
+        }
+    }
+    return sp;
 }
 
 int gemm_ks_bm(int cfg) {

@@ -483,6 +483,34 @@ F32Split plan_f32_split(int64_t M, int64_t N, int64_t K, int64_t x_rows, int64_t
     pl.bytes = off;
     return pl;
 }
+// K slices of a BF16 product on the cooperative tiles (f32 result): see
+// coop_slices(); 0 bytes where it runs whole
+size_t coop_part_bytes(int64_t M, int64_t N, int64_t K, int64_t ic, bool y_bf16, int *splits) {
+    *splits = y_bf16 ? 1 : gemm_coop_slices(M, N, K, ic);
+    return *splits > 1 ? align256((size_t) *splits * (size_t) (N * M) * 4) : 0;
+}
+// g.p[0] (f32 result, with its bias) as `splits` slices in part, then their sum
+hipError_t coop_sliced(GemmGroup &g, float *part, int splits, bool xf32, hipStream_t s) {
+    GemmProblem &q = g.p[0];
+    const float *bias = q.bias;
+    float *y = (float *) q.y;
+    const int64_t ld_y = q.ld_y;
+    q.bias = nullptr; q.y = part; q.ld_y = q.M; q.splits = splits;
+    const hipError_t e = xf32 ? launch_gemm_coop_xf32(g, EPI_PARTIAL, s) : launch_gemm_coop(g, EPI_PARTIAL, s);
+    return e == hipSuccess ? launch_sum_slices(part, splits, (int64_t) q.N * q.M, bias, q.N, q.M, y, ld_y, s) : e;
+}
+// f32 activations of BF16 weights rounded inside the product's kernel instead
+// of by a launch before it: the launch and its pass over memory against twice
+// the activation bytes and the conversions in every tile. Up to 4000 64 x 64
+// x 64 tile steps, more for narrow linear layers, whose rows few tiles share
+// (us with the launch / without: K = 1024, N = 388, M = 1024 11.4 / 9.5, 3072
+// 12.3 / 12.4 on new inputs, 6144 16.5 / 17.6; N = 2080, M = 1024 19.7 / 16.7; K = 64 7.5 /
+// 4.0; k3 convolution of 1292 rows 29 / 36)
+bool coop_xf32(int64_t M, int64_t N, int64_t K, int64_t ic, int64_t ld_w) {
+    if (K % 64 || ic % 64 || ld_w % 8) return false;
+    const int64_t steps = ((M + 63) / 64) * ((N + 63) / 64) * (K / 64);
+    return steps <= (M <= 1024 && !ic ? 15000 : 4000);
+}
 SplitRows split_job(const F32Rows &r, int halo, char *y, char *e) {
     SplitRows j;
     memset(&j, 0, sizeof(j));
@@ -536,8 +564,12 @@ int f32_split(const F32Split &pl, char *ws, const F32Rows &w, int64_t N, const F
 struct MulMatPlan {
     bool uni;            // rows of b and dst uniformly strided: one GEMM of Nslice rows
     int64_t nslices, Nslice;
+    bool gemv;           // a few rows, no scratch
     bool coop;           // BF16 weights on the cooperative tiles
-    size_t cast_bytes;   // coop with f32 b: b rounded to bf16 rows
+    bool xf32;           // coop with f32 b: rounded in the kernel, or
+    size_t cast_bytes;   // b rounded to bf16 rows
+    size_t part_bytes;   // coop in K slices, if their scratch can be had as well
+    int splits;
     size_t wbytes;       // Q8_0: the weights repacked into planes
     size_t act_bytes;    // Q8_0 / Q8_0_SPLIT: the quantized activation planes
     size_t bytes;        // scratch the call needs
@@ -552,7 +584,15 @@ MulMatPlan plan_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tens
     pl.uni = rows_uniform(b) && rows_uniform(dst);
     pl.nslices = pl.uni ? 1 : b->ne[2] * b->ne[3];
     pl.Nslice = pl.uni ? b->ne[1] * b->ne[2] * b->ne[3] : b->ne[1];
+    // Few rows. From 5 rows on every wave's own conversion of the activations
+    // costs as much as a launch of it where there are many waves (8 rows, tiles
+    // against rows: BF16 M = 1024 10.1 / 5.5 us, M = 6144 9.6 / 9.8; Q8_0 M =
+    // 1024 11.8 / 8.7, M = 2816 11.5 / 13.1; F32 without conversion 24.7 / 9.1)
+    pl.gemv = pl.uni && pl.Nslice <= (a->type == TSK_TYPE_F32 || M <= 2048 ? GEMV_MAX_ROWS : 4);
+    if (pl.gemv && a->type != TSK_TYPE_Q8_0) return pl;      // (Q8_0 blocks are repacked first)
     pl.coop = a->type == TSK_TYPE_BF16 && pl.uni && M % 16 == 0 && K % 32 == 0 && a->nb[1] % 16 == 0;
+    pl.xf32 = pl.coop && b->type == TSK_TYPE_F32 && coop_xf32(M, pl.Nslice, K, 0, (int64_t) (a->nb[1] / 2));
+    // (asked for in either case: one size per node, whatever the route)
     if (pl.coop && b->type == TSK_TYPE_F32) pl.cast_bytes = align256((size_t) (pl.Nslice * K) * 2);
     if (a->type == TSK_TYPE_Q8_0 || a->type == TSK_TYPE_Q8_0_SPLIT) {
         pl.wbytes = a->type == TSK_TYPE_Q8_0 ? align256(tsk_q8_0_split_nbytes(K, M)) : 0;
@@ -560,6 +600,7 @@ MulMatPlan plan_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tens
         pl.act_bytes = align256(pl.act_bytes);
     }
     pl.bytes = pl.cast_bytes + pl.wbytes + pl.act_bytes;
+    if (pl.coop) pl.part_bytes = coop_part_bytes(M, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16, &pl.splits);
     if (a->type == TSK_TYPE_F32 && pl.uni)
         pl.split = plan_f32_split(M, pl.Nslice, K, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16);
     return pl;
@@ -573,13 +614,37 @@ int mul_mat_impl(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bia
     const MulMatPlan pl = plan_mul_mat(a, b, dst);
     int rc;
     char *ws = nullptr;
+    if (pl.gemv) {
+        GemvRows q;
+        memset(&q, 0, sizeof(q));
+        q.x = b->data; q.x_bf16 = b->type == TSK_TYPE_BF16; q.ld_x = (int64_t) (b->nb[1] / es_b);
+        if (a->type == TSK_TYPE_Q8_0 || a->type == TSK_TYPE_Q8_0_SPLIT) {
+            const char *w = (const char *) a->data;
+            if (a->type == TSK_TYPE_Q8_0) {
+                if ((rc = scr.get(pl.bytes, (void **) &ws))) return rc;
+                const hipError_t e = launch_q8_repack(a->data, (int64_t) a->nb[1], M, K, ws, s);
+                if (e != hipSuccess) return hip_fail(e, "q8 repack");
+                w = ws;
+            }
+            q.qw = (const int8_t *) w;
+            q.dw = (const uint16_t *) (w + (size_t) (M * K));
+        } else {
+            q.w = a->data; q.w_f32 = a->type == TSK_TYPE_F32; q.ld_w = (int64_t) (a->nb[1] / elt_size(a->type));
+        }
+        q.bias = bias ? (const float *) bias->data : nullptr;
+        q.y = dst->data; q.y_bf16 = dst->type == TSK_TYPE_BF16; q.ld_y = (int64_t) (dst->nb[1] / es_d);
+        q.N = (int) pl.Nslice; q.M = (int) M; q.K = (int) K;
+        const hipError_t e = launch_gemv_rows(q, s);
+        return e == hipSuccess ? TSK_OK : hip_fail(e, "mul_mat rows launch");
+    }
     if (pl.split.on && (ws = scr.optional(pl.split.bytes))) {
         const F32Rows w{(const float *) a->data, (int64_t) (a->nb[1] / 4), 0, 0, M, (int) K};
         const F32Rows x{(const float *) b->data, (int64_t) (b->nb[1] / 4), 0, 0, pl.Nslice, (int) K};
         return f32_split(pl.split, ws, w, pl.Nslice, x, F32Conv{}, bias ? (const float *) bias->data : nullptr, dst->data,
                          dst->type == TSK_TYPE_BF16, (int64_t) (dst->nb[1] / es_d), s);
     }
-    if ((rc = scr.get(pl.bytes, (void **) &ws))) return rc;
+    const bool sliced = pl.part_bytes && (ws = scr.optional(pl.bytes + pl.part_bytes));
+    if (!sliced && (rc = scr.get(pl.bytes, (void **) &ws))) return rc;
     const int64_t nslices = pl.nslices, Nslice = pl.Nslice;
 
     // BF16 weights with M % 16 == 0, K % 32 == 0 and uniformly strided rows:
@@ -589,7 +654,7 @@ int mul_mat_impl(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bia
         uint16_t *xb = nullptr;
         const int64_t N = Nslice;
         const int64_t ld_b = (int64_t) (b->nb[1] / es_b);
-        if (b->type == TSK_TYPE_F32) {
+        if (b->type == TSK_TYPE_F32 && !pl.xf32) {
             xb = (uint16_t *) ws;
             hipError_t e = launch_cast_rows_bf16((const float *) b->data, ld_b, 0, (int) std::min<int64_t>(N, 1 << 30), N,
                                                  (int) K, xb, s);
@@ -607,7 +672,9 @@ int mul_mat_impl(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bia
         q.y = dst->data;
         q.ld_y = (int64_t) (dst->nb[1] / es_d);
         q.M = (int) M; q.N = (int) N; q.K = (int) K; q.splits = 1;
-        hipError_t e = launch_gemm_coop(g, dst->type == TSK_TYPE_BF16 ? EPI_STORE_BF16 : EPI_STORE_F32, s);
+        const int epi = dst->type == TSK_TYPE_BF16 ? EPI_STORE_BF16 : EPI_STORE_F32;
+        hipError_t e = sliced ? coop_sliced(g, (float *) (ws + pl.bytes), pl.splits, pl.xf32, s)
+                     : pl.xf32 ? launch_gemm_coop_xf32(g, epi, s) : launch_gemm_coop(g, epi, s);
         return e == hipSuccess ? TSK_OK : hip_fail(e, "mul_mat launch");
     }
 
@@ -1181,13 +1248,15 @@ size_t conv_cast_bytes(int wtype, int x_f32, int64_t IC, int64_t IW, int64_t B, 
 // stride xb in elements), y rows [B * OW][OC] (ld_y); kw-major weight rows.
 // swiglu: w3 rows given -> y = silu(x * w) * (x * w3) (BF16 kernels only).
 // xcast: conv_cast_bytes() of scratch, or nullptr when that is 0.
+// part: scratch of `splits` K slices of an f32 result, or nullptr.
 int conv_gemm(int wtype, const void *wrows, const void *w3rows, int64_t ld_w, const float *bias, int KW, int IC, int OC,
               const void *x, int x_f32, int64_t ld_x, int64_t xb, int IW, int B, int s0, int p0, int d0, void *y,
-              int y_bf16, int64_t ld_y, uint16_t *xcast, hipStream_t s) {
+              int y_bf16, int64_t ld_y, uint16_t *xcast, hipStream_t s, float *part = nullptr, int splits = 1,
+              bool xf32 = false) {
     const int OW = (int) conv_out_len(IW, KW, s0, p0, d0);
-    const bool coop = conv_coop(wtype, IC, OC) && (!x_f32 || xcast) && ld_w % 8 == 0 &&
+    const bool coop = conv_coop(wtype, IC, OC) && (!x_f32 || xcast || xf32) && ld_w % 8 == 0 &&
                       ((uintptr_t) wrows & 15) == 0 && ((uintptr_t) w3rows & 15) == 0;
-    if (coop && x_f32) {
+    if (coop && x_f32 && !xf32) {
         hipError_t e = launch_cast_rows_bf16((const float *) x, ld_x, xb, IW, (int64_t) B * IW, IC, xcast, s);
         if (e != hipSuccess) return hip_fail(e, "conv input cast");
         x = xcast;
@@ -1215,7 +1284,9 @@ int conv_gemm(int wtype, const void *wrows, const void *w3rows, int64_t ld_w, co
         q.w3 = (const uint16_t *) w3rows;
         g.p[0] = q;
         const int epi = w3rows ? (y_bf16 ? EPI_SWIGLU_BF16 : EPI_SWIGLU_F32) : (y_bf16 ? EPI_STORE_BF16 : EPI_STORE_F32);
-        e = coop ? launch_gemm_coop(g, epi, s) : launch_gemm_group(g, x_f32 ? GEMM_X_F32 : 0, epi, s);
+        e = coop && part && epi == EPI_STORE_F32 ? coop_sliced(g, part, splits, xf32, s)
+            : coop && xf32 ? launch_gemm_coop_xf32(g, epi, s)
+            : coop ? launch_gemm_coop(g, epi, s) : launch_gemm_group(g, x_f32 ? GEMM_X_F32 : 0, epi, s);
     }
     return e == hipSuccess ? TSK_OK : hip_fail(e, "conv GEMM launch");
 }
@@ -1228,7 +1299,21 @@ F32Split plan_conv_split(const tsk_tensor *w, const tsk_tensor *x, int s0, int p
                           dst->type == TSK_TYPE_BF16);
 }
 
+// BF16 kernels in K slices (after conv1d_ws_bytes)
+size_t conv1d_part_bytes(const tsk_tensor *w, const tsk_tensor *x, int s0, int p0, int d0, const tsk_tensor *dst, int *splits) {
+    const int64_t KW = w->ne[0], IC = w->ne[1], OC = w->ne[2];
+    *splits = 1;
+    if (!conv_coop(w->type, (int) IC, (int) OC)) return 0;
+    return coop_part_bytes(OC, x->ne[2] * conv_out_len(x->ne[1], KW, s0, p0, d0), KW * IC, IC, dst->type == TSK_TYPE_BF16,
+                           splits);
+}
+
 // scratch of tsk_conv1d: the kw-major kernel copy and the bf16 input rows
+bool conv1d_xf32(const tsk_tensor *w, const tsk_tensor *x) {
+    const int64_t K = w->ne[0] * w->ne[1];
+    return conv_coop(w->type, (int) w->ne[1], (int) w->ne[2]) && x->type == TSK_TYPE_F32 &&
+           coop_xf32(w->ne[2], x->ne[1] * x->ne[2], K, w->ne[1], kw_major(w) && w->ne[2] > 1 ? (int64_t) (w->nb[2] / 2) : K);
+}
 size_t conv1d_ws_bytes(const tsk_tensor *w, const tsk_tensor *x) {
     return conv_pack_bytes(w) + conv_cast_bytes(w->type, x->type == TSK_TYPE_F32, w->ne[1], x->ne[1], x->ne[2], w->ne[2]);
 }
@@ -1302,11 +1387,15 @@ extern "C" int tsk_conv1d(const tsk_tensor *w, const tsk_tensor *bias, const tsk
     hipStream_t s = (hipStream_t) stream;
     char *ws = nullptr;
     const int x_f32 = x->type == TSK_TYPE_F32;
+    const bool xf32 = conv1d_xf32(w, x);
     const size_t cast = conv_cast_bytes(w->type, x_f32, w->ne[1], x->ne[1], x->ne[2], w->ne[2]);
     const size_t need = conv1d_ws_bytes(w, x);
     const F32Split sp = plan_conv_split(w, x, s0, p0, d0, dst);
     const bool split = sp.on && (ws = Scratch{s, nullptr, 0}.optional(need + sp.bytes));
-    if (!split && (rc = workspace(s, need, (void **) &ws))) return rc;
+    int splits = 1;
+    const size_t pbytes = conv1d_part_bytes(w, x, s0, p0, d0, dst, &splits);
+    const bool sliced = pbytes && (ws = Scratch{s, nullptr, 0}.optional(need + pbytes));
+    if (!split && !sliced && (rc = workspace(s, need, (void **) &ws))) return rc;
     uint16_t *xcast = cast ? (uint16_t *) ws : nullptr;
     char *pk = ws + cast;
     const void *wr = nullptr;
@@ -1326,7 +1415,8 @@ extern "C" int tsk_conv1d(const tsk_tensor *w, const tsk_tensor *bias, const tsk
     return conv_gemm(w->type, wr, nullptr, ld_w, bias ? (const float *) bias->data : nullptr, (int) w->ne[0],
                      (int) w->ne[1], (int) w->ne[2], x->data, x_f32, (int64_t) (x->nb[1] / esx),
                      (int64_t) (x->nb[2] / esx), (int) x->ne[1], (int) x->ne[2], s0, p0, d0, dst->data,
-                     dst->type == TSK_TYPE_BF16, (int64_t) (dst->nb[1] / esy), xcast, s);
+                     dst->type == TSK_TYPE_BF16, (int64_t) (dst->nb[1] / esy), xcast, s,
+                     sliced ? (float *) (ws + need) : nullptr, splits, xf32);
 }
 
 extern "C" int tsk_swiglu(const tsk_tensor *a, const tsk_tensor *b, tsk_tensor *dst, tsk_stream stream) {
@@ -1365,12 +1455,16 @@ struct SwigluSplit {
     bool on;
     F32Split a, b;
     size_t bytes;
+    int splits2;             // BF16 kernels: K slices of w2 and their scratch (bytes), 1: none
 };
 SwigluSplit plan_swiglu_split(const tsk_tensor *w1, int KW1, int IC, int HID, int KW2, int OC, int pad, int IW, int B,
                               bool y_bf16) {
     SwigluSplit q;
     memset(&q, 0, sizeof(q));
     const int64_t OW1 = conv_out_len(IW, KW1, 1, pad, 1), OW2 = conv_out_len(OW1, KW2, 1, pad, 1);
+    q.splits2 = 1;
+    if (w1->type == TSK_TYPE_BF16 && OW1 >= 1 && OW2 >= 1 && conv_coop(w1->type, HID, OC))
+        q.bytes = coop_part_bytes(OC, B * OW2, (int64_t) KW2 * HID, HID, y_bf16, &q.splits2);
     if (w1->type != TSK_TYPE_F32 || OW1 < 1 || OW2 < 1 || KW1 - 1 > SPLIT_HALO || KW2 - 1 > SPLIT_HALO) return q;
     q.a = plan_f32_split(2 * (int64_t) HID, B * OW1, (int64_t) KW1 * IC, (int64_t) B * IW, IC, KW1 - 1, false, true);
     q.b = plan_f32_split(OC, B * OW2, (int64_t) KW2 * HID, B * OW1, HID, KW2 - 1, y_bf16);
@@ -1395,8 +1489,8 @@ int swiglu_mlp(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2,
     int rc;
     const size_t need = swiglu_mlp_ws_bytes(w1, w3, w2, KW1, IC, HID, pad, x_f32, IW, B);
     const SwigluSplit sp = plan_swiglu_split(w1, KW1, IC, HID, KW2, OC, pad, IW, B, y_bf16);
-    const bool split = sp.on && (ws = Scratch{s, nullptr, 0}.optional(need + sp.bytes));
-    if (!split && (rc = workspace(s, need, (void **) &ws))) return rc;
+    const bool more = sp.bytes && (ws = Scratch{s, nullptr, 0}.optional(need + sp.bytes)), split = more && sp.on;
+    if (!more && (rc = workspace(s, need, (void **) &ws))) return rc;
     void *h = ws;
     float *h3 = bf16 ? nullptr : (float *) (ws + hbytes);
     uint16_t *xcast = cast ? (uint16_t *) (ws + hbytes + h3bytes) : nullptr;
@@ -1452,7 +1546,7 @@ int swiglu_mlp(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2,
         if (e != hipSuccess) return hip_fail(e, "swiglu launch");
     }
     return conv_gemm(w2->type, r2, nullptr, ld2, nullptr, KW2, HID, OC, h, !bf16, HID, (int64_t) OW1 * HID, OW1, B, 1,
-                     pad, 1, y, y_bf16, ld_y, nullptr, s);
+                     pad, 1, y, y_bf16, ld_y, nullptr, s, more ? (float *) (ws + need) : nullptr, sp.splits2);
 }
 
 int check_mlp_types(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2, const tsk_tensor *x) {
@@ -1630,7 +1724,7 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
             if ((rc = need(2)) || (rc = validate_mul_mat(&t[0], &t[1], opt(2), &d))) return rc;
         {
             const MulMatPlan pl = plan_mul_mat(&t[0], &t[1], &d);
-            *bytes = std::max(pl.bytes, pl.split.bytes);
+            *bytes = std::max(pl.bytes + pl.part_bytes, pl.split.bytes);
             return TSK_OK;
         }
         case TSK_OP_FLASH_ATTN_EXT:
@@ -1640,8 +1734,12 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
             return TSK_OK;
         case TSK_OP_CONV1D:
             if ((rc = need(2)) || (rc = validate_conv(&t[0], opt(2), &t[1], 1, 1, 1, &d))) return rc;
-            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + plan_conv_split(&t[0], &t[1], 1, 1, 1, &d).bytes;
+        {
+            int sp;
+            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + plan_conv_split(&t[0], &t[1], 1, 1, 1, &d).bytes +
+                     conv1d_part_bytes(&t[0], &t[1], 1, 1, 1, &d, &sp);
             return TSK_OK;
+        }
         case TSK_OP_CONV_MLP_SWIGLU:
             if ((rc = need(4)) || (rc = validate_conv_mlp(&t[0], &t[1], &t[2], &t[3], &d))) return rc;
             *bytes = swiglu_mlp_ws_bytes(&t[0], &t[1], &t[2], (int) t[0].ne[0], (int) t[0].ne[1], (int) t[0].ne[2], 1,
