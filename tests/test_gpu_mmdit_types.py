@@ -5,7 +5,7 @@ types, and the GGUF loader (ts_dit::load, src/mmdit.cpp:104-116):
 - Q8_0 (convert/quantize_gguf.py:9-15): 2-D linears with ne0 % 32 == 0 as
   Q8_0 x Q8_0 products (qkv, every adaLN, the text stream's linear1 / MLP,
   the input and conditioning linears), the 3-D convolution kernels and the
-  t_embed MLP F32 (the convolutions as three bf16 products each by default,
+  t_embed MLP F32 (the convolutions as three fp16 products of split operands by default,
   the t_embed MLP as fp32 products);
 - F32 (the F32 GGUF, the "GGML F32 path" of the accuracy targets);
 - files read by tsk_mmdit_create_from_gguf: a Q8_0 GGUF and a BF16 GGUF give
@@ -141,8 +141,8 @@ def test_f32_graph_forward(env):
 
 
 def test_f32_split_products(env, monkeypatch):
-    """F32 matrices as three bf16 products (the default, TSK_F32_SPLIT=1: the
-    weight's planes [hi | lo | hi] against the rows' [hi | hi | lo]) against
+    """F32 matrices as three fp16 products of split operands (the default,
+    TSK_F32_SPLIT=1) against
     fp32 MFMA products (TSK_F32_SPLIT=0, read on every call) in the same
     model, at the 9 s token counts. The latent input projection (x_in: a k3
     convolution and a convMLP, every kernel F32 in both GGUFs, no attention)

@@ -88,15 +88,10 @@ def test_vae_reference_channels(env):
 
 
 def test_vae_split_products(env, monkeypatch):
-    """The opt-in split products (TSK_VAE_SPLIT=1 when the model is created:
-    every convolution but the output one as three bf16 products over weight
-    planes [hi | lo | hi] and input planes [hi | hi | lo], which the previous
-    convolution's epilogue writes with its SnakeBeta): about 2^-17 of |x w|
-    per term, which the decoder amplifies 50-100 times on its way to the audio
-    (fp32 products: ~6e-5 from the oracle), so the audio is held to 1e-3;
-    TSK_VAE_SPLIT=0 on the same model (read on every call) is the fp32 path
-    again, held to TOL. The split planes' layout is checked by the same
-    comparison: a plane in the wrong place moves the audio by O(1)."""
+    """The split products run in every model now (three fp16 products of
+    scaled halves); TSK_VAE_SPLIT, once their switch, must change nothing:
+    the audio stays within 1e-3 with it set and within TOL without. A split
+    operand in the wrong place moves the audio by O(1)."""
     tsk, orc = env
     monkeypatch.setenv("TSK_VAE_SPLIT", "1")
     tsk.init(0, reread=True)

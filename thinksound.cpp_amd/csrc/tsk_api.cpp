@@ -501,15 +501,16 @@ hipError_t coop_sliced(GemmGroup &g, float *part, int splits, bool xf32, hipStre
 }
 // f32 activations of BF16 weights rounded inside the product's kernel instead
 // of by a launch before it: the launch and its pass over memory against twice
-// the activation bytes and the conversions in every tile. Up to 4000 64 x 64
-// x 64 tile steps, more for narrow linear layers, whose rows few tiles share
-// (us with the launch / without: K = 1024, N = 388, M = 1024 11.4 / 9.5, 3072
-// 12.3 / 12.4 on new inputs, 6144 16.5 / 17.6; N = 2080, M = 1024 19.7 / 16.7; K = 64 7.5 /
-// 4.0; k3 convolution of 1292 rows 29 / 36)
-bool coop_xf32(int64_t M, int64_t N, int64_t K, int64_t ic, int64_t ld_w) {
+// the activation bytes in a ring of two stages. That ring hides less of the
+// weights' latency, so only products (or K slices) of few 64-wide stages run
+// so: up to 4 (weights from memory, us with the launch / without: K = 64, 388
+// rows 6.0 / 4.5, K = 192 convolution of 1292 rows 8.3 / 7.3; K = 1024, 64 rows
+// 10.3 / 11.2, K = 2048 15.3 / 19.4), and up to 16 where K slices stand in for
+// one long product (K = 2816, 64 rows 19.1 / 12.0, K = 4096, 388 rows 32 / 21)
+bool coop_xf32(int64_t M, int64_t N, int64_t K, int64_t ic, int64_t ld_w, int splits) {
     if (K % 64 || ic % 64 || ld_w % 8) return false;
-    const int64_t steps = ((M + 63) / 64) * ((N + 63) / 64) * (K / 64);
-    return steps <= (M <= 1024 && !ic ? 15000 : 4000);
+    const int64_t stages = K / 64, steps = ((M + 63) / 64) * ((N + 63) / 64) * stages;
+    return stages / splits <= (splits > 1 ? 16 : 4) && steps <= (M <= 1024 && !ic ? 15000 : 4000);
 }
 SplitRows split_job(const F32Rows &r, int halo, char *y, char *e) {
     SplitRows j;
@@ -566,8 +567,7 @@ struct MulMatPlan {
     int64_t nslices, Nslice;
     bool gemv;           // a few rows, no scratch
     bool coop;           // BF16 weights on the cooperative tiles
-    bool xf32;           // coop with f32 b: rounded in the kernel, or
-    size_t cast_bytes;   // b rounded to bf16 rows
+    size_t cast_bytes;   // coop with f32 b: b rounded to bf16 rows
     size_t part_bytes;   // coop in K slices, if their scratch can be had as well
     int splits;
     size_t wbytes;       // Q8_0: the weights repacked into planes
@@ -591,8 +591,7 @@ MulMatPlan plan_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tens
     pl.gemv = pl.uni && pl.Nslice <= (a->type == TSK_TYPE_F32 || M <= 2048 ? GEMV_MAX_ROWS : 4);
     if (pl.gemv && a->type != TSK_TYPE_Q8_0) return pl;      // (Q8_0 blocks are repacked first)
     pl.coop = a->type == TSK_TYPE_BF16 && pl.uni && M % 16 == 0 && K % 32 == 0 && a->nb[1] % 16 == 0;
-    pl.xf32 = pl.coop && b->type == TSK_TYPE_F32 && coop_xf32(M, pl.Nslice, K, 0, (int64_t) (a->nb[1] / 2));
-    // (asked for in either case: one size per node, whatever the route)
+    // (asked for also where the kernel rounds them: one size per node, whatever the route)
     if (pl.coop && b->type == TSK_TYPE_F32) pl.cast_bytes = align256((size_t) (pl.Nslice * K) * 2);
     if (a->type == TSK_TYPE_Q8_0 || a->type == TSK_TYPE_Q8_0_SPLIT) {
         pl.wbytes = a->type == TSK_TYPE_Q8_0 ? align256(tsk_q8_0_split_nbytes(K, M)) : 0;
@@ -600,6 +599,7 @@ MulMatPlan plan_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tens
         pl.act_bytes = align256(pl.act_bytes);
     }
     pl.bytes = pl.cast_bytes + pl.wbytes + pl.act_bytes;
+    pl.splits = 1;
     if (pl.coop) pl.part_bytes = coop_part_bytes(M, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16, &pl.splits);
     if (a->type == TSK_TYPE_F32 && pl.uni)
         pl.split = plan_f32_split(M, pl.Nslice, K, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16);
@@ -654,7 +654,9 @@ int mul_mat_impl(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bia
         uint16_t *xb = nullptr;
         const int64_t N = Nslice;
         const int64_t ld_b = (int64_t) (b->nb[1] / es_b);
-        if (b->type == TSK_TYPE_F32 && !pl.xf32) {
+        const bool xf32 = b->type == TSK_TYPE_F32 &&
+                          coop_xf32(M, N, K, 0, (int64_t) (a->nb[1] / 2), sliced ? pl.splits : 1);
+        if (b->type == TSK_TYPE_F32 && !xf32) {
             xb = (uint16_t *) ws;
             hipError_t e = launch_cast_rows_bf16((const float *) b->data, ld_b, 0, (int) std::min<int64_t>(N, 1 << 30), N,
                                                  (int) K, xb, s);
@@ -673,8 +675,8 @@ int mul_mat_impl(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bia
         q.ld_y = (int64_t) (dst->nb[1] / es_d);
         q.M = (int) M; q.N = (int) N; q.K = (int) K; q.splits = 1;
         const int epi = dst->type == TSK_TYPE_BF16 ? EPI_STORE_BF16 : EPI_STORE_F32;
-        hipError_t e = sliced ? coop_sliced(g, (float *) (ws + pl.bytes), pl.splits, pl.xf32, s)
-                     : pl.xf32 ? launch_gemm_coop_xf32(g, epi, s) : launch_gemm_coop(g, epi, s);
+        hipError_t e = sliced ? coop_sliced(g, (float *) (ws + pl.bytes), pl.splits, xf32, s)
+                     : xf32 ? launch_gemm_coop_xf32(g, epi, s) : launch_gemm_coop(g, epi, s);
         return e == hipSuccess ? TSK_OK : hip_fail(e, "mul_mat launch");
     }
 
@@ -1309,10 +1311,11 @@ size_t conv1d_part_bytes(const tsk_tensor *w, const tsk_tensor *x, int s0, int p
 }
 
 // scratch of tsk_conv1d: the kw-major kernel copy and the bf16 input rows
-bool conv1d_xf32(const tsk_tensor *w, const tsk_tensor *x) {
+bool conv1d_xf32(const tsk_tensor *w, const tsk_tensor *x, int splits) {
     const int64_t K = w->ne[0] * w->ne[1];
     return conv_coop(w->type, (int) w->ne[1], (int) w->ne[2]) && x->type == TSK_TYPE_F32 &&
-           coop_xf32(w->ne[2], x->ne[1] * x->ne[2], K, w->ne[1], kw_major(w) && w->ne[2] > 1 ? (int64_t) (w->nb[2] / 2) : K);
+           coop_xf32(w->ne[2], x->ne[1] * x->ne[2], K, w->ne[1], kw_major(w) && w->ne[2] > 1 ? (int64_t) (w->nb[2] / 2) : K,
+                     splits);
 }
 size_t conv1d_ws_bytes(const tsk_tensor *w, const tsk_tensor *x) {
     return conv_pack_bytes(w) + conv_cast_bytes(w->type, x->type == TSK_TYPE_F32, w->ne[1], x->ne[1], x->ne[2], w->ne[2]);
@@ -1387,7 +1390,6 @@ extern "C" int tsk_conv1d(const tsk_tensor *w, const tsk_tensor *bias, const tsk
     hipStream_t s = (hipStream_t) stream;
     char *ws = nullptr;
     const int x_f32 = x->type == TSK_TYPE_F32;
-    const bool xf32 = conv1d_xf32(w, x);
     const size_t cast = conv_cast_bytes(w->type, x_f32, w->ne[1], x->ne[1], x->ne[2], w->ne[2]);
     const size_t need = conv1d_ws_bytes(w, x);
     const F32Split sp = plan_conv_split(w, x, s0, p0, d0, dst);
@@ -1395,6 +1397,7 @@ extern "C" int tsk_conv1d(const tsk_tensor *w, const tsk_tensor *bias, const tsk
     int splits = 1;
     const size_t pbytes = conv1d_part_bytes(w, x, s0, p0, d0, dst, &splits);
     const bool sliced = pbytes && (ws = Scratch{s, nullptr, 0}.optional(need + pbytes));
+    const bool xf32 = conv1d_xf32(w, x, sliced ? splits : 1);
     if (!split && !sliced && (rc = workspace(s, need, (void **) &ws))) return rc;
     uint16_t *xcast = cast ? (uint16_t *) ws : nullptr;
     char *pk = ws + cast;
