@@ -253,3 +253,24 @@ def test_conv1d_bf16_f32_rows_and_slices(env, B, IW, IC, OC, KW, s0, p0, d0):
     got = tsk.conv1d(wd, tsk.to_device(x), bd, s0, p0, d0).numpy()
     assert rel_l2(got, orc.conv1d(w, x, bias, s0, p0, d0, w_type=orc.BF16)) <= 2e-6
     assert np.array_equal(got, tsk.conv1d(wd, tsk.bf16_to_device(orc.f32_to_bf16_bits(x)), bd, s0, p0, d0).numpy())
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_conv1d_single_row_any_stride(env, bf16):
+    """one output row whose row stride is no multiple of 16 bytes (a single row's stride says nothing) in K slices and
+    as split products: the result of a plain row"""
+    import ctypes
+    tsk, orc = env
+    rng = np.random.default_rng(7)
+    w, x = kernel(orc, rng, 64, 1024, 3, bf16=bf16), rng.standard_normal((1, 1, 1024)).astype(np.float32)
+    wd, xd = (tsk.bf16_to_device if bf16 else tsk.to_device)(w), tsk.to_device(x)
+    ref = tsk.conv1d(wd, xd).numpy()
+    out = tsk.empty((1, 1, 64))
+    d, dw, dx = tsk.desc(out, tsk.F32), tsk.desc(wd, tsk.BF16 if bf16 else tsk.F32), tsk.desc(xd, tsk.F32)
+    for t in (d, dx):
+        t.nb[1] = 4 * 1025 + 4
+        t.nb[2] = t.nb[3] = t.nb[1]
+    tsk.check(tsk.load().tsk_conv1d(ctypes.byref(dw), None, ctypes.byref(dx), 1, 1, 1, ctypes.byref(d), None))
+    tsk.synchronize()
+    assert np.array_equal(out.numpy(), ref)
+    assert rel_l2(ref, orc.conv1d(w, x, w_type=orc.BF16 if bf16 else orc.F32)) <= (3e-4 if bf16 else 1e-5)

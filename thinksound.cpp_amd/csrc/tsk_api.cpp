@@ -494,7 +494,7 @@ hipError_t coop_sliced(GemmGroup &g, float *part, int splits, bool xf32, hipStre
     GemmProblem &q = g.p[0];
     const float *bias = q.bias;
     float *y = (float *) q.y;
-    const int64_t ld_y = q.ld_y;
+    const int64_t ld_y = q.N == 1 ? q.M : q.ld_y;            // (a single row's stride may be anything)
     q.bias = nullptr; q.y = part; q.ld_y = q.M; q.splits = splits;
     const hipError_t e = xf32 ? launch_gemm_coop_xf32(g, EPI_PARTIAL, s) : launch_gemm_coop(g, EPI_PARTIAL, s);
     return e == hipSuccess ? launch_sum_slices(part, splits, (int64_t) q.N * q.M, bias, q.N, q.M, y, ld_y, s) : e;
@@ -515,7 +515,8 @@ bool coop_xf32(int64_t M, int64_t N, int64_t K, int64_t ic, int64_t ld_w, int sp
 SplitRows split_job(const F32Rows &r, int halo, char *y, char *e) {
     SplitRows j;
     memset(&j, 0, sizeof(j));
-    j.x = r.x; j.ld_x = r.rows_b == 1 ? 0 : r.ld; j.ld_b = r.ld_b; j.rows_b = r.rows_b;
+    j.x = r.x; j.ld_x = r.rows_b == 1 || r.rows == 1 ? 0 : r.ld;   // (a single row's stride may be anything)
+    j.ld_b = r.ld_b; j.rows_b = r.rows_b;
     j.rows = r.rows; j.cols = r.cols; j.halo = halo;
     j.y = (uint32_t *) y; j.e = (int *) e;
     return j;
@@ -531,7 +532,7 @@ int run_f32_split(const F32Split &pl, char *ws, const F32Rows &w, const float *w
     q.we = (const int *) (ws + pl.we);
     q.xe = (const int *) (ws + pl.xe); q.xe_per_row = 1;
     q.bias = bias;
-    q.y = y; q.ld_y = ld_y; q.y_bf16 = y_bf16;
+    q.y = y; q.ld_y = N == 1 ? M : ld_y; q.y_bf16 = y_bf16;
     q.M = (int) M; q.N = (int) N; q.K = w.cols;
     q.splits = splits; q.part_stride = part_stride;
     if (cv.KW) {
@@ -557,7 +558,8 @@ int f32_split(const F32Split &pl, char *ws, const F32Rows &w, int64_t N, const F
     int rc = run_f32_split(pl, ws, w, nullptr, (int) M, M, N, x, cv, sl ? nullptr : bias, sl ? ws + pl.part : y, y_bf16,
                            sl ? M : ld_y, pl.splits, N * M, s);
     if (rc || !sl) return rc;
-    e = launch_sum_slices((const float *) (ws + pl.part), pl.splits, N * M, bias, N, (int) M, (float *) y, ld_y, s);
+    e = launch_sum_slices((const float *) (ws + pl.part), pl.splits, N * M, bias, N, (int) M, (float *) y,
+                          N == 1 ? M : ld_y, s);
     return e == hipSuccess ? TSK_OK : hip_fail(e, "f32 split sum");
 }
 
@@ -1256,6 +1258,8 @@ int conv_gemm(int wtype, const void *wrows, const void *w3rows, int64_t ld_w, co
               int y_bf16, int64_t ld_y, uint16_t *xcast, hipStream_t s, float *part = nullptr, int splits = 1,
               bool xf32 = false) {
     const int OW = (int) conv_out_len(IW, KW, s0, p0, d0);
+    if (IW == 1) ld_x = IC;                      // (a single row's or item's stride may be anything)
+    if (B == 1) xb = 0;
     const bool coop = conv_coop(wtype, IC, OC) && (!x_f32 || xcast || xf32) && ld_w % 8 == 0 &&
                       ((uintptr_t) wrows & 15) == 0 && ((uintptr_t) w3rows & 15) == 0;
     if (coop && x_f32 && !xf32) {
@@ -1532,7 +1536,8 @@ int swiglu_mlp(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2,
         rc = run_f32_split(sp.b, wb, f2, nullptr, OC, OC, N2, hr, F32Conv{KW2, OW1, OW2, 1, pad, 1}, nullptr,
                            sl ? (void *) (wb + sp.b.part) : y, y_bf16, sl ? OC : ld_y, sp.b.splits, N2 * OC, s);
         if (rc || !sl) return rc;
-        e = launch_sum_slices((const float *) (wb + sp.b.part), sp.b.splits, N2 * OC, nullptr, N2, OC, (float *) y, ld_y, s);
+        e = launch_sum_slices((const float *) (wb + sp.b.part), sp.b.splits, N2 * OC, nullptr, N2, OC, (float *) y,
+                              N2 == 1 ? OC : ld_y, s);
         return e == hipSuccess ? TSK_OK : hip_fail(e, "f32 split sum");
     }
     if (bf16) {
