@@ -349,10 +349,7 @@ int tsk_supports_op(int op, const tsk_tensor *const *srcs, int n_srcs,
  * (tsk_set_workspace); 0 for operators that need none. Validates the
  * descriptors like the entry point (data pointers are not inspected) and
  * returns its status. Counterpart of a ggml backend's buffer sizing
- * (ggml_backend_buft_get_alloc_size); srcs as for tsk_supports_op. For F32
- * weights the size is that of the split products; with a smaller bound buffer
- * (or one that would have to grow while the stream is captured) the node runs
- * as fp32 products, slower. */
+ * (ggml_backend_buft_get_alloc_size); srcs as for tsk_supports_op. */
 int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_srcs,
                        const tsk_tensor *dst, size_t *bytes);
 

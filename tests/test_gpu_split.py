@@ -1,5 +1,8 @@
-"""F32 products on the fp16 matrix cores (split operands, csrc/gemm_split.hip)
-at the sizes where the tiles, taps and exponents can go wrong."""
+"""F32 products on the 16-bit matrix cores (operands in bf16 parts,
+csrc/gemm_f32x6.hip) at the sizes where the tiles and taps can go wrong, and
+over operands whose values differ widely in size."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -62,7 +65,7 @@ def test_vae_split_nan_stays_local(vae):
 # ---------------------------------------------------------------- F32 nodes
 def rows_close(got, w, x, bound):
     """every output row against 64-bit products, relative to |w| |x| of its own row (its sum's condition):
-    operands to 2^-23, the products left out 2^-22, both with random signs, and sums of K terms in fp32"""
+    exact operands, products left out 2^-25, and sums of K terms in fp32"""
     ref = x.astype(np.float64) @ w.astype(np.float64).T
     scale = np.sqrt(((np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T) ** 2).sum(-1))
     err = np.sqrt(((got - ref) ** 2).sum(-1)) / np.maximum(scale, 1e-300)
@@ -70,10 +73,10 @@ def rows_close(got, w, x, bound):
     return err.max() <= bound
 
 
-@pytest.mark.parametrize("N,K,M", [(1, 448, 4), (63, 480, 132), (65, 1024, 128), (129, 2080, 64), (388, 4096, 96),
+@pytest.mark.parametrize("N,K,M", [(9, 32, 4), (63, 480, 132), (65, 1024, 128), (129, 2080, 64), (388, 4096, 96),
                                    (600, 512, 1028)])
 def test_mul_mat_split(env, N, K, M):
-    """remainders of every tile and of the K slices; rows and weights of very different size keep their own precision"""
+    """remainders of every tile and of the K halves; rows and weights of very different size keep their own precision"""
     tsk, _ = env
     rng = np.random.default_rng(N + K)
     x = (rng.standard_normal((N, K)) * 2.0 ** rng.integers(-40, 40, (N, 1))).astype(np.float32)
@@ -124,22 +127,84 @@ def test_split_infinities(env):
     assert np.array_equal(y[same], clean[same])
 
 
-def test_split_without_scratch(env):
-    """a bound workspace too small for the split products: fp32 products, as before"""
-    tsk, orc = env
+@pytest.mark.parametrize("p", [20, 30, 60])
+def test_mul_mat_outlier(env, p):
+    """one input column 2^p above the rest against zero weights: it may cost the others nothing. Bound: the sums'
+    (2^-24 sqrt(K) of the terms at most)"""
+    tsk, _ = env
+    rng = np.random.default_rng(p)
+    x, w = rng.standard_normal((70, 1024)).astype(np.float32), rng.standard_normal((132, 1024)).astype(np.float32)
+    x[:, 7] *= 2.0 ** p
+    w[:, 7] = 0
+    y = tsk.mul_mat(tsk.to_device(w), tsk.to_device(x)).numpy()
+    assert rows_close(y, w, x, 2.0 ** -24)
+
+
+def test_mul_mat_spread_undone_by_the_weights(env):
+    """values of a row spread over 2^60 that the weights undo: every product counts the same"""
+    tsk, _ = env
+    rng = np.random.default_rng(4)
+    e = rng.integers(-30, 31, 1024)
+    x = (rng.standard_normal((70, 1024)) * 2.0 ** e).astype(np.float32)
+    w = (rng.standard_normal((68, 1024)) * 2.0 ** -e).astype(np.float32)
+    y = tsk.mul_mat(tsk.to_device(w), tsk.to_device(x)).numpy()
+    assert rows_close(y, w, x, 2.0 ** -24)
+
+
+def test_mul_mat_copies_values(env):
+    """against a unit matrix every value comes back, all 24 bits of it, whatever the rest of its row is (down to
+    2^-102, where its smallest part meets fp32's smallest normal number)"""
+    tsk, _ = env
+    rng = np.random.default_rng(5)
+    x = (rng.standard_normal((100, 512)) * 2.0 ** rng.integers(-96, 100, (100, 512))).astype(np.float32)
+    assert np.array_equal(tsk.mul_mat(tsk.to_device(np.eye(512, dtype=np.float32)), tsk.to_device(x)).numpy(), x)
+
+
+def test_conv1d_large_rows_beside_small_ones(env):
+    """rows just outside an output's taps do not touch it, however much larger they are (2^170 over three rows here),
+    and zero rows between them change nothing"""
+    tsk, _ = env
+    rng = np.random.default_rng(6)
+    e = np.array([-100, -100, -50, -50, 120, 120, 0, -100, 0, 45, 45, -60])
+    x = (rng.standard_normal((1, 12, 512)) * 2.0 ** e[None, :, None]).astype(np.float32)
+    x[0, 8] = 0
+    w = (rng.standard_normal((64, 512, 3)) * 0.05).astype(np.float32)
+    y = tsk.conv1d(tsk.to_device(w), tsk.to_device(x)).numpy().reshape(12, 64)
+    xp = np.concatenate([np.zeros((1, 512), np.float32), x[0], np.zeros((1, 512), np.float32)])
+    cols = np.concatenate([xp[k:k + 12] for k in range(3)], 1)
+    assert rows_close(y, w.transpose(0, 2, 1).reshape(64, -1), cols, 2.0 ** -23)
+
+
+def test_f32_nodes_need_no_scratch(env):
+    """F32 weights (kernels laid out kw-major): no workspace, and the same bits whatever is bound to the stream and
+    when the call is captured"""
+    tsk, _ = env
     rng = np.random.default_rng(3)
     x, w = rng.standard_normal((100, 512)).astype(np.float32), rng.standard_normal((64, 512)).astype(np.float32)
     xd, wd, y = tsk.to_device(x), tsk.to_device(w), tsk.empty((100, 64))
-    n = tsk.workspace_size(tsk.OP_MUL_MAT, [wd, xd], y)
-    s = tsk.Stream()
-    outs = []
-    for size in (n, n - 256):
-        buf = tsk.empty((size,), "u8")
-        tsk.set_workspace(buf, stream=s)
-        tsk.mul_mat(wd, xd, out=y, stream=s)
-        s.synchronize()
-        outs.append(y.numpy())
-        assert rel_l2(outs[-1], orc.mul_mat(w, x)) <= 1e-5
-    assert not np.array_equal(*outs)                              # two sets of products
+    assert tsk.workspace_size(tsk.OP_MUL_MAT, [wd, xd], y) == 0
+    kd = tsk.to_device(np.ascontiguousarray(rng.standard_normal((32, 3, 128)).astype(np.float32)))
+    kw, xc, yc = tsk.desc(kd, tsk.F32), tsk.to_device(x.reshape(1, 400, 128)), tsk.empty((1, 400, 32))
+    kw.ne[0], kw.ne[1], kw.ne[2] = 3, 128, 32
+    kw.nb[0], kw.nb[1], kw.nb[2], kw.nb[3] = 4 * 128, 4, 4 * 384, 4 * 384 * 32
+    dx, dy = tsk.desc(xc, tsk.F32), tsk.desc(yc, tsk.F32)
+    n = ctypes.c_size_t(1)
+    srcs = (ctypes.POINTER(type(kw)) * 2)(ctypes.pointer(kw), ctypes.pointer(dx))
+    tsk.check(tsk.load().tsk_workspace_size(tsk.OP_CONV1D, srcs, 2, ctypes.byref(dy), ctypes.byref(n)))
+    assert n.value == 0
+    tsk.mul_mat(wd, xd, out=y)
+    tsk.synchronize()
+    ref = y.numpy()
+    s, buf = tsk.Stream(), tsk.empty((256,), "u8")
+    tsk.set_workspace(buf, stream=s)
+    tsk.mul_mat(wd, xd, out=y, stream=s)
+    s.synchronize()
+    assert np.array_equal(y.numpy(), ref)
     tsk.set_workspace(None, stream=s)
+    g = tsk.Graph(s, lambda: tsk.mul_mat(wd, xd, out=y, stream=s))
+    for _ in range(3):
+        g.launch()
+        s.synchronize()
+        assert np.array_equal(y.numpy(), ref)
+    g.destroy()
     s.destroy()

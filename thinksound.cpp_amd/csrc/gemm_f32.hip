@@ -415,6 +415,7 @@ hipError_t launch_gemm_f32(const GemmProblem &p, int y_bf16, hipStream_t s, cons
     if (p.conv_ic && (p.conv_ic % 4 || p.K % p.conv_ic || p.x_group_rows || p.conv_ow < 1 || p.conv_iw < 1 ||
                       p.conv_s < 1 || p.conv_d < 1 || p.conv_p < 0 || p.N % p.conv_ow))
         return hipErrorInvalidValue;
+    if ((snake || !p.accumulate) && gemm_f32x6_fits(p)) return launch_gemm_f32x6(p, y_bf16, s, snake);
     // 128 x 128 workgroup tiles (4 x 4 per wave, 72 KiB of LDS: two workgroups
     // per CU) where there are enough such tiles: unsplit products (the VAE's
     // convolutions, k7 at 128-1024 channels 62.5-67.7 -> 69.7-74.2 % of the

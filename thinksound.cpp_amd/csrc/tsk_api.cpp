@@ -437,52 +437,6 @@ struct Scratch {
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t) 255; }
 
-// F32 products on the fp16 matrix cores (gemm_split.hip): the weights and the
-// activations split into scratch in one launch, the product, and where its
-// tiles are few the sum of its K slices. A call whose stream has no room for
-// the scratch runs on fp32 MFMAs instead.
-struct F32Rows {           // f32 rows in memory
-    const float *x;
-    int64_t ld, ld_b;
-    int rows_b;            // rows per batch item (0: plain rows)
-    int64_t rows;
-    int cols;
-};
-struct F32Conv {           // the rows' convolution (KW = 0: none)
-    int KW, IW, OW, s, p, d;
-};
-struct F32Split {
-    bool on;
-    int splits;
-    size_t w, x, we, xe, part, bytes;    // offsets into the scratch
-};
-F32Split plan_f32_split(int64_t M, int64_t N, int64_t K, int64_t x_rows, int64_t cols, int halo, bool y_bf16,
-                        bool always_part = false) {
-    F32Split pl;
-    memset(&pl, 0, sizeof(pl));
-    // K from 448: the fp32 kernel's time is its K chain, 0.042 us per k (1024
-    // outputs, 128 rows: K = 448 22.9 against 21.6 us, K = 320 17.4 against
-    // 18.7, K = 3072 at 1292 rows 150 against 50). Over few rows of large
-    // weights the split pass alone moves more than that kernel does (3 rows:
-    // 2^25 weights 171 against 85 us, 2^27 297 against 363).
-    pl.on = tuning().f32_split && K >= 448 && (N >= 512 || M * K <= ((int64_t) 1 << 25)) && cols % 32 == 0 &&
-            halo <= SPLIT_HALO && split_gemm_fits(M, K, x_rows, cols, 2) && x_rows < ((int64_t) 1 << 31);
-    if (!pl.on) return pl;
-    pl.splits = y_bf16 ? 1 : split_gemm_slices(M, N, K, 8);
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        const size_t o = off;
-        off += align256(bytes);
-        return o;
-    };
-    pl.w = take((size_t) (M * K) * 4);
-    pl.x = take((size_t) (x_rows * cols) * 4);
-    pl.we = take((size_t) M * 4);
-    pl.xe = take((size_t) x_rows * 4);
-    pl.part = take(pl.splits > 1 || always_part ? (size_t) pl.splits * (size_t) (N * M) * 4 : 0);
-    pl.bytes = off;
-    return pl;
-}
 // K slices of a BF16 product on the cooperative tiles (f32 result): see
 // coop_slices(); 0 bytes where it runs whole
 size_t coop_part_bytes(int64_t M, int64_t N, int64_t K, int64_t ic, bool y_bf16, int *splits) {
@@ -512,57 +466,6 @@ bool coop_xf32(int64_t M, int64_t N, int64_t K, int64_t ic, int64_t ld_w, int sp
     const int64_t stages = K / 64, steps = ((M + 63) / 64) * ((N + 63) / 64) * stages;
     return stages / splits <= (splits > 1 ? 16 : 4) && steps <= (M <= 1024 && !ic ? 15000 : 4000);
 }
-SplitRows split_job(const F32Rows &r, int halo, char *y, char *e) {
-    SplitRows j;
-    memset(&j, 0, sizeof(j));
-    j.x = r.x; j.ld_x = r.rows_b == 1 || r.rows == 1 ? 0 : r.ld;   // (a single row's stride may be anything)
-    j.ld_b = r.ld_b; j.rows_b = r.rows_b;
-    j.rows = r.rows; j.cols = r.cols; j.halo = halo;
-    j.y = (uint32_t *) y; j.e = (int *) e;
-    return j;
-}
-// the product of split operands at ws + pl: w [M][K] (f32 rows wf, from wf_rows on wf2), x and its convolution
-int run_f32_split(const F32Split &pl, char *ws, const F32Rows &w, const float *wf2, int wf_rows, int64_t M, int64_t N,
-                  const F32Rows &x, const F32Conv &cv, const float *bias, void *y, int y_bf16, int64_t ld_y, int splits,
-                  int64_t part_stride, hipStream_t s) {
-    SplitGemm q;
-    memset(&q, 0, sizeof(q));
-    q.x = (const uint32_t *) (ws + pl.x); q.ld_x = x.cols;
-    q.w = (const uint32_t *) (ws + pl.w); q.ld_w = w.cols;
-    q.we = (const int *) (ws + pl.we);
-    q.xe = (const int *) (ws + pl.xe); q.xe_per_row = 1;
-    q.bias = bias;
-    q.y = y; q.ld_y = N == 1 ? M : ld_y; q.y_bf16 = y_bf16;
-    q.M = (int) M; q.N = (int) N; q.K = w.cols;
-    q.splits = splits; q.part_stride = part_stride;
-    if (cv.KW) {
-        q.conv_ic = x.cols; q.conv_iw = cv.IW; q.conv_ow = cv.OW;
-        q.conv_s = cv.s; q.conv_p = cv.p; q.conv_d = cv.d;
-    }
-    q.xf = x.x; q.ld_xf = x.ld; q.xf_batch = x.ld_b;
-    q.wf = w.x; q.wf2 = wf2; q.wf_rows = wf_rows; q.ld_wf = w.ld;
-    hipError_t e = launch_gemm_split(q, s);
-    return e == hipSuccess ? TSK_OK : hip_fail(e, "f32 split gemm");
-}
-// y = x w (+ bias), scratch ws of pl.bytes
-int f32_split(const F32Split &pl, char *ws, const F32Rows &w, int64_t N, const F32Rows &x, const F32Conv &cv,
-              const float *bias, void *y, int y_bf16, int64_t ld_y, hipStream_t s) {
-    const int64_t M = w.rows;
-    SplitRowsGroup g;
-    g.n = 2;
-    g.j[0] = split_job(w, 0, ws + pl.w, ws + pl.we);
-    g.j[1] = split_job(x, cv.KW > 1 ? (cv.KW - 1) * cv.d : 0, ws + pl.x, ws + pl.xe);
-    hipError_t e = launch_split_rows(g, s);
-    if (e != hipSuccess) return hip_fail(e, "f32 split rows");
-    const bool sl = pl.splits > 1;
-    int rc = run_f32_split(pl, ws, w, nullptr, (int) M, M, N, x, cv, sl ? nullptr : bias, sl ? ws + pl.part : y, y_bf16,
-                           sl ? M : ld_y, pl.splits, N * M, s);
-    if (rc || !sl) return rc;
-    e = launch_sum_slices((const float *) (ws + pl.part), pl.splits, N * M, bias, N, (int) M, (float *) y,
-                          N == 1 ? M : ld_y, s);
-    return e == hipSuccess ? TSK_OK : hip_fail(e, "f32 split sum");
-}
-
 // How tsk_mul_mat runs a validated node, and the scratch it needs.
 struct MulMatPlan {
     bool uni;            // rows of b and dst uniformly strided: one GEMM of Nslice rows
@@ -575,7 +478,6 @@ struct MulMatPlan {
     size_t wbytes;       // Q8_0: the weights repacked into planes
     size_t act_bytes;    // Q8_0 / Q8_0_SPLIT: the quantized activation planes
     size_t bytes;        // scratch the call needs
-    F32Split split;      // F32 weights on the fp16 matrix cores, if its scratch can be had
 };
 
 MulMatPlan plan_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *dst) {
@@ -603,8 +505,6 @@ MulMatPlan plan_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tens
     pl.bytes = pl.cast_bytes + pl.wbytes + pl.act_bytes;
     pl.splits = 1;
     if (pl.coop) pl.part_bytes = coop_part_bytes(M, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16, &pl.splits);
-    if (a->type == TSK_TYPE_F32 && pl.uni)
-        pl.split = plan_f32_split(M, pl.Nslice, K, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16);
     return pl;
 }
 
@@ -638,12 +538,6 @@ int mul_mat_impl(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bia
         q.N = (int) pl.Nslice; q.M = (int) M; q.K = (int) K;
         const hipError_t e = launch_gemv_rows(q, s);
         return e == hipSuccess ? TSK_OK : hip_fail(e, "mul_mat rows launch");
-    }
-    if (pl.split.on && (ws = scr.optional(pl.split.bytes))) {
-        const F32Rows w{(const float *) a->data, (int64_t) (a->nb[1] / 4), 0, 0, M, (int) K};
-        const F32Rows x{(const float *) b->data, (int64_t) (b->nb[1] / 4), 0, 0, pl.Nslice, (int) K};
-        return f32_split(pl.split, ws, w, pl.Nslice, x, F32Conv{}, bias ? (const float *) bias->data : nullptr, dst->data,
-                         dst->type == TSK_TYPE_BF16, (int64_t) (dst->nb[1] / es_d), s);
     }
     const bool sliced = pl.part_bytes && (ws = scr.optional(pl.bytes + pl.part_bytes));
     if (!sliced && (rc = scr.get(pl.bytes, (void **) &ws))) return rc;
@@ -1297,14 +1191,6 @@ int conv_gemm(int wtype, const void *wrows, const void *w3rows, int64_t ld_w, co
     return e == hipSuccess ? TSK_OK : hip_fail(e, "conv GEMM launch");
 }
 
-// F32 kernels on the fp16 matrix cores (after conv1d_ws_bytes)
-F32Split plan_conv_split(const tsk_tensor *w, const tsk_tensor *x, int s0, int p0, int d0, const tsk_tensor *dst) {
-    const int64_t KW = w->ne[0], IC = w->ne[1], OC = w->ne[2], IW = x->ne[1], B = x->ne[2];
-    if (w->type != TSK_TYPE_F32 || (KW - 1) * d0 > SPLIT_HALO) return F32Split{};
-    return plan_f32_split(OC, B * conv_out_len(IW, KW, s0, p0, d0), KW * IC, B * IW, IC, (int) (KW - 1) * d0,
-                          dst->type == TSK_TYPE_BF16);
-}
-
 // BF16 kernels in K slices (after conv1d_ws_bytes)
 size_t conv1d_part_bytes(const tsk_tensor *w, const tsk_tensor *x, int s0, int p0, int d0, const tsk_tensor *dst, int *splits) {
     const int64_t KW = w->ne[0], IC = w->ne[1], OC = w->ne[2];
@@ -1396,29 +1282,17 @@ extern "C" int tsk_conv1d(const tsk_tensor *w, const tsk_tensor *bias, const tsk
     const int x_f32 = x->type == TSK_TYPE_F32;
     const size_t cast = conv_cast_bytes(w->type, x_f32, w->ne[1], x->ne[1], x->ne[2], w->ne[2]);
     const size_t need = conv1d_ws_bytes(w, x);
-    const F32Split sp = plan_conv_split(w, x, s0, p0, d0, dst);
-    const bool split = sp.on && (ws = Scratch{s, nullptr, 0}.optional(need + sp.bytes));
     int splits = 1;
     const size_t pbytes = conv1d_part_bytes(w, x, s0, p0, d0, dst, &splits);
     const bool sliced = pbytes && (ws = Scratch{s, nullptr, 0}.optional(need + pbytes));
     const bool xf32 = conv1d_xf32(w, x, sliced ? splits : 1);
-    if (!split && !sliced && (rc = workspace(s, need, (void **) &ws))) return rc;
+    if (!sliced && (rc = workspace(s, need, (void **) &ws))) return rc;
     uint16_t *xcast = cast ? (uint16_t *) ws : nullptr;
     char *pk = ws + cast;
     const void *wr = nullptr;
     int64_t ld_w = 0;
     if ((rc = conv_weight_rows(w, &pk, &wr, &ld_w, s))) return rc;
     const int esx = elt_size(x->type), esy = elt_size(dst->type);
-    if (split) {
-        const int KW = (int) w->ne[0], IC = (int) w->ne[1], IW = (int) x->ne[1], B = (int) x->ne[2];
-        const F32Rows wrows{(const float *) wr, ld_w, 0, 0, w->ne[2], KW * IC};
-        const F32Rows xrows{(const float *) x->data, (int64_t) (x->nb[1] / 4), B > 1 ? (int64_t) (x->nb[2] / 4) : 0, IW,
-                            (int64_t) B * IW, IC};
-        const int OW = (int) dst->ne[1];
-        return f32_split(sp, ws + need, wrows, (int64_t) B * OW, xrows, F32Conv{KW, IW, OW, s0, p0, d0},
-                         bias ? (const float *) bias->data : nullptr, dst->data, dst->type == TSK_TYPE_BF16,
-                         (int64_t) (dst->nb[1] / esy), s);
-    }
     return conv_gemm(w->type, wr, nullptr, ld_w, bias ? (const float *) bias->data : nullptr, (int) w->ne[0],
                      (int) w->ne[1], (int) w->ne[2], x->data, x_f32, (int64_t) (x->nb[1] / esx),
                      (int64_t) (x->nb[2] / esx), (int) x->ne[1], (int) x->ne[2], s0, p0, d0, dst->data,
@@ -1456,28 +1330,13 @@ size_t swiglu_mlp_ws_bytes(const tsk_tensor *w1, const tsk_tensor *w3, const tsk
            conv_pack_bytes(w3) + conv_pack_bytes(w2);
 }
 
-// F32 kernels on the fp16 matrix cores: w1 | w3 as one product of 2 HID
-// outputs, then w2 of the f32 hidden state h; scratch after swiglu_mlp_ws_bytes
-struct SwigluSplit {
-    bool on;
-    F32Split a, b;
-    size_t bytes;
-    int splits2;             // BF16 kernels: K slices of w2 and their scratch (bytes), 1: none
-};
-SwigluSplit plan_swiglu_split(const tsk_tensor *w1, int KW1, int IC, int HID, int KW2, int OC, int pad, int IW, int B,
-                              bool y_bf16) {
-    SwigluSplit q;
-    memset(&q, 0, sizeof(q));
+// BF16 kernels: K slices of w2 (after swiglu_mlp_ws_bytes)
+size_t swiglu_part_bytes(const tsk_tensor *w1, int KW1, int HID, int KW2, int OC, int pad, int IW, int B, bool y_bf16,
+                         int *splits) {
     const int64_t OW1 = conv_out_len(IW, KW1, 1, pad, 1), OW2 = conv_out_len(OW1, KW2, 1, pad, 1);
-    q.splits2 = 1;
-    if (w1->type == TSK_TYPE_BF16 && OW1 >= 1 && OW2 >= 1 && conv_coop(w1->type, HID, OC))
-        q.bytes = coop_part_bytes(OC, B * OW2, (int64_t) KW2 * HID, HID, y_bf16, &q.splits2);
-    if (w1->type != TSK_TYPE_F32 || OW1 < 1 || OW2 < 1 || KW1 - 1 > SPLIT_HALO || KW2 - 1 > SPLIT_HALO) return q;
-    q.a = plan_f32_split(2 * (int64_t) HID, B * OW1, (int64_t) KW1 * IC, (int64_t) B * IW, IC, KW1 - 1, false, true);
-    q.b = plan_f32_split(OC, B * OW2, (int64_t) KW2 * HID, B * OW1, HID, KW2 - 1, y_bf16);
-    q.on = q.a.on && q.b.on;
-    q.bytes = q.a.bytes + q.b.bytes;
-    return q;
+    *splits = 1;
+    if (OW1 < 1 || OW2 < 1 || !conv_coop(w1->type, HID, OC)) return 0;
+    return coop_part_bytes(OC, B * OW2, (int64_t) KW2 * HID, HID, y_bf16, splits);
 }
 
 // convmlp / mlp on validated operands: geometry of the two convolutions
@@ -1495,9 +1354,10 @@ int swiglu_mlp(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2,
     char *ws = nullptr;
     int rc;
     const size_t need = swiglu_mlp_ws_bytes(w1, w3, w2, KW1, IC, HID, pad, x_f32, IW, B);
-    const SwigluSplit sp = plan_swiglu_split(w1, KW1, IC, HID, KW2, OC, pad, IW, B, y_bf16);
-    const bool more = sp.bytes && (ws = Scratch{s, nullptr, 0}.optional(need + sp.bytes)), split = more && sp.on;
-    if (!more && (rc = workspace(s, need, (void **) &ws))) return rc;
+    int splits2;
+    const size_t pbytes = swiglu_part_bytes(w1, KW1, HID, KW2, OC, pad, IW, B, y_bf16, &splits2);
+    const bool sliced = pbytes && (ws = Scratch{s, nullptr, 0}.optional(need + pbytes));
+    if (!sliced && (rc = workspace(s, need, (void **) &ws))) return rc;
     void *h = ws;
     float *h3 = bf16 ? nullptr : (float *) (ws + hbytes);
     uint16_t *xcast = cast ? (uint16_t *) (ws + hbytes + h3bytes) : nullptr;
@@ -1508,38 +1368,6 @@ int swiglu_mlp(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2,
         (rc = conv_weight_rows(w2, &pk, &r2, &ld2, s)))
         return rc;
     if (ld1 != ld3) return fail(TSK_ERR_STRIDE, "w1 and w3 row strides differ");
-    if (split) {
-        char *wa = ws + need, *wb = wa + sp.a.bytes;
-        const F32Rows f1{(const float *) r1, ld1, 0, 0, HID, KW1 * IC}, f3{(const float *) r3, ld3, 0, 0, HID, KW1 * IC};
-        const F32Rows f2{(const float *) r2, ld2, 0, 0, OC, KW2 * HID};
-        const F32Rows xr{(const float *) x, ld_x, B > 1 ? xb : 0, pad || B > 1 ? IW : 0, (int64_t) B * IW, IC};
-        const F32Rows hr{(const float *) h, HID, (int64_t) OW1 * HID, OW1, (int64_t) B * OW1, HID};
-        const int64_t N1 = (int64_t) B * OW1, N2 = (int64_t) B * OW2;
-        SplitRowsGroup g;
-        g.n = 4;
-        g.j[0] = split_job(f1, 0, wa + sp.a.w, wa + sp.a.we);
-        g.j[1] = split_job(f3, 0, wa + sp.a.w + (size_t) HID * KW1 * IC * 4, wa + sp.a.we + (size_t) HID * 4);
-        g.j[2] = split_job(f2, 0, wb + sp.b.w, wb + sp.b.we);
-        g.j[3] = split_job(xr, KW1 - 1, wa + sp.a.x, wa + sp.a.xe);
-        hipError_t e = launch_split_rows(g, s);
-        if (e != hipSuccess) return hip_fail(e, "f32 split rows");
-        float *p1 = (float *) (wa + sp.a.part);
-        if ((rc = run_f32_split(sp.a, wa, f1, f3.x, HID, 2 * (int64_t) HID, N1, xr, F32Conv{KW1, IW, OW1, 1, pad, 1},
-                                nullptr, p1, 0, 2 * (int64_t) HID, sp.a.splits, N1 * 2 * HID, s)))
-            return rc;
-        e = launch_silu_mul_rows(p1, sp.a.splits, N1 * 2 * HID, N1, HID, (float *) h, s);
-        if (e != hipSuccess) return hip_fail(e, "swiglu launch");
-        g.n = 1;
-        g.j[0] = split_job(hr, KW2 - 1, wb + sp.b.x, wb + sp.b.xe);
-        if ((e = launch_split_rows(g, s)) != hipSuccess) return hip_fail(e, "f32 split rows");
-        const bool sl = sp.b.splits > 1;
-        rc = run_f32_split(sp.b, wb, f2, nullptr, OC, OC, N2, hr, F32Conv{KW2, OW1, OW2, 1, pad, 1}, nullptr,
-                           sl ? (void *) (wb + sp.b.part) : y, y_bf16, sl ? OC : ld_y, sp.b.splits, N2 * OC, s);
-        if (rc || !sl) return rc;
-        e = launch_sum_slices((const float *) (wb + sp.b.part), sp.b.splits, N2 * OC, nullptr, N2, OC, (float *) y,
-                              N2 == 1 ? OC : ld_y, s);
-        return e == hipSuccess ? TSK_OK : hip_fail(e, "f32 split sum");
-    }
     if (bf16) {
         if ((rc = conv_gemm(TSK_TYPE_BF16, r1, r3, ld1, nullptr, KW1, IC, HID, x, x_f32, ld_x, xb, IW, B, 1, pad, 1, h,
                             1, HID, xcast, s)))
@@ -1554,7 +1382,7 @@ int swiglu_mlp(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2,
         if (e != hipSuccess) return hip_fail(e, "swiglu launch");
     }
     return conv_gemm(w2->type, r2, nullptr, ld2, nullptr, KW2, HID, OC, h, !bf16, HID, (int64_t) OW1 * HID, OW1, B, 1,
-                     pad, 1, y, y_bf16, ld_y, nullptr, s, more ? (float *) (ws + need) : nullptr, sp.splits2);
+                     pad, 1, y, y_bf16, ld_y, nullptr, s, sliced ? (float *) (ws + need) : nullptr, splits2);
 }
 
 int check_mlp_types(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2, const tsk_tensor *x) {
@@ -1726,13 +1554,13 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
     d.data = dummy;
     auto opt = [&](int i) -> const tsk_tensor * { return i < n_srcs && srcs[i] ? &t[i] : nullptr; };
     auto need = [&](int n) { return n_srcs >= n ? TSK_OK : fail(TSK_ERR_INVALID_ARG, "op %d needs %d srcs", op, n); };
-    int rc;
+    int rc, sp;
     switch (op) {
         case TSK_OP_MUL_MAT:
             if ((rc = need(2)) || (rc = validate_mul_mat(&t[0], &t[1], opt(2), &d))) return rc;
         {
             const MulMatPlan pl = plan_mul_mat(&t[0], &t[1], &d);
-            *bytes = std::max(pl.bytes + pl.part_bytes, pl.split.bytes);
+            *bytes = pl.bytes + pl.part_bytes;
             return TSK_OK;
         }
         case TSK_OP_FLASH_ATTN_EXT:
@@ -1742,18 +1570,14 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
             return TSK_OK;
         case TSK_OP_CONV1D:
             if ((rc = need(2)) || (rc = validate_conv(&t[0], opt(2), &t[1], 1, 1, 1, &d))) return rc;
-        {
-            int sp;
-            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + plan_conv_split(&t[0], &t[1], 1, 1, 1, &d).bytes +
-                     conv1d_part_bytes(&t[0], &t[1], 1, 1, 1, &d, &sp);
+            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + conv1d_part_bytes(&t[0], &t[1], 1, 1, 1, &d, &sp);
             return TSK_OK;
-        }
         case TSK_OP_CONV_MLP_SWIGLU:
             if ((rc = need(4)) || (rc = validate_conv_mlp(&t[0], &t[1], &t[2], &t[3], &d))) return rc;
             *bytes = swiglu_mlp_ws_bytes(&t[0], &t[1], &t[2], (int) t[0].ne[0], (int) t[0].ne[1], (int) t[0].ne[2], 1,
                                          t[3].type == TSK_TYPE_F32, (int) t[3].ne[1], (int) t[3].ne[2]) +
-                     plan_swiglu_split(&t[0], (int) t[0].ne[0], (int) t[0].ne[1], (int) t[0].ne[2], (int) t[2].ne[0],
-                                       (int) t[2].ne[2], 1, (int) t[3].ne[1], (int) t[3].ne[2], d.type == TSK_TYPE_BF16).bytes;
+                     swiglu_part_bytes(&t[0], (int) t[0].ne[0], (int) t[0].ne[2], (int) t[2].ne[0], (int) t[2].ne[2], 1,
+                                       (int) t[3].ne[1], (int) t[3].ne[2], d.type == TSK_TYPE_BF16, &sp);
             return TSK_OK;
         case TSK_OP_MLP_SWIGLU:
             if ((rc = need(4)) || (rc = validate_mlp(&t[0], &t[1], &t[2], &t[3], &d))) return rc;
@@ -1762,8 +1586,8 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
             const tsk_tensor k1 = linear_as_kernel(&t[0]), k3 = linear_as_kernel(&t[1]), k2 = linear_as_kernel(&t[2]);
             *bytes = swiglu_mlp_ws_bytes(&k1, &k3, &k2, 1, (int) t[0].ne[0], (int) t[0].ne[1], 0,
                                          t[3].type == TSK_TYPE_F32, (int) (t[3].ne[1] * t[3].ne[2] * t[3].ne[3]), 1) +
-                     plan_swiglu_split(&k1, 1, (int) t[0].ne[0], (int) t[0].ne[1], 1, (int) t[2].ne[1], 0,
-                                       (int) (t[3].ne[1] * t[3].ne[2] * t[3].ne[3]), 1, d.type == TSK_TYPE_BF16).bytes;
+                     swiglu_part_bytes(&k1, 1, (int) t[0].ne[1], 1, (int) t[2].ne[1], 0,
+                                       (int) (t[3].ne[1] * t[3].ne[2] * t[3].ne[3]), 1, d.type == TSK_TYPE_BF16, &sp);
             return TSK_OK;
         }
         case TSK_OP_RMS_NORM_Q8_0:

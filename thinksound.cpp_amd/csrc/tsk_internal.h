@@ -208,6 +208,7 @@ struct GemmProblem {
     int splits;                    // K slices (EPI_PARTIAL), else 1
     const uint16_t *w3;            // EPI_SWIGLU_*: the second weight (same layout as w)
     const float *wf;               // launch_gemm_f32: f32 weights [M][K] row-major (ld_w)
+    const float *wf3;              // launch_gemm_f32x6: a second weight, its outputs M .. 2 M - 1 (nullable)
     int accumulate;                // launch_gemm_f32: y += acc + bias (f32 y)
     // implicit im2col (conv_ic > 0): row n of X is output position ow = n % conv_ow
     // of batch item b = n / conv_ow, and column k = kw * conv_ic + ic reads
@@ -433,6 +434,20 @@ struct F32Snake {
 // (plain rows or implicit im2col), y f32 or bf16 (+bias), optionally followed
 // by a SnakeBeta (f32 y only)
 hipError_t launch_gemm_f32(const GemmProblem &p, int y_bf16, hipStream_t s, const F32Snake *snake = nullptr);
+// the same as six bf16 products of operands in three parts (gemm_f32x6.hip):
+// M % 4, K (and conv_ic) % 32, 16-byte aligned rows, a tile's rows within 2 GiB;
+// y += with a SnakeBeta only. launch_gemm_f32 takes it where it fits. unit: y and
+// the SnakeBeta are those of a second, k1 convolution (w2, p.bias) of the first
+// one's bias and SnakeBeta (M <= 128, M % 32)
+struct F32Unit {
+    const float *w2;               // [M][M]
+    const float *bias, *ea, *eb;   // [M]
+};
+bool gemm_f32x6_fits(const GemmProblem &p);    // and tuning().f32_split
+// K slices that fill the chip with the tiles of an M x N x K product
+int gemm_f32x6_slices(int64_t M, int64_t N, int64_t K, int most);
+hipError_t launch_gemm_f32x6(const GemmProblem &p, int y_bf16, hipStream_t s, const F32Snake *snake = nullptr,
+                             const F32Unit *unit = nullptr);
 // F32 products on the fp16 matrix cores (gemm_split.hip): operands as split
 // rows (32 hi, 32 lo fp16 per group of 32 values, of the value times
 // 2^(15 - e); one 4-byte word per value, strides in words)

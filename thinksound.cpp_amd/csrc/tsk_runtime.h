@@ -41,11 +41,10 @@ bool workspace_can(hipStream_t s, size_t bytes);
 //   TSK_GRAPH_KSPLIT / TSK_GRAPH_KSWG  most K slices of the reference graph's bf16 k3 convolutions (4) and
 //                 the workgroup count (64 x 64 tiles x slices) they stop below (1536)
 //   TSK_ATTN_Q8   Q8_0 driver: the attention writes linear1's Q8_0 activations itself (1), or f32 + quantize (0)
-//   TSK_F32_DL / TSK_F32_DL_NS  F32 GEMM with direct global -> LDS loads (1, default; 0 = register staged)
+//   TSK_F32_DL / TSK_F32_DL_NS  fp32 MFMA GEMM with direct global -> LDS loads (1, default; 0 = register staged)
 //                 and its ring depth (2, default; 3)
-//   TSK_F32_SPLIT F32 weights of the C-ABI nodes and of the reference graph as three fp16 products of scaled halves
-//                 (1, default) or fp32 MFMA products (0); the graph reads it when a model is created, which then
-//                 holds split copies, and on every call
+//   TSK_F32_SPLIT F32 products as six bf16 products of operands in three parts (1, default) or fp32 MFMA
+//                 products (0), read on every call; a reference graph created with 1 holds fp16 split copies
 //   TSK_SPLIT_WG  most 128 x 128 tiles times K slices of the graph's bf16 convolutions into plain rows (512)
 struct Tuning {
     int q8_cfg = 0;
