@@ -38,8 +38,7 @@ def vae(env):
 @pytest.mark.parametrize("T,scale", [(1, 1.0), (3, 1.0), (5, 2.0 ** -12)])
 def test_vae_split(vae, T, scale):
     """one output tile and less, odd lengths, and a latent whose values are far
-    below 1 (its exponent follows it). Bound: the fp32 decode's 2e-4 (products
-    with an error of 2^-22 per term and fp32 sums, amplified 50-100 times)"""
+    below 1. Bound: the fp32 decode's 2e-4 (fp32 sums, amplified 50-100 times)"""
     v, ov = vae
     lat = (np.random.default_rng(T).standard_normal((32, T)) * scale).astype(np.float32)
     a, r = v.decode(lat), ov.decode(lat)
@@ -50,8 +49,7 @@ def test_vae_split(vae, T, scale):
 
 
 def test_vae_split_nan_stays_local(vae):
-    """a NaN latent frame reaches its receptive field (about 12 frames) only:
-    the exponents come from the finite values"""
+    """a NaN latent frame reaches its receptive field (about 12 frames) only"""
     v, _ = vae
     lat = np.random.default_rng(9).standard_normal((32, 48)).astype(np.float32)
     ref = v.decode(lat)
@@ -60,6 +58,60 @@ def test_vae_split_nan_stays_local(vae):
     assert np.isnan(a[:, :2048]).all()
     far = slice(20 * 2048, None)
     assert np.isfinite(a[:, far]).all() and rel_l2(a[:, far], ref[:, far]) <= 2e-4
+
+
+@pytest.fixture(scope="module")
+def copier(env):
+    """a decoder that repeats its latent: unit kernels (every phase of a transposed convolution reads its own frame),
+    zero residual units, SnakeBetas that add nothing (exp(alpha) = 0); 32 output channels"""
+    tsk, _ = env
+    v = tsk.Vae(tsk.vae_config(latent_dim=32, channels=32, c_mults=[1, 1, 1, 1, 1], out_channels=32, max_latent=8))
+    for name, ne in v.tensors():
+        w = np.zeros([int(n) for n in reversed(ne) if n > 1], np.float32)
+        if name.endswith(".alpha"):
+            w[:] = -1000
+        elif w.ndim == 3 and w.shape[2] != 7:                          # stride s: taps s / 2 .. 3 s / 2 - 1
+            s = w.shape[2] // 2
+            w[np.arange(32), np.arange(32), s // 2:3 * s // 2] = 1
+        elif name in ("decoder.layers.0.weight", "decoder.layers.7.weight"):
+            w[np.arange(32), np.arange(32), 3] = 1
+        v.set_tensor(name, w)
+    yield v
+    v.close()
+
+
+def test_vae_keeps_every_bit(copier):
+    """values that differ by 2^60 within a frame and from frame to frame come through all 36 convolutions as they are:
+    no channel and no loud passage costs another one bits"""
+    rng = np.random.default_rng(8)
+    lat = (rng.standard_normal((32, 8)) * 2.0 ** rng.integers(-30, 30, (32, 8))).astype(np.float32)
+    a = copier.decode(lat)
+    assert np.array_equal(a, np.repeat(lat, copier.hop, 1))
+
+
+def test_vae_snake_accuracy(copier):
+    """v + sin^2(e^alpha v) e^-beta against 64 bits, arguments up to 2^18: sin^2 to 1.2e-7 (what the fp32 sinf gives)
+    and the roundings of the product with e^-beta and of the sum"""
+    libm = ctypes.CDLL("libm.so.6")
+    libm.expf.restype, libm.expf.argtypes = ctypes.c_float, [ctypes.c_float]
+    rng = np.random.default_rng(9)
+    try:
+        worst = 0.0
+        for alpha, beta in [(0.0, 0.0), (0.0, -7.0), (5.0, -7.0), (11.0, -7.0)]:
+            ea, eb = np.float32(libm.expf(alpha)), np.float32(libm.expf(-beta))
+            copier.set_tensor("decoder.layers.6.alpha", np.full(32, alpha, np.float32))
+            copier.set_tensor("decoder.layers.6.beta", np.full(32, beta, np.float32))
+            for _ in range(8):
+                lat = rng.uniform(-4, 4, (32, 8)).astype(np.float32)
+                got = copier.decode(lat)[:, ::copier.hop].astype(np.float64)
+                arg = (lat * ea).astype(np.float64)
+                ref = lat + np.sin(arg) ** 2 * np.float64(eb)
+                err = (np.abs(got - ref) - 2.0 ** -24 * (np.abs(ref) + np.float64(eb))) / np.float64(eb)
+                worst = max(worst, float(err.max()))
+        print(f"sin^2: max error {worst:.2e}", flush=True)
+        assert worst <= 1.2e-7
+    finally:
+        copier.set_tensor("decoder.layers.6.alpha", np.full(32, -1000, np.float32))
 
 
 # ---------------------------------------------------------------- F32 nodes

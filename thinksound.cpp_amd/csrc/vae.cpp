@@ -3,8 +3,8 @@
 //
 // Activations are token-major rows [T][C] (channels fastest), so every
 // convolution is one F32 GEMM over implicit im2col rows:
-// y[t][oc] = sum_{kw, ic} W[oc][kw][ic] x[t + kw d - p][ic], its products on the
-// fp16 matrix cores from split operands (gemm_split.hip) where the channel
+// y[t][oc] = sum_{kw, ic} W[oc][kw][ic] x[t + kw d - p][ic], as six bf16
+// products of operands in three parts (gemm_f32x6.hip) where the channel
 // counts allow, else fp32 MFMAs (gemm_f32.hip).
 // The reference keeps [T, C] with time fastest and runs im2col + mul_mat; the
 // sums are the same products in another order.
@@ -25,7 +25,6 @@
 // with padding 1; taps 1, 2 without), skipping the zero taps.
 #include <hip/hip_runtime.h>
 
-#include <cmath>
 #include <cstring>
 #include <string>
 #include <unordered_map>
@@ -48,8 +47,6 @@ struct VW {
     int stride;             // ct: the stride s
     size_t offset;          // device float offset of the prepared layout
     size_t count;           // floats stored
-    size_t woffset;         // split products: int offset of the rows' exponents
-    float l1, amax;         // split products: max over the rows of sum |w|, max |w| (biases, exp(-beta): max)
 };
 
 }  // namespace
@@ -63,13 +60,6 @@ struct tsk_vae {
     float *lat = nullptr;                          // latent rows [T][latent_dim]
     size_t act_cap = 0;
     int hop = 1;
-    // split products (every channel count a multiple of 32): the kernels in
-    // the blob and the snakes in act[1], act[2], lat are split rows
-    // (gemm_split.hip); the residual stream act[0] stays f32
-    bool split = false;
-    int *wexp = nullptr;                           // exponents of the kernels' rows
-    float *slots = nullptr;                        // max |snake| and max |residual| per convolution
-    int *exps = nullptr;                           // exponent of each split tensor
 };
 
 namespace {
@@ -84,8 +74,7 @@ void addv(tsk_vae *v, const std::string &name, int64_t a, int64_t b, int64_t c, 
     x.conv = conv;
     x.ct = ct;
     x.stride = stride;
-    x.offset = x.woffset = 0;
-    x.l1 = x.amax = 0.0f;
+    x.offset = 0;
     // prepared layouts: conv kw-major [OC][K * IC]; transposed conv the merged
     // 3-tap kernel [s * OC][3 * IC] and its bias replicated [s * OC]
     x.count = ct ? (size_t) stride * c * 3 * b : (size_t) (a * b * c);
@@ -110,10 +99,9 @@ F32Snake snake_epi(const tsk_vae *v, const std::string &p, int C, float *y2) {
     return F32Snake{wp(v, p + ".alpha"), wp(v, p + ".beta"), y2, C};
 }
 
-// y rows [T_out][OC] = conv(x rows [T_in][IC]) + bias, stride 1 (F32 GEMM),
-// optionally followed by a SnakeBeta
-int conv(const tsk_vae *v, const std::string &p, bool bias, const float *x, int IC, int T_in, int pad, int dil,
-         float *y, bool accumulate, hipStream_t s, const F32Snake *sk = nullptr) {
+// the problem of y rows [T_out][OC] = conv(x rows [T_in][IC]) + bias, stride 1
+GemmProblem conv_problem(const tsk_vae *v, const std::string &p, bool bias, const float *x, int IC, int T_in, int pad,
+                         int dil, float *y, bool accumulate) {
     const VW &w = wi(v, p + ".weight");
     const int KW = (int) w.ne[0], OC = (int) w.ne[2];
     GemmProblem q;
@@ -128,7 +116,13 @@ int conv(const tsk_vae *v, const std::string &p, bool bias, const float *x, int 
         q.conv_ic = IC; q.conv_iw = T_in; q.conv_ow = T_out; q.conv_s = 1; q.conv_p = pad; q.conv_d = dil;
     }
     q.accumulate = accumulate ? 1 : 0;
-    return hipcheck(launch_gemm_f32(q, 0, s, sk), "vae conv");
+    return q;
+}
+
+// the convolution, optionally followed by a SnakeBeta
+int conv(const tsk_vae *v, const std::string &p, bool bias, const float *x, int IC, int T_in, int pad, int dil,
+         float *y, bool accumulate, hipStream_t s, const F32Snake *sk = nullptr) {
+    return hipcheck(launch_gemm_f32(conv_problem(v, p, bias, x, IC, T_in, pad, dil, y, accumulate), 0, s, sk), "vae conv");
 }
 
 // the first phase that reads input frames q and q + 1 (c(r) = 0) when the
@@ -186,112 +180,18 @@ int conv_t(const tsk_vae *v, const std::string &p, const float *x, int IC, int T
     return TSK_OK;
 }
 
-// ---- split products. Convolution number i of the decode reads the split
-// tensor i (exponent exps[i], max |value| slots[2 i]) and writes tensor i + 1
-// (slots[2 i + 2]) as the SnakeBeta of its output; the residual stream it
-// leaves has max |value| slots[2 i + 3].
-constexpr int VAE_CONVS = 1 + 5 * 7;
-constexpr int VAE_SLOTS = 2 * (VAE_CONVS + 1);
-
-struct SplitStep {
-    int i;                 // convolution number
-    const float *x;        // split rows in
-    float *y;              // f32 output rows (nullable: not written)
-    int old;               // >= 0: y += conv, the old y left by convolution `old`
-    std::string snake;     // SnakeBeta parameters' prefix
-    int C;                 // its period (channels)
-    float *out;            // the snake: split rows, or f32 rows (last)
-    bool last;
-};
-
-SplitGemm split_gemm(const tsk_vae *v, const std::string &p, const SplitStep &t, int IC) {
-    const VW &w = wi(v, p + ".weight"), &b = wi(v, p + ".bias"), &sb = wi(v, t.snake + ".beta");
-    SplitGemm q;
-    memset(&q, 0, sizeof(q));
-    q.x = (const uint32_t *) t.x; q.ld_x = IC;
-    q.w = (const uint32_t *) (v->blob + w.offset);
-    q.we = v->wexp + w.woffset;
-    q.xe = v->exps + t.i;
-    q.bias = v->blob + b.offset;
-    q.y = t.y; q.accumulate = t.old >= 0;
-    q.splits = 1;
-    q.conv_s = q.conv_d = 1;
-    q.ea = wp(v, t.snake + ".alpha"); q.eb = v->blob + sb.offset; q.period = t.C;
-    if (t.last) q.y2 = t.out;
-    else q.yp = (uint32_t *) t.out;
-    q.l1 = 1.01f * w.l1; q.badd = 1.01f * (b.amax + sb.amax);
-    q.amax_x = v->slots + 2 * t.i;
-    q.amax_old = t.old >= 0 ? v->slots + 2 * t.old + 3 : nullptr;
-    q.e_out = v->exps + t.i + 1;
-    q.amax_s = v->slots + 2 * t.i + 2;
-    q.amax_y = t.y ? v->slots + 2 * t.i + 3 : nullptr;
-    return q;
-}
-
-int conv_split(const tsk_vae *v, const std::string &p, int IC, int T_in, int pad, int dil, const SplitStep &t,
-               hipStream_t s) {
-    const VW &w = wi(v, p + ".weight");
-    const int KW = (int) w.ne[0], OC = (int) w.ne[2];
-    SplitGemm q = split_gemm(v, p, t, IC);
-    q.ld_w = (int64_t) KW * IC;
-    q.ld_y = OC;
-    const int T_out = T_in + 2 * pad - dil * (KW - 1);
-    q.M = OC; q.N = T_out; q.K = KW * IC;
-    if (KW > 1 || pad) {
-        q.conv_ic = IC; q.conv_iw = T_in; q.conv_ow = T_out; q.conv_p = pad; q.conv_d = dil;
-    }
-    return hipcheck(launch_gemm_split(q, s), "vae split conv");
-}
-
-// a residual unit of at most 128 channels (convolutions i and i + 1 of t) in one launch
-int unit_split(const tsk_vae *v, const std::string &rp, int C, int T, int dil, const SplitStep &t, hipStream_t s) {
-    const VW &w1 = wi(v, rp + ".layers.1.weight"), &w2 = wi(v, rp + ".layers.3.weight");
-    const VW &b1 = wi(v, rp + ".layers.1.bias"), &eb1 = wi(v, rp + ".layers.2.beta");
-    const int KW = (int) w1.ne[0];
-    SplitStep last = t;
-    last.i = t.i + 1;
-    SplitGemm q = split_gemm(v, rp + ".layers.3", last, C);
-    q.w2 = q.w; q.we2 = q.we;
-    q.w = (const uint32_t *) (v->blob + w1.offset);
-    q.we = v->wexp + w1.woffset;
-    q.xe = v->exps + t.i;
-    q.amax_x = v->slots + 2 * t.i;
-    q.mid_bias = v->blob + b1.offset;
-    q.mid_ea = wp(v, rp + ".layers.2.alpha"); q.mid_eb = v->blob + eb1.offset;
-    q.mid_l1 = 1.01f * w1.l1; q.mid_badd = 1.01f * (b1.amax + eb1.amax);
-    q.l1 = 1.01f * w2.l1;
-    q.ld_w = (int64_t) KW * C;
-    q.ld_y = C;
-    q.M = C; q.N = T; q.K = KW * C;
-    q.conv_ic = C; q.conv_iw = T; q.conv_ow = T; q.conv_p = dil * (KW / 2); q.conv_d = dil;
-    return hipcheck(launch_gemm_split(q, s), "vae residual unit");
-}
-
-// the transposed convolution of conv_t: the merged kernel's two-tap phase groups
-int conv_t_split(const tsk_vae *v, const std::string &p, int IC, int T_in, const SplitStep &t, hipStream_t s) {
-    const VW &w = wi(v, p + ".weight");
-    const int OC = (int) w.ne[2], st = w.stride;
-    const int ra = ct_split_phase(w.ne[0], st);
-    const SplitGemm q0 = split_gemm(v, p, t, IC);
-    for (int g = 0; g < 2; ++g) {
-        const int r0 = ra < 0 ? 0 : g ? ra : 0, r1 = ra < 0 || g ? st : ra;
-        if (r1 <= r0 || (ra < 0 && g)) continue;
-        const int64_t row0 = (int64_t) r0 * OC;
-        SplitGemm q = q0;
-        q.w += row0 * 3 * IC + (ra >= 0 && g ? IC : 0);     // taps 1, 2 for the second group
-        q.ld_w = (int64_t) 3 * IC;
-        q.we += row0;
-        q.bias += row0;
-        q.y = (float *) q.y + row0;
-        q.ld_y = (int64_t) st * OC;
-        if (q.yp) q.yp += row0;                              // row0 is a multiple of the period OC
-        if (q.y2) q.y2 += row0;
-        q.M = (r1 - r0) * OC; q.N = T_in; q.K = (ra < 0 ? 3 : 2) * IC;
-        q.conv_ic = IC; q.conv_iw = T_in; q.conv_ow = T_in; q.conv_p = ra < 0 || !g ? 1 : 0;
-        const int rc = hipcheck(launch_gemm_split(q, s), "vae split transposed conv");
-        if (rc) return rc;
-    }
-    return TSK_OK;
+// x += conv_k1(snake(conv_k7(sx))) with t = the snake of x after it, one launch:
+// a residual unit of at most 128 channels, or false where it runs as two
+bool unit_fits(const GemmProblem &q) { return q.M <= 128 && q.M % 32 == 0 && gemm_f32x6_fits(q); }
+int unit(const tsk_vae *v, const std::string &rp, GemmProblem q, float *x, const F32Snake &sk, hipStream_t s) {
+    F32Unit u;
+    u.w2 = wp(v, rp + ".layers.3.weight");
+    u.bias = q.bias;
+    u.ea = wp(v, rp + ".layers.2.alpha"); u.eb = wp(v, rp + ".layers.2.beta");
+    q.bias = wp(v, rp + ".layers.3.bias");
+    q.y = x;
+    q.accumulate = 1;
+    return hipcheck(launch_gemm_f32x6(q, 0, s, &sk, &u), "vae residual unit");
 }
 
 int validate(const tsk_vae_config *c) {
@@ -326,9 +226,6 @@ extern "C" void tsk_vae_destroy(tsk_vae *v) {
     for (float *a : v->act)
         if (a) (void) hipFree(a);
     if (v->lat) (void) hipFree(v->lat);
-    if (v->wexp) (void) hipFree(v->wexp);
-    if (v->slots) (void) hipFree(v->slots);
-    if (v->exps) (void) hipFree(v->exps);
     delete v;
 }
 
@@ -384,21 +281,6 @@ extern "C" int tsk_vae_create(const tsk_vae_config *cfg, tsk_vae **out) {
         off += (x.count + 63) & ~(size_t) 63;
     }
     v->act_cap = (size_t) c.max_latent * (size_t) max_ch_t;
-    // split products need whole 32-channel groups in every tensor a convolution
-    // reads or writes but the final k7's, and 31-bit byte offsets into a kernel
-    v->split = c.latent_dim % 32 == 0;
-    for (int n = 0; n < 5; ++n) {
-        int ci, co, st;
-        block_dims(c, n, &ci, &co, &st);
-        v->split = v->split && ci % 32 == 0 && co % 32 == 0;
-    }
-    size_t nexp = 0;
-    for (auto &x : v->w)
-        if ((x.conv || x.ct) && x.name != "decoder.layers.7.weight") {
-            v->split = v->split && sizeof(float) * x.count < ((size_t) 1 << 31);
-            x.woffset = nexp;
-            nexp += (size_t) (x.ct ? x.stride : 1) * x.ne[2];
-        }
     auto alloc = [&](void **p, size_t bytes) -> int {
         hipError_t e = hipMalloc(p, bytes);
         if (e != hipSuccess) return fail(TSK_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
@@ -408,15 +290,11 @@ extern "C" int tsk_vae_create(const tsk_vae_config *cfg, tsk_vae **out) {
         (rc = alloc((void **) &v->act[0], sizeof(float) * v->act_cap)) ||
         (rc = alloc((void **) &v->act[1], sizeof(float) * v->act_cap)) ||
         (rc = alloc((void **) &v->act[2], sizeof(float) * v->act_cap)) ||
-        (rc = alloc((void **) &v->lat, sizeof(float) * (size_t) c.max_latent * c.latent_dim)) ||
-        (v->split && ((rc = alloc((void **) &v->wexp, sizeof(int) * nexp)) ||
-                      (rc = alloc((void **) &v->slots, sizeof(float) * VAE_SLOTS)) ||
-                      (rc = alloc((void **) &v->exps, sizeof(int) * (VAE_CONVS + 1)))))) {
+        (rc = alloc((void **) &v->lat, sizeof(float) * (size_t) c.max_latent * c.latent_dim))) {
         tsk_vae_destroy(v);
         return rc;
     }
     hipError_t e = hipMemset(v->blob, 0, sizeof(float) * off);
-    if (e == hipSuccess && v->split) e = hipMemset(v->wexp, 0, sizeof(int) * nexp);
     if (e != hipSuccess) { tsk_vae_destroy(v); return hip_fail(e, "vae init"); }
     *out = v;
     return TSK_OK;
@@ -439,14 +317,13 @@ extern "C" int tsk_vae_set_tensor(tsk_vae *v, const char *name, const float *src
     if (!v || !name || !src) return fail(TSK_ERR_INVALID_ARG, "NULL argument");
     auto it = v->idx.find(name);
     if (it == v->idx.end()) return fail(TSK_ERR_INVALID_ARG, "unknown tensor '%s'", name);
-    VW &x = v->w[it->second];
+    const VW &x = v->w[it->second];
     const int64_t N = x.ne[0] * x.ne[1] * x.ne[2];
     if (n != N) return fail(TSK_ERR_SHAPE, "'%s' has %lld elements, got %lld", name, (long long) N, (long long) n);
     std::vector<float> t(x.count, 0.0f);
     const std::string nm = name;
     const bool is_alpha = nm.size() > 6 && nm.compare(nm.size() - 6, 6, ".alpha") == 0;
     const bool is_beta = nm.size() > 5 && nm.compare(nm.size() - 5, 5, ".beta") == 0;
-    x.amax = x.l1 = 0.0f;
     if (x.ct) {
         // merged 3-tap kernel: row r * OC + oc, tap j (input frame q - 1 + j),
         // channel ic = W'[oc][ic][k] for the phase's two taps k
@@ -473,26 +350,6 @@ extern "C" int tsk_vae_set_tensor(tsk_vae *v, const char *name, const float *src
         for (int64_t i = 0; i < n; ++i) t[i] = is_alpha ? expf(src[i]) : is_beta ? expf(-src[i]) : src[i];
     }
     hipError_t e = hipMemcpy(v->blob + x.offset, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice);
-    if (v->split) {
-        for (float a : t) x.amax = std::max(x.amax, std::isfinite(a) ? std::fabs(a) : 0.0f);
-        if ((x.conv || x.ct) && nm != "decoder.layers.7.weight") {
-            // the row bounds, and the rows split in place
-            const size_t rows = (size_t) (x.ct ? x.stride : 1) * x.ne[2], K = t.size() / rows;
-            for (size_t r = 0; r < rows; ++r) {
-                float l1 = 0.0f;
-                for (size_t k = 0; k < K; ++k) l1 += std::isfinite(t[r * K + k]) ? std::fabs(t[r * K + k]) : 0.0f;
-                x.l1 = std::max(x.l1, l1);
-            }
-            SplitRowsGroup sg;
-            memset(&sg, 0, sizeof(sg));
-            sg.n = 1;
-            sg.j[0].x = v->blob + x.offset; sg.j[0].ld_x = (int64_t) K;
-            sg.j[0].rows = (int64_t) rows; sg.j[0].cols = (int) K;
-            sg.j[0].y = (uint32_t *) (v->blob + x.offset); sg.j[0].e = v->wexp + x.woffset;
-            if (e == hipSuccess) e = launch_split_rows(sg, nullptr);
-            if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-        }
-    }
     return hipcheck(e, "vae set_tensor copy");
 }
 
@@ -523,52 +380,6 @@ int decode_impl(tsk_vae *v, int T, const float *latent_d, float *audio_d, hipStr
     float *x = v->act[0], *sx = v->act[1], *t = v->act[2];
     int in0, out0, s0;
     block_dims(c, 0, &in0, &out0, &s0);
-    if (v->split) {
-        // the latent's exponent and rows, then the chain on split rows (the
-        // residual stream x f32, the final snake f32 in sx)
-        if ((rc = hipcheck(launch_split_begin(latent_d, (int64_t) T * c.latent_dim, v->slots, VAE_SLOTS, v->exps, st),
-                           "vae latent")) ||
-            (rc = hipcheck(launch_split_transpose(latent_d, c.latent_dim, T, v->exps, (uint32_t *) v->lat, st),
-                           "vae latent")) ||
-            (rc = conv_split(v, "decoder.layers.0", c.latent_dim, T, 3, 1,
-                             SplitStep{0, v->lat, nullptr, -1, "decoder.layers.1.layers.0", in0, sx, false}, st)))
-            return rc;
-        int64_t fr = T;
-        int i = 1, res = 0, Cs = in0;                        // next convolution; the one that wrote x last
-        const int dl[3] = {1, 3, 9};
-        for (int n = 0; n < 5; ++n) {
-            int ci, co, s;
-            block_dims(c, n, &ci, &co, &s);
-            const std::string bp = "decoder.layers." + std::to_string(n + 1);
-            if ((rc = conv_t_split(v, bp + ".layers.1", ci, (int) fr,
-                                   SplitStep{i, sx, x, -1, bp + ".layers.2.layers.0", co, t, false}, st)))
-                return rc;
-            std::swap(sx, t);
-            res = i++;
-            fr *= s;
-            Cs = co;
-            for (int r = 0; r < 3; ++r) {
-                const std::string rp = bp + ".layers." + std::to_string(r + 2);
-                const bool last = n == 4 && r == 2;
-                const std::string np = r < 2 ? bp + ".layers." + std::to_string(r + 3) + ".layers.0"
-                                     : n < 4 ? "decoder.layers." + std::to_string(n + 2) + ".layers.0"
-                                             : std::string("decoder.layers.6");
-                if (Cs <= 128) {
-                    if ((rc = unit_split(v, rp, Cs, (int) fr, dl[r], SplitStep{i, sx, x, res, np, Cs, t, last}, st)))
-                        return rc;
-                    std::swap(sx, t);
-                } else if ((rc = conv_split(v, rp + ".layers.1", Cs, (int) fr, 3 * dl[r], dl[r],
-                                     SplitStep{i, sx, nullptr, -1, rp + ".layers.2", Cs, t, false}, st)) ||
-                           (rc = conv_split(v, rp + ".layers.3", Cs, (int) fr, 0, 1,
-                                            SplitStep{i + 1, t, x, res, np, Cs, sx, last}, st))) {
-                    return rc;
-                }
-                res = i + 1;
-                i += 2;
-            }
-        }
-        return decode_out(v, sx, t, Cs, fr, audio_d, st);
-    }
     // latent ne = [T, latent_dim] (time fastest) -> rows [T][latent_dim]
     if ((rc = hipcheck(launch_transpose_ct(latent_d, 1, c.latent_dim, T, v->lat, st), "vae latent"))) return rc;
     // conv k7 -> snake of block 1 (the conv's own output is not used again)
@@ -590,13 +401,19 @@ int decode_impl(tsk_vae *v, int T, const float *latent_d, float *audio_d, hipStr
         for (int r = 0; r < 3; ++r) {
             // x += conv_k1(snake(conv_k7_dil(snake(x))))  (the residual unit, :99-105)
             const std::string rp = bp + ".layers." + std::to_string(r + 2);
-            sk = snake_epi(v, rp + ".layers.2", C, nullptr);
-            if ((rc = conv(v, rp + ".layers.1", true, sx, C, (int) frames, 3 * dil[r], dil[r], t, false, st, &sk)))
-                return rc;
             // the next snake of x: the next unit's, the next block's, or the final one
             const std::string np = r < 2 ? bp + ".layers." + std::to_string(r + 3) + ".layers.0"
                                  : n < 4 ? "decoder.layers." + std::to_string(n + 2) + ".layers.0"
                                          : std::string("decoder.layers.6");
+            const GemmProblem k7 =
+                conv_problem(v, rp + ".layers.1", true, sx, C, (int) frames, 3 * dil[r], dil[r], t, false);
+            if (unit_fits(k7)) {
+                if ((rc = unit(v, rp, k7, x, snake_epi(v, np, C, t), st))) return rc;
+                std::swap(sx, t);
+                continue;
+            }
+            sk = snake_epi(v, rp + ".layers.2", C, nullptr);
+            if ((rc = hipcheck(launch_gemm_f32(k7, 0, st, &sk), "vae conv"))) return rc;
             sk = snake_epi(v, np, C, sx);
             if ((rc = conv(v, rp + ".layers.3", true, t, C, (int) frames, 0, 1, x, true, st, &sk))) return rc;
         }
