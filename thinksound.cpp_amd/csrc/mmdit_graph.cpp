@@ -62,9 +62,6 @@ struct MW {
     bool qkv_perm;          // rows (or entries) of a qkv projection: (h d j) -> [q | k | v]
     size_t offset;          // F32 / BF16 values, or the Q8_0 int8 plane [M][K]
     size_t offset_d;        // Q8_0: the fp16 block-scale plane [M][K / 32]
-    size_t offset_s;        // split F32 matrix: its split rows (gemm_split.hip) and their exponents
-    size_t offset_e;
-    bool split;             // F32 matrix also held as split rows (products on the fp16 matrix cores)
     float amax;             // max |value| of a vector as last set
 };
 
@@ -75,8 +72,6 @@ struct Lin {
     const float *wf;        // F32
     const int8_t *qw;       // Q8_0 planes
     const uint16_t *dw;
-    const uint32_t *ws;     // F32 held split: split rows and their exponents
-    const int *we;
     const float *b;
     int K, M;
 };
@@ -85,8 +80,6 @@ struct Conv {
     int type;
     const uint16_t *w;
     const float *wf;
-    const uint32_t *ws;     // F32 held split: split rows and their exponents
-    const int *we;
     const float *b;
     int KW, IC, OC;
 };
@@ -142,10 +135,6 @@ struct tsk_mmdit {
     // SwiGLU hidden state and its halves, and the conversion scratch of the
     // BF16 / Q8_0 products
     float *xn32 = nullptr, *o32 = nullptr, *qkv32 = nullptr, *hid32 = nullptr, *h1 = nullptr, *h3 = nullptr;
-    uint32_t *xsplit = nullptr;           // split products: the activations' split rows and exponents
-    int *xexp = nullptr;
-    size_t xsplit_cap = 0;                // values of xsplit, rows of xexp
-    int xexp_cap = 0;
     uint16_t *cvt16 = nullptr;
     int8_t *qx = nullptr;
     float *dx = nullptr;
@@ -182,8 +171,7 @@ void addw(tsk_mmdit *m, const std::string &name, int64_t a, int64_t b, int64_t c
     x.kind = kind;
     x.type = TSK_TYPE_F32;
     x.qkv_perm = perm;
-    x.offset = x.offset_d = x.offset_s = x.offset_e = 0;
-    x.split = false;
+    x.offset = x.offset_d = 0;
     x.amax = 0.0f;
     m->idx[name] = (int) m->w.size();
     m->w.push_back(x);
@@ -252,7 +240,6 @@ Lin lin_of(const tsk_mmdit *m, const std::string &p, bool bias) {
     if (x.type == TSK_TYPE_F32) L.wf = (const float *) base;
     else if (x.type == TSK_TYPE_BF16) L.w = (const uint16_t *) base;
     else { L.qw = (const int8_t *) base; L.dw = (const uint16_t *) (m->blob + x.offset_d); }
-    if (x.split) { L.ws = (const uint32_t *) (m->blob + x.offset_s); L.we = (const int *) (m->blob + x.offset_e); }
     L.b = bias ? wp<float>(m, p + ".bias") : nullptr;
     return L;
 }
@@ -264,7 +251,6 @@ Conv conv_of(const tsk_mmdit *m, const std::string &p, bool bias) {
     C.type = x.type;
     if (x.type == TSK_TYPE_F32) C.wf = wp<float>(m, p + ".weight");
     else C.w = wp<uint16_t>(m, p + ".weight");
-    if (x.split) { C.ws = (const uint32_t *) (m->blob + x.offset_s); C.we = (const int *) (m->blob + x.offset_e); }
     C.b = bias ? wp<float>(m, p + ".bias") : nullptr;
     C.KW = (int) x.ne[0];
     C.IC = (int) x.ne[1];
@@ -468,63 +454,11 @@ int rows_bf16(tsk_mmdit *m, const Rows &src, int N, int K, hipStream_t s) {
                     "mmdit bf16 rows");
 }
 
-// F32 products on the fp16 matrix cores (TSK_F32_SPLIT, for a model created
-// with it): split rows of the weight, held since it was set, and of the
-// activations, written to m->xsplit before each product
-bool split_on(const uint32_t *ws) { return ws && tuning().f32_split; }
-struct SplitW {
-    const uint32_t *ws;
-    const int *we;
-    const float *wf, *wf2;   // the f32 rows; from wf_rows on wf2's (w1 | w3 side by side)
-    int wf_rows, M, K;
-};
-SplitW split_w(const Lin &L) { return SplitW{L.ws, L.we, L.wf, nullptr, L.M, L.M, L.K}; }
-SplitW split_w(const Conv &C) { return SplitW{C.ws, C.we, C.wf, nullptr, C.OC, C.OC, C.KW * C.IC}; }
-// w1 | w3 as one weight of twice the rows (their split rows and exponents are placed back to back)
-SplitW split_pair(SplitW a, const SplitW &b) {
-    a.wf2 = b.wf;
-    a.M *= 2;
-    return a;
-}
-bool adjacent(const SplitW &a, const SplitW &b) {
-    return b.ws == a.ws + (size_t) a.M * a.K && b.we == a.we + a.M && a.M == b.M && a.K == b.K;
-}
-// y [N][ld_y] = rows . w (+ bias), the rows [N][cols] or the convolution of KW
-// = K / cols taps over items of IW = src.grp of them (padding pad), or with
-// splits > 1 (no bias) K-split slices `stride` apart
-int split_product(tsk_mmdit *m, const SplitW &w, const Rows &src, int rows, int cols, int pad, const float *bias, float *y,
-                  int64_t ld_y, int splits, int64_t stride, hipStream_t s) {
-    if ((size_t) rows * cols > m->xsplit_cap || rows > m->xexp_cap)
-        return fail(TSK_ERR_SHAPE, "split rows of %d x %d exceed the scratch", rows, cols);
-    const int KW = w.K / cols, IW = src.grp, OW = IW + 2 * pad - (KW - 1);
-    SplitRowsGroup g;
-    memset(&g, 0, sizeof(g));
-    g.n = 1;
-    g.j[0].x = src.x; g.j[0].ld_x = src.ld; g.j[0].rows_b = src.grp; g.j[0].ld_b = src.grp ? src.gstride : 0;
-    g.j[0].rows = rows; g.j[0].cols = cols; g.j[0].halo = KW - 1;
-    g.j[0].y = m->xsplit; g.j[0].e = m->xexp;
-    int rc = hipcheck(launch_split_rows(g, s), "mmdit split rows");
-    if (rc) return rc;
-    SplitGemm q;
-    memset(&q, 0, sizeof(q));
-    q.x = m->xsplit; q.ld_x = cols;
-    q.xe = m->xexp; q.xe_per_row = 1;
-    q.w = w.ws; q.ld_w = w.K; q.we = w.we;
-    q.bias = bias;
-    q.y = y; q.ld_y = ld_y;
-    q.M = w.M; q.K = w.K;
-    q.N = src.grp ? rows / IW * OW : rows;
-    q.splits = splits; q.part_stride = stride;
-    if (src.grp) { q.conv_ic = cols; q.conv_iw = IW; q.conv_ow = OW; q.conv_s = q.conv_d = 1; q.conv_p = pad; }
-    q.xf = src.x; q.ld_xf = src.ld; q.xf_batch = src.gstride;
-    q.wf = w.wf; q.wf2 = w.wf2; q.wf_rows = w.wf_rows; q.ld_wf = w.K;
-    return hipcheck(launch_gemm_split(q, s), "mmdit split product");
-}
 // K slices of a split product of S rows per batch item: counted with the
 // batch capacity, so that a batch row is summed in the same order whatever the
 // call's batch (the tile shape changes no sum)
 int split_slices_f32(const tsk_mmdit *m, int M, int K, int S, int most) {
-    return split_gemm_slices(M, (int64_t) S * m->cfg.max_batch, K, most);
+    return gemm_f32x6_slices(M, (int64_t) S * m->cfg.max_batch, K, most);
 }
 // K slices of a bf16 convolution into plain rows: the most, up to `most`,
 // that keep the 128 x 128 tiles times slices within TSK_SPLIT_WG (512); every
@@ -565,7 +499,7 @@ int conv_plain(tsk_mmdit *m, const Conv &C, const uint16_t *x, int64_t ld_x, int
 // products by split_slices_f32; BF16 kernels unsplit
 int res_splits(const tsk_mmdit *m, const Conv &C, int S) {
     if (C.type != TSK_TYPE_F32) return 1;
-    return split_on(C.ws) ? split_slices_f32(m, C.OC, C.KW * C.IC, S, PART_SLICES) : f32_splits(m, C.OC, C.KW * C.IC, S);
+    return tuning().f32_split ? split_slices_f32(m, C.OC, C.KW * C.IC, S, PART_SLICES) : f32_splits(m, C.OC, C.KW * C.IC, S);
 }
 
 // y[n][m] = x[n] . W[m] (+ b), any storage type
@@ -574,8 +508,6 @@ int res_splits(const tsk_mmdit *m, const Conv &C, int S) {
 int g_lin(tsk_mmdit *m, const Lin &L, const Rows &src, int N, float *y, int64_t ld_y, bool bias, hipStream_t s,
           const QkvScatter *qs = nullptr) {
     const float *b = bias ? L.b : nullptr;
-    if (L.type == TSK_TYPE_F32 && split_on(L.ws))
-        return split_product(m, split_w(L), src, N, L.K, 0, b, y, ld_y, 1, 0, s);
     if (L.type == TSK_TYPE_F32) {
         GemmProblem q;
         memset(&q, 0, sizeof(q));
@@ -623,24 +555,6 @@ int g_lin(tsk_mmdit *m, const Lin &L, const Rows &src, int N, float *y, int64_t 
 int g_conv(tsk_mmdit *m, const Conv &C, const float *x, int64_t ld_x, int64_t xb, int IW, int B, int pad, float *y,
            int64_t ld_y, bool bias, hipStream_t s, int splits = 1) {
     if (splits > 1 && bias) return fail(TSK_ERR_INVALID_ARG, "K-split slices carry no bias");
-    if (C.type == TSK_TYPE_F32 && split_on(C.ws)) {
-        // a plain output over few tiles (the input projections' and the final
-        // layer's convolutions, up to K = 8448): K-split slices into m->h1
-        // (free outside the SwiGLU halves), summed with the bias
-        const Rows src{x, ld_x, IW, xb};
-        const int OW = IW + 2 * pad - (C.KW - 1), N = B * OW;
-        const size_t cap = (size_t) 2 * F32_KSPLIT_MAX * m->Rmax * m->cfg.mlp_hidden;   // floats of m->h1
-        const int most = (int) std::min<size_t>(SPLIT_SUM_MAX, cap / ((size_t) m->cfg.max_batch * OW * C.OC));
-        const int sp = splits == 1 && C.OC % 4 == 0 && ld_y % 4 == 0 && ((uintptr_t) y & 15) == 0
-                           ? split_slices_f32(m, C.OC, C.KW * C.IC, OW, most) : 1;
-        if (sp > 1) {
-            int rc = split_product(m, split_w(C), src, B * IW, C.IC, pad, nullptr, m->h1, C.OC, sp, (int64_t) N * C.OC, s);
-            if (rc) return rc;
-            return hipcheck(launch_sum_slices(m->h1, sp, (int64_t) N * C.OC, bias ? C.b : nullptr, N, C.OC, y, ld_y, s),
-                            "mmdit split slices");
-        }
-        return split_product(m, split_w(C), src, B * IW, C.IC, pad, bias ? C.b : nullptr, y, ld_y, splits, N * ld_y, s);
-    }
     if (C.type == TSK_TYPE_F32) {
         GemmProblem q;
         memset(&q, 0, sizeof(q));
@@ -648,10 +562,22 @@ int g_conv(tsk_mmdit *m, const Conv &C, const float *x, int64_t ld_x, int64_t xb
         q.wf = C.wf; q.ld_w = (int64_t) C.KW * C.IC;
         q.bias = bias ? C.b : nullptr;
         q.y = y; q.ld_y = ld_y;
-        const int OW = IW + 2 * pad - (C.KW - 1);
-        q.M = C.OC; q.N = B * OW; q.K = C.KW * C.IC; q.splits = splits;
+        const int OW = IW + 2 * pad - (C.KW - 1), N = B * OW;
+        q.M = C.OC; q.N = N; q.K = C.KW * C.IC; q.splits = splits;
         q.conv_ic = C.IC; q.conv_iw = IW; q.conv_ow = OW; q.conv_s = 1; q.conv_p = pad; q.conv_d = 1;
-        return hipcheck(launch_gemm_f32(q, 0, s), "mmdit f32 conv");
+        // a plain output over few tiles (the input projections' and the final
+        // layer's convolutions, up to K = 8448): K-split slices into m->h1
+        // (free outside the SwiGLU halves), summed with the bias
+        const size_t cap = (size_t) 2 * F32_KSPLIT_MAX * m->Rmax * m->cfg.mlp_hidden;   // floats of m->h1
+        const int most = (int) std::min<size_t>(SPLIT_SUM_MAX, cap / ((size_t) m->cfg.max_batch * OW * C.OC));
+        const int sp = tuning().f32_split && splits == 1 && C.OC % 4 == 0 && ld_y % 4 == 0 && ((uintptr_t) y & 15) == 0
+                           ? split_slices_f32(m, C.OC, C.KW * C.IC, OW, most) : 1;
+        if (sp == 1) return hipcheck(launch_gemm_f32(q, 0, s), "mmdit f32 conv");
+        q.y = m->h1; q.ld_y = C.OC; q.bias = nullptr; q.splits = sp;
+        const int rc = hipcheck(launch_gemm_f32(q, 0, s), "mmdit f32 conv");
+        if (rc) return rc;
+        return hipcheck(launch_sum_slices(m->h1, sp, (int64_t) N * C.OC, bias ? C.b : nullptr, N, C.OC, y, ld_y, s),
+                        "mmdit conv slices");
     }
     const Rows src{x, ld_x, IW, xb};
     int rc = rows_bf16(m, src, B * IW, C.IC, s);
@@ -670,16 +596,25 @@ int g_swiglu(tsk_mmdit *m, bool is_conv, const Conv &c1, const Conv &c3, const C
     const int N = B * S;
     const int F = is_conv ? c1.OC : l1.M;
     const int t1 = is_conv ? c1.type : l1.type, t3 = is_conv ? c3.type : l3.type;
-    const SplitW s1 = is_conv ? split_w(c1) : split_w(l1), s3 = is_conv ? split_w(c3) : split_w(l3);
-    const bool split = t1 == TSK_TYPE_F32 && t3 == TSK_TYPE_F32 && split_on(s1.ws) && split_on(s3.ws) && adjacent(s1, s3);
     int rc;
-    if (split) {
+    GemmProblem q;
+    memset(&q, 0, sizeof(q));
+    if (t1 == TSK_TYPE_F32 && t3 == TSK_TYPE_F32) {
         // both halves as one product of 2 F outputs, its K slices summed by the SiLU * gate kernel
-        const int sp = split_slices_f32(m, 2 * F, s1.K, S, F32_KSPLIT_MAX);
-        const Rows src = is_conv ? Rows{x, ld_x, S, xb} : Rows{x, ld_x, 0, 0};
-        if ((rc = split_product(m, split_pair(s1, s3), src, N, is_conv ? c1.IC : l1.K, is_conv ? 1 : 0, nullptr, m->h1,
-                                2 * F, sp, (int64_t) N * 2 * F, s)) ||
-            (rc = hipcheck(launch_silu_mul_rows(m->h1, sp, (int64_t) N * 2 * F, N, F, m->hid32, s), "mmdit silu * gate")))
+        q.x = x; q.ld_x = ld_x;
+        q.wf = is_conv ? c1.wf : l1.wf; q.wf3 = is_conv ? c3.wf : l3.wf;
+        q.M = F; q.N = N; q.K = is_conv ? c1.KW * c1.IC : l1.K;
+        q.ld_w = q.K;
+        q.y = m->h1; q.ld_y = 2 * F;
+        if (is_conv) {
+            q.x_group_stride = xb;
+            q.conv_ic = c1.IC; q.conv_iw = S; q.conv_ow = S; q.conv_s = 1; q.conv_p = 1; q.conv_d = 1;
+        }
+        q.splits = split_slices_f32(m, 2 * F, q.K, S, F32_KSPLIT_MAX);
+    }
+    if (q.wf && gemm_f32x6_fits(q)) {
+        if ((rc = hipcheck(launch_gemm_f32x6(q, 0, s), "mmdit swiglu w1 | w3")) ||
+            (rc = hipcheck(launch_silu_mul_rows(m->h1, q.splits, (int64_t) N * 2 * F, N, F, m->hid32, s), "mmdit silu * gate")))
             return rc;
     } else if (t1 == TSK_TYPE_BF16 && t3 == TSK_TYPE_BF16) {
         // both halves in one cooperative GEMM with the SwiGLU epilogue, f32 out
@@ -1061,7 +996,7 @@ extern "C" void tsk_mmdit_destroy(tsk_mmdit *m) {
     void *bufs[] = {m->blob, m->lat, m->clip, m->txt, m->sync, m->ext, m->clip0, m->txt0, m->silu_ext, m->silu_gc,
                     m->vec, m->vec16, m->mods_lat, m->mods_gc, m->xn, m->hid, m->o, m->q, m->k, m->vt, m->part,
                     m->tmp32, m->rope_l, m->rope_c, m->in16, m->in32, m->act16, m->freq, m->temb, m->xn32, m->o32,
-                    m->qkv32, m->hid32, m->h1, m->xsplit, m->xexp, m->cvt16, m->qx, m->dx, m->xs, m->f0, m->flow2};
+                    m->qkv32, m->hid32, m->h1, m->cvt16, m->qx, m->dx, m->xs, m->f0, m->flow2};
     for (void *b : bufs)
         if (b) (void) hipFree(b);
     delete m;
@@ -1134,19 +1069,6 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
         any_q8 = any_q8 || t == TSK_TYPE_Q8_0;
         m->fast = m->fast && t == rule_type(TSK_TYPE_BF16, x);
     }
-    // F32 matrices also held as split rows (TSK_F32_SPLIT): every
-    // linear and convolution of the f32 path but the adaLN sets (one GEMM
-    // over a whole set) and the t_embed MLP (B rows, fp32 products)
-    bool any_split = false;
-    if (!m->fast && tuning().f32_split)
-        for (MW &x : m->w) {
-            x.split = x.type == TSK_TYPE_F32 && x.kind != K_VEC &&
-                      split_gemm_fits(x.kind == K_CONV ? x.ne[2] : x.ne[1], x.kind == K_CONV ? x.ne[0] * x.ne[1] : x.ne[0],
-                                      (int64_t) c.max_batch * (c.max_latent + c.max_clip + c.max_sync + X),
-                                      x.kind == K_CONV ? x.ne[1] : x.ne[0], 2) && x.name.find("adaLN_modulation") == std::string::npos &&
-                      x.name.find("t_embed") == std::string::npos;
-            any_split = any_split || x.split;
-        }
     // blob placement: the adaLN weights (each plane of them), then biases, of
     // the latent blocks and the final layer back to back (rows of one [Ml][H]
     // matrix, 256-byte multiples: no gaps), the same for the clip and text
@@ -1164,10 +1086,9 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
         const int i = m->idx.at(name);
         MW &x = m->w[i];
         const int64_t n = x.ne[0] * x.ne[1] * x.ne[2];
-        const size_t rows = (size_t) (x.kind == K_CONV ? x.ne[2] : x.ne[1]);
-        const size_t bytes = plane >= 2 ? (x.split ? 4 * (plane == 2 ? (size_t) n : rows) : 0) : type_bytes(x.type, n, plane);
+        const size_t bytes = type_bytes(x.type, n, plane);
         if (!bytes) return;
-        (plane == 3 ? x.offset_e : plane == 2 ? x.offset_s : plane ? x.offset_d : x.offset) = off;
+        (plane ? x.offset_d : x.offset) = off;
         off += (bytes + 255) & ~(size_t) 255;
         placed[i] |= 1 << plane;
     };
@@ -1179,9 +1100,6 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
     for (size_t i = 0; i < m->w.size(); ++i)
         for (int plane = 0; plane < 2; ++plane)
             if (!(placed[i] & (1 << plane))) place(m->w[i].name, plane);
-    // split rows, then exponents: a w1 and its w3 follow one another (mlp_hidden % 64: no gaps)
-    for (int plane = 2; plane < 4; ++plane)
-        for (size_t i = 0; i < m->w.size(); ++i) place(m->w[i].name, plane);
     const int B = c.max_batch, T = c.max_latent, C = c.max_clip, S = c.max_sync;
     const int64_t Ml = (int64_t) (nj + c.fused_depth) * 6 * H + 2 * H;          // latent blocks + final layer
     const int64_t Mg = (int64_t) 2 * (nj - 1) * 6 * H + 2 * 2 * H;             // clip + text (last pre_only)
@@ -1250,12 +1168,6 @@ int create_impl(const tsk_mmdit_config *cfg, const TypeFn &type_of, tsk_mmdit **
         if (any_bf16) {
             m->cvt_cap = conv_rows * Wcv;
             a(&m->cvt16, 2 * m->cvt_cap);
-        }
-        if (any_split) {
-            m->xsplit_cap = conv_rows * Wcv;
-            m->xexp_cap = (int) conv_rows;
-            a(&m->xsplit, 4 * m->xsplit_cap);
-            a(&m->xexp, sizeof(int) * conv_rows);
         }
         if (any_q8) {
             m->q_cap = conv_rows * Wcv;
@@ -1400,17 +1312,6 @@ extern "C" int tsk_mmdit_set_tensor(tsk_mmdit *m, const char *name, const float 
     }
     if (x.type == TSK_TYPE_F32) {
         e = hipMemcpy(m->blob + x.offset, v.data(), 4 * (size_t) n, hipMemcpyHostToDevice);
-        if (e == hipSuccess && x.split) {
-            SplitRowsGroup g;
-            memset(&g, 0, sizeof(g));
-            g.n = 1;
-            g.j[0].rows = x.kind == K_CONV ? x.ne[2] : x.ne[1];
-            g.j[0].cols = (int) (n / g.j[0].rows);
-            g.j[0].x = (const float *) (m->blob + x.offset); g.j[0].ld_x = g.j[0].cols;
-            g.j[0].y = (uint32_t *) (m->blob + x.offset_s); g.j[0].e = (int *) (m->blob + x.offset_e);
-            e = launch_split_rows(g, nullptr);
-            if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-        }
     } else if (x.type == TSK_TYPE_BF16) {
         std::vector<uint16_t> bf((size_t) n);
         for (int64_t i = 0; i < n; ++i) bf[i] = host_bf16_bits(v[i]);

@@ -448,82 +448,6 @@ bool gemm_f32x6_fits(const GemmProblem &p);    // and tuning().f32_split
 int gemm_f32x6_slices(int64_t M, int64_t N, int64_t K, int most);
 hipError_t launch_gemm_f32x6(const GemmProblem &p, int y_bf16, hipStream_t s, const F32Snake *snake = nullptr,
                              const F32Unit *unit = nullptr);
-// F32 products on the fp16 matrix cores (gemm_split.hip): operands as split
-// rows (32 hi, 32 lo fp16 per group of 32 values, of the value times
-// 2^(15 - e); one 4-byte word per value, strides in words)
-struct SplitGemm {
-    const uint32_t *x, *w;         // split activation rows, split weight rows [M][K] (ld_w)
-    int64_t ld_x, ld_w;
-    const int *we;                 // [M] exponents of the weight rows
-    const int *xe;                 // exponent of x, or with xe_per_row (no SnakeBeta) one per row of x
-    int xe_per_row;
-    const float *bias;             // [M], nullable
-    void *y;                       // f32 (or y_bf16) rows; with a SnakeBeta nullable
-    int64_t ld_y;                  // also the row stride of y2 and yp
-    int y_bf16, accumulate;        // accumulate: y += (SnakeBeta form only)
-    int M, N, K;
-    int splits;                    // K slices: slice z into y + z * part_stride, no bias (1: none)
-    int64_t part_stride;
-    // implicit im2col as GemmProblem's, over contiguous batch items of conv_iw rows
-    int conv_ic, conv_iw, conv_ow, conv_s, conv_p, conv_d;
-    // without a SnakeBeta: the f32 operands (results of infinities and NaN);
-    // rows from wf_rows on are wf2's (two kernels of one input side by side)
-    const float *xf, *wf, *wf2;
-    int64_t ld_xf, xf_batch, ld_wf;
-    int wf_rows;
-    // SnakeBeta of y (ea non-null; F32Snake's parameters): split rows yp, or f32 rows y2
-    const float *ea, *eb;
-    int period;
-    float *y2;
-    uint32_t *yp;
-    // yp's exponent, from a bound: l1 * *amax_x + badd (+ 1.01 * *amax_old), written to *e_out;
-    // slots raised to max |y| / max |snake| (nullable)
-    float l1, badd;
-    const float *amax_x, *amax_old;
-    int *e_out;
-    float *amax_y, *amax_s;
-    // residual unit (w2 non-null; M <= 128, M % 32): a second, k1 convolution of the
-    // SnakeBeta (mid_*) of the first one; bias, ea, eb, y, l1, badd are the second's.
-    // The first's output is bounded by mid_l1 * *amax_x + mid_badd
-    const uint32_t *w2;            // [M][M] split rows
-    const int *we2;
-    const float *mid_bias, *mid_ea, *mid_eb;   // [M]
-    float mid_l1, mid_badd;
-    // set by the launcher
-    int tiles_m, tiles_n, m_inner, per_xcd;
-    int64_t x_rows;
-};
-// M % 4, K (and conv_ic) % 32, 16-byte aligned rows (strides % 4)
-hipError_t launch_gemm_split(SplitGemm &p, hipStream_t s);
-bool split_gemm_fits(int64_t M, int64_t K, int64_t x_rows, int64_t ld_x, int items);
-// K slices that fill the chip with the tiles of an M x N x K split product
-int split_gemm_slices(int64_t M, int64_t N, int64_t K, int most);
-// f32 rows -> split rows [rows][cols] (cols % 32) and their exponents, up to
-// four sets in one launch; in place with y == x, ld_x == cols. Row r is at x +
-// r * ld_x, or with rows_b (rows per batch item) at x + r / rows_b * ld_b + r %
-// rows_b * ld_x. halo (<= SPLIT_HALO): (KW - 1) * dilation of the convolution
-// that reads the rows
-constexpr int SPLIT_RB = 8, SPLIT_HALO = 12;
-struct SplitRows {
-    const float *x;
-    int64_t ld_x, ld_b;
-    int rows_b;
-    int64_t rows;
-    int cols, halo;
-    uint32_t *y;
-    int *e;
-    // set by the launcher
-    int rows_wg, begin;
-};
-struct SplitRowsGroup {
-    SplitRows j[4];
-    int n;
-};
-hipError_t launch_split_rows(SplitRowsGroup &g, hipStream_t s);
-// slot[0] = max |x| of the finite values, *e its exponent, slot[1 .. nslot) = 0
-hipError_t launch_split_begin(const float *x, int64_t n, float *slot, int nslot, int *e, hipStream_t s);
-// x [C][T] f32 -> split rows [T][C] at exponent *e (C % 32 == 0)
-hipError_t launch_split_transpose(const float *x, int C, int T, const int *e, uint32_t *y, hipStream_t s);
 // y = silu(a) * b, f32, n elements
 hipError_t launch_silu_mul(const float *a, const float *b, float *y, int64_t n, hipStream_t s);
 // y[n][f] = silu(a) * b for rows of 2 F: a = p[n][f], b = p[n][F + f], each the

@@ -44,7 +44,7 @@ bool workspace_can(hipStream_t s, size_t bytes);
 //   TSK_F32_DL / TSK_F32_DL_NS  fp32 MFMA GEMM with direct global -> LDS loads (1, default; 0 = register staged)
 //                 and its ring depth (2, default; 3)
 //   TSK_F32_SPLIT F32 products as six bf16 products of operands in three parts (1, default) or fp32 MFMA
-//                 products (0), read on every call; a reference graph created with 1 holds fp16 split copies
+//                 products (0), read on every call
 //   TSK_SPLIT_WG  most 128 x 128 tiles times K slices of the graph's bf16 convolutions into plain rows (512)
 struct Tuning {
     int q8_cfg = 0;
