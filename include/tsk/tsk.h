@@ -159,9 +159,11 @@ int tsk_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bias
  * tsk_mul_mat; its scratch (the bf16 rows of f32 activations, the Q8_0
  * repack and activation planes) lives in one fixed array of
  * TSK_MUL_MAT_NOALLOC_SCRATCH bytes per GPU, resident until the process
- * ends; a node needing more (tsk_workspace_size) returns TSK_ERR_NOMEM
- * before any launch. Every call on one GPU shares that GPU's array: calls
- * that overlap on one GPU (other streams or threads) race.
+ * ends; a node whose conversions need more returns TSK_ERR_NOMEM before any
+ * launch (of the size tsk_workspace_size gives, the K slices of a BF16 product
+ * are left out where they do not fit: the same bits). F32 weights, and BF16
+ * weights with BF16 b, use none of it. Every call on one GPU shares that
+ * GPU's array: calls that overlap on one GPU (other streams or threads) race.
  */
 #define TSK_MUL_MAT_NOALLOC_SCRATCH (32u << 20)
 int tsk_mul_mat_noalloc(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bias,
@@ -349,7 +351,10 @@ int tsk_supports_op(int op, const tsk_tensor *const *srcs, int n_srcs,
  * (tsk_set_workspace); 0 for operators that need none. Validates the
  * descriptors like the entry point (data pointers are not inspected) and
  * returns its status. Counterpart of a ggml backend's buffer sizing
- * (ggml_backend_buft_get_alloc_size); srcs as for tsk_supports_op. */
+ * (ggml_backend_buft_get_alloc_size); srcs as for tsk_supports_op. For BF16
+ * weights over a long K the size includes K slices of the product: with a
+ * smaller workspace that holds the rest the node runs in one piece, slower,
+ * with the same bits. */
 int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_srcs,
                        const tsk_tensor *dst, size_t *bytes);
 

@@ -274,3 +274,24 @@ def test_conv1d_single_row_any_stride(env, bf16):
     tsk.synchronize()
     assert np.array_equal(out.numpy(), ref)
     assert rel_l2(ref, orc.conv1d(w, x, w_type=orc.BF16 if bf16 else orc.F32)) <= (3e-4 if bf16 else 1e-5)
+
+
+def test_slices_do_not_depend_on_the_scratch(env):
+    """the BF16 convolution and conv MLP give the same bits with the workspace tsk_workspace_size asks for and with one
+    that leaves no room for their K slices"""
+    tsk, orc = env
+    rng = np.random.default_rng(12)
+    x = tsk.to_device(rng.standard_normal((2, 100, 1024)).astype(np.float32))
+    w = [tsk.bf16_to_device(kernel(orc, rng, *s)) for s in ((128, 1024, 3), (1024, 1024, 3), (1024, 1024, 3), (1024, 1024, 3))]
+    y, ym = tsk.empty((2, 100, 128)), tsk.empty((2, 100, 1024))
+    for op, srcs, dst, run in ((tsk.OP_CONV1D, [w[0], x], y, lambda: tsk.conv1d(w[0], x).numpy()),
+                               (tsk.OP_CONV_MLP_SWIGLU, [w[1], w[2], w[3], x], ym,
+                                lambda: tsk.conv_mlp_swiglu(w[1], w[2], w[3], x).numpy())):
+        ref, n = run(), tsk.workspace_size(op, srcs, dst)
+        try:
+            for size in (n, n - 256):
+                buf = tsk.empty((size,), "u8")
+                tsk.set_workspace(buf)
+                assert np.array_equal(run(), ref), (op, size)
+        finally:
+            tsk.set_workspace(None)

@@ -195,3 +195,37 @@ def test_bf16_gemm_f32_rows_and_slices(env, N, K, M):
     assert rel_l2(y, orc.mul_mat(wb, x, a_type=orc.BF16) + bias) <= 2e-6
     y16 = tsk.mul_mat(wd, tsk.bf16_to_device(orc.f32_to_bf16_bits(x)), bias=bd).numpy()
     assert np.array_equal(y, y16)
+
+
+@pytest.mark.parametrize("N,K,M", [(64, 4096, 1024), (9, 2816, 80), (388, 4096, 1024)])
+def test_bf16_bits_do_not_depend_on_the_scratch(env, N, K, M):
+    """long K over few tiles: the same bits in K slices and in one piece -- with the workspace tsk_workspace_size asks
+    for, with only the rows' bf16 copy's, captured, through tsk_mul_mat_noalloc, and from bf16 rows, which need none"""
+    tsk, orc = env
+    rng = np.random.default_rng(N + K)
+    wb = orc.f32_to_bf16_bits((rng.standard_normal((M, K)) * 0.05).astype(np.float32))
+    x, bias = rng.standard_normal((N, K)).astype(np.float32), rng.standard_normal(M).astype(np.float32)
+    wd, bd, xd, y = tsk.bf16_to_device(wb), tsk.to_device(bias), tsk.to_device(x), tsk.empty((N, M))
+    xb = tsk.bf16_to_device(orc.f32_to_bf16_bits(x))
+    need, most = (N * K * 2 + 255) // 256 * 256, tsk.workspace_size(tsk.OP_MUL_MAT, [wd, xd], y)
+    assert most > need and tsk.workspace_size(tsk.OP_MUL_MAT, [wd, xb], y) == 0
+    ref = tsk.mul_mat(wd, xd, bias=bd).numpy()
+    assert rel_l2(ref, orc.mul_mat(wb, x, a_type=orc.BF16) + bias) <= 2e-6
+    s = tsk.Stream()
+    for size in (most, need):
+        buf = tsk.empty((size,), "u8")
+        tsk.set_workspace(buf, stream=s)
+        tsk.mul_mat(wd, xd, bias=bd, out=y, stream=s)
+        s.synchronize()
+        assert np.array_equal(y.numpy(), ref), size
+        g = tsk.Graph(s, lambda: tsk.mul_mat(wd, xd, bias=bd, out=y, stream=s))
+        for _ in range(3):
+            g.launch()
+            s.synchronize()
+            assert np.array_equal(y.numpy(), ref), size
+        g.destroy()
+    tsk.set_workspace(None, stream=s)
+    s.destroy()
+    assert np.array_equal(tsk.mul_mat(wd, xb, bias=bd).numpy(), ref)
+    assert np.array_equal(tsk.mul_mat_noalloc(wd, xd, bias=bd).numpy(), ref)
+    assert np.array_equal(tsk.mul_mat_noalloc(wd, xb, bias=bd).numpy(), ref)

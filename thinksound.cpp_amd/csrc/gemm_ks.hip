@@ -460,6 +460,12 @@ __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord t
 #pragma unroll
         for (int s = 0; s < R - 1; ++s)
             if (s < ns) cissue(s, s);
+        // SUMS: the sum of every sum_stages stages on its own, then those in
+        // order, as EPI_PARTIAL slices and the pass over them give
+        constexpr bool SUMS = EPI == EPI_STORE_F32_SUMS;
+        f32x4 tot[SUMS ? TMW : 1][SUMS ? TNW : 1];
+        int left = SUMS ? p.sum_stages : 0;
+        bool first = true;
         int slot = 0;
         for (int t = 0; t < ns; ++t) {
             wait_stages<LW, R - 1>(min(ns - 1 - t, R - 2));
@@ -467,6 +473,25 @@ __device__ __forceinline__ void gemm_ks_tile(const GemmProblem &p, const Coord t
             if (t + R - 1 < ns) cissue(t + R - 1, slot == 0 ? R - 1 : slot - 1);
             compute(lds + slot * STG);
             slot = slot + 1 == R ? 0 : slot + 1;
+            if constexpr (SUMS) {
+                if (--left == 0) {
+#pragma unroll
+                    for (int i = 0; i < TMW; ++i)
+#pragma unroll
+                        for (int j = 0; j < TNW; ++j) {
+                            tot[i][j] = first ? acc[i][j] : tot[i][j] + acc[i][j];
+                            acc[i][j] = f32x4{0, 0, 0, 0};
+                        }
+                    first = false;
+                    left = p.sum_stages;
+                }
+            }
+        }
+        if constexpr (SUMS) {
+#pragma unroll
+            for (int i = 0; i < TMW; ++i)
+#pragma unroll
+                for (int j = 0; j < TNW; ++j) acc[i][j] = tot[i][j];
         }
         }
     } else if constexpr (PIPE) {
@@ -940,9 +965,15 @@ hipError_t conv_epi(GemmGroup &g, int epi, hipStream_t s) {
         case EPI_SWIGLU_F32: return ks_launch<TM, TN, R, MODE, EPI_SWIGLU_F32, 1, CONV>(g, s);
         case EPI_SWIGLU_BF16: return ks_launch<TM, TN, R, MODE, EPI_SWIGLU_BF16, 1, CONV>(g, s);
         case EPI_PARTIAL: return ks_launch<TM, TN, R, MODE, EPI_PARTIAL, 1, CONV>(g, s);
+        case EPI_STORE_F32_SUMS:
+            if constexpr (MODE == MODE_COOP64) return ks_launch<TM, TN, R, MODE, EPI_STORE_F32_SUMS, 1, CONV>(g, s);
+            return hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
     }
 }
+
+// EPI_STORE_F32_SUMS: whole sums of 64-wide stages
+bool sums_ok(const GemmProblem &p) { return p.sum_stages > 0 && p.K % 64 == 0 && p.K / 64 % p.sum_stages == 0; }
 
 }  // namespace
 
@@ -955,6 +986,7 @@ hipError_t launch_gemm_coop_xf32(GemmGroup &g, int epi, hipStream_t s) {
     if (conv && (p.conv_ic % 64 || p.K % p.conv_ic || p.x_group_rows || p.conv_ow < 1 || p.conv_iw < 1 || p.conv_s < 1 ||
                  p.conv_d < 1 || p.conv_p < 0 || p.N % p.conv_ow || p.x_group_stride % 4))
         return hipErrorInvalidValue;
+    if (epi == EPI_STORE_F32_SUMS && !sums_ok(p)) return hipErrorInvalidValue;
     // a two-stage ring: three workgroups per CU (three stages, two: 388 x 1024
     // -> 3072 11.9 / 12.3 us, 2080 rows 40 / 51)
     switch (epi) {
@@ -964,6 +996,9 @@ hipError_t launch_gemm_coop_xf32(GemmGroup &g, int epi, hipStream_t s) {
         case EPI_STORE_BF16:
             return conv ? ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_BF16, 1, true>(g, s)
                         : ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_BF16, 1, false>(g, s);
+        case EPI_STORE_F32_SUMS:
+            return conv ? ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_F32_SUMS, 1, true>(g, s)
+                        : ks_launch<4, 4, 2, MODE_COOP64F, EPI_STORE_F32_SUMS, 1, false>(g, s);
         case EPI_PARTIAL:
             return conv ? ks_launch<4, 4, 2, MODE_COOP64F, EPI_PARTIAL, 1, true>(g, s)
                         : ks_launch<4, 4, 2, MODE_COOP64F, EPI_PARTIAL, 1, false>(g, s);
@@ -1008,6 +1043,10 @@ hipError_t launch_gemm_coop(GemmGroup &g, int epi, hipStream_t s) {
     int cfg = k64 ? (tiles128 >= 400 ? 32 : tiles >= 400 ? 29 : 30) : (tiles >= 512 ? 12 : 22);
     if (tuning().coop_cfg) cfg = tuning().coop_cfg;
     if (!k64 && cfg >= 28) cfg = tiles >= 512 ? 12 : 22;
+    if (epi == EPI_STORE_F32_SUMS) {
+        if (g.nprob != 1 || !k64 || !sums_ok(g.p[0])) return hipErrorInvalidValue;
+        if (cfg < 28) cfg = 30;
+    }
     switch (cfg) {
         case 12: return conv ? conv_epi<8, 4, 4, true>(g, epi, s) : conv_epi<8, 4, 4, false>(g, epi, s);
         case 22: return conv ? conv_epi<4, 4, 4, true>(g, epi, s) : conv_epi<4, 4, 4, false>(g, epi, s);

@@ -438,21 +438,34 @@ struct Scratch {
 size_t align256(size_t n) { return (n + 255) & ~(size_t) 255; }
 
 // K slices of a BF16 product on the cooperative tiles (f32 result): see
-// coop_slices(); 0 bytes where it runs whole
-size_t coop_part_bytes(int64_t M, int64_t N, int64_t K, int64_t ic, bool y_bf16, int *splits) {
+// gemm_coop_slices(). They take scratch only where the node needs some anyway
+// (need > 0; a node without any stays so, whatever runs on other streams and in
+// captured graphs), and only if it can be had; the product in one piece sums
+// the same slices in the same order, so the bits depend on the operands alone.
+size_t coop_part_bytes(size_t need, int64_t M, int64_t N, int64_t K, int64_t ic, bool y_bf16, int *splits) {
     *splits = y_bf16 ? 1 : gemm_coop_slices(M, N, K, ic);
-    return *splits > 1 ? align256((size_t) *splits * (size_t) (N * M) * 4) : 0;
+    return need && *splits > 1 ? align256((size_t) *splits * (size_t) (N * M) * 4) : 0;
 }
-// g.p[0] (f32 result, with its bias) as `splits` slices in part, then their sum
-hipError_t coop_sliced(GemmGroup &g, float *part, int splits, bool xf32, hipStream_t s) {
+// g.p[0] (with its bias) on the cooperative tiles, an f32 result as `splits`
+// slices in part and their sum, or (part null) in one piece
+hipError_t coop_product(GemmGroup &g, int epi, float *part, int splits, bool xf32, hipStream_t s) {
     GemmProblem &q = g.p[0];
     const float *bias = q.bias;
     float *y = (float *) q.y;
     const int64_t ld_y = q.N == 1 ? q.M : q.ld_y;            // (a single row's stride may be anything)
-    q.bias = nullptr; q.y = part; q.ld_y = q.M; q.splits = splits;
-    const hipError_t e = xf32 ? launch_gemm_coop_xf32(g, EPI_PARTIAL, s) : launch_gemm_coop(g, EPI_PARTIAL, s);
-    return e == hipSuccess ? launch_sum_slices(part, splits, (int64_t) q.N * q.M, bias, q.N, q.M, y, ld_y, s) : e;
+    const bool slices = epi == EPI_STORE_F32 && splits > 1;
+    if (slices && part) {
+        q.bias = nullptr; q.y = part; q.ld_y = q.M; q.splits = splits;
+        epi = EPI_PARTIAL;
+    } else if (slices) {
+        q.sum_stages = q.K / 64 / splits;
+        epi = EPI_STORE_F32_SUMS;
+    }
+    const hipError_t e = xf32 ? launch_gemm_coop_xf32(g, epi, s) : launch_gemm_coop(g, epi, s);
+    return e == hipSuccess && slices && part
+               ? launch_sum_slices(part, splits, (int64_t) q.N * q.M, bias, q.N, q.M, y, ld_y, s) : e;
 }
+
 // f32 activations of BF16 weights rounded inside the product's kernel instead
 // of by a launch before it: the launch and its pass over memory against twice
 // the activation bytes in a ring of two stages. That ring hides less of the
@@ -504,7 +517,7 @@ MulMatPlan plan_mul_mat(const tsk_tensor *a, const tsk_tensor *b, const tsk_tens
     }
     pl.bytes = pl.cast_bytes + pl.wbytes + pl.act_bytes;
     pl.splits = 1;
-    if (pl.coop) pl.part_bytes = coop_part_bytes(M, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16, &pl.splits);
+    if (pl.coop) pl.part_bytes = coop_part_bytes(pl.bytes, M, pl.Nslice, K, 0, dst->type == TSK_TYPE_BF16, &pl.splits);
     return pl;
 }
 
@@ -571,8 +584,7 @@ int mul_mat_impl(const tsk_tensor *a, const tsk_tensor *b, const tsk_tensor *bia
         q.ld_y = (int64_t) (dst->nb[1] / es_d);
         q.M = (int) M; q.N = (int) N; q.K = (int) K; q.splits = 1;
         const int epi = dst->type == TSK_TYPE_BF16 ? EPI_STORE_BF16 : EPI_STORE_F32;
-        hipError_t e = sliced ? coop_sliced(g, (float *) (ws + pl.bytes), pl.splits, xf32, s)
-                     : xf32 ? launch_gemm_coop_xf32(g, epi, s) : launch_gemm_coop(g, epi, s);
+        hipError_t e = coop_product(g, epi, sliced ? (float *) (ws + pl.bytes) : nullptr, pl.splits, xf32, s);
         return e == hipSuccess ? TSK_OK : hip_fail(e, "mul_mat launch");
     }
 
@@ -1146,7 +1158,7 @@ size_t conv_cast_bytes(int wtype, int x_f32, int64_t IC, int64_t IW, int64_t B, 
 // stride xb in elements), y rows [B * OW][OC] (ld_y); kw-major weight rows.
 // swiglu: w3 rows given -> y = silu(x * w) * (x * w3) (BF16 kernels only).
 // xcast: conv_cast_bytes() of scratch, or nullptr when that is 0.
-// part: scratch of `splits` K slices of an f32 result, or nullptr.
+// splits: K slices of an f32 result on the cooperative tiles, part: their scratch, or nullptr.
 int conv_gemm(int wtype, const void *wrows, const void *w3rows, int64_t ld_w, const float *bias, int KW, int IC, int OC,
               const void *x, int x_f32, int64_t ld_x, int64_t xb, int IW, int B, int s0, int p0, int d0, void *y,
               int y_bf16, int64_t ld_y, uint16_t *xcast, hipStream_t s, float *part = nullptr, int splits = 1,
@@ -1184,20 +1196,9 @@ int conv_gemm(int wtype, const void *wrows, const void *w3rows, int64_t ld_w, co
         q.w3 = (const uint16_t *) w3rows;
         g.p[0] = q;
         const int epi = w3rows ? (y_bf16 ? EPI_SWIGLU_BF16 : EPI_SWIGLU_F32) : (y_bf16 ? EPI_STORE_BF16 : EPI_STORE_F32);
-        e = coop && part && epi == EPI_STORE_F32 ? coop_sliced(g, part, splits, xf32, s)
-            : coop && xf32 ? launch_gemm_coop_xf32(g, epi, s)
-            : coop ? launch_gemm_coop(g, epi, s) : launch_gemm_group(g, x_f32 ? GEMM_X_F32 : 0, epi, s);
+        e = coop ? coop_product(g, epi, part, splits, xf32, s) : launch_gemm_group(g, x_f32 ? GEMM_X_F32 : 0, epi, s);
     }
     return e == hipSuccess ? TSK_OK : hip_fail(e, "conv GEMM launch");
-}
-
-// BF16 kernels in K slices (after conv1d_ws_bytes)
-size_t conv1d_part_bytes(const tsk_tensor *w, const tsk_tensor *x, int s0, int p0, int d0, const tsk_tensor *dst, int *splits) {
-    const int64_t KW = w->ne[0], IC = w->ne[1], OC = w->ne[2];
-    *splits = 1;
-    if (!conv_coop(w->type, (int) IC, (int) OC)) return 0;
-    return coop_part_bytes(OC, x->ne[2] * conv_out_len(x->ne[1], KW, s0, p0, d0), KW * IC, IC, dst->type == TSK_TYPE_BF16,
-                           splits);
 }
 
 // scratch of tsk_conv1d: the kw-major kernel copy and the bf16 input rows
@@ -1209,6 +1210,14 @@ bool conv1d_xf32(const tsk_tensor *w, const tsk_tensor *x, int splits) {
 }
 size_t conv1d_ws_bytes(const tsk_tensor *w, const tsk_tensor *x) {
     return conv_pack_bytes(w) + conv_cast_bytes(w->type, x->type == TSK_TYPE_F32, w->ne[1], x->ne[1], x->ne[2], w->ne[2]);
+}
+
+// BF16 kernels in K slices over OW output positions of each item (after conv1d_ws_bytes)
+size_t conv1d_part_bytes(const tsk_tensor *w, const tsk_tensor *x, int64_t OW, const tsk_tensor *dst, int *splits) {
+    const int64_t KW = w->ne[0], IC = w->ne[1], OC = w->ne[2];
+    *splits = 1;
+    if (!conv_coop(w->type, (int) IC, (int) OC)) return 0;
+    return coop_part_bytes(conv1d_ws_bytes(w, x), OC, x->ne[2] * OW, KW * IC, IC, dst->type == TSK_TYPE_BF16, splits);
 }
 
 int validate_im2col(const tsk_tensor *kernel, const tsk_tensor *x, int s0, int p0, int d0, const tsk_tensor *dst) {
@@ -1283,7 +1292,7 @@ extern "C" int tsk_conv1d(const tsk_tensor *w, const tsk_tensor *bias, const tsk
     const size_t cast = conv_cast_bytes(w->type, x_f32, w->ne[1], x->ne[1], x->ne[2], w->ne[2]);
     const size_t need = conv1d_ws_bytes(w, x);
     int splits = 1;
-    const size_t pbytes = conv1d_part_bytes(w, x, s0, p0, d0, dst, &splits);
+    const size_t pbytes = conv1d_part_bytes(w, x, dst->ne[1], dst, &splits);
     const bool sliced = pbytes && (ws = Scratch{s, nullptr, 0}.optional(need + pbytes));
     const bool xf32 = conv1d_xf32(w, x, sliced ? splits : 1);
     if (!sliced && (rc = workspace(s, need, (void **) &ws))) return rc;
@@ -1331,12 +1340,12 @@ size_t swiglu_mlp_ws_bytes(const tsk_tensor *w1, const tsk_tensor *w3, const tsk
 }
 
 // BF16 kernels: K slices of w2 (after swiglu_mlp_ws_bytes)
-size_t swiglu_part_bytes(const tsk_tensor *w1, int KW1, int HID, int KW2, int OC, int pad, int IW, int B, bool y_bf16,
+size_t swiglu_part_bytes(size_t need, const tsk_tensor *w1, int KW1, int HID, int KW2, int OC, int pad, int IW, int B, bool y_bf16,
                          int *splits) {
     const int64_t OW1 = conv_out_len(IW, KW1, 1, pad, 1), OW2 = conv_out_len(OW1, KW2, 1, pad, 1);
     *splits = 1;
     if (OW1 < 1 || OW2 < 1 || !conv_coop(w1->type, HID, OC)) return 0;
-    return coop_part_bytes(OC, B * OW2, (int64_t) KW2 * HID, HID, y_bf16, splits);
+    return coop_part_bytes(need, OC, B * OW2, (int64_t) KW2 * HID, HID, y_bf16, splits);
 }
 
 // convmlp / mlp on validated operands: geometry of the two convolutions
@@ -1355,7 +1364,7 @@ int swiglu_mlp(const tsk_tensor *w1, const tsk_tensor *w3, const tsk_tensor *w2,
     int rc;
     const size_t need = swiglu_mlp_ws_bytes(w1, w3, w2, KW1, IC, HID, pad, x_f32, IW, B);
     int splits2;
-    const size_t pbytes = swiglu_part_bytes(w1, KW1, HID, KW2, OC, pad, IW, B, y_bf16, &splits2);
+    const size_t pbytes = swiglu_part_bytes(need, w1, KW1, HID, KW2, OC, pad, IW, B, y_bf16, &splits2);
     const bool sliced = pbytes && (ws = Scratch{s, nullptr, 0}.optional(need + pbytes));
     if (!sliced && (rc = workspace(s, need, (void **) &ws))) return rc;
     void *h = ws;
@@ -1570,13 +1579,13 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
             return TSK_OK;
         case TSK_OP_CONV1D:
             if ((rc = need(2)) || (rc = validate_conv(&t[0], opt(2), &t[1], 1, 1, 1, &d))) return rc;
-            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + conv1d_part_bytes(&t[0], &t[1], 1, 1, 1, &d, &sp);
+            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + conv1d_part_bytes(&t[0], &t[1], d.ne[1], &d, &sp);
             return TSK_OK;
         case TSK_OP_CONV_MLP_SWIGLU:
             if ((rc = need(4)) || (rc = validate_conv_mlp(&t[0], &t[1], &t[2], &t[3], &d))) return rc;
             *bytes = swiglu_mlp_ws_bytes(&t[0], &t[1], &t[2], (int) t[0].ne[0], (int) t[0].ne[1], (int) t[0].ne[2], 1,
                                          t[3].type == TSK_TYPE_F32, (int) t[3].ne[1], (int) t[3].ne[2]) +
-                     swiglu_part_bytes(&t[0], (int) t[0].ne[0], (int) t[0].ne[2], (int) t[2].ne[0], (int) t[2].ne[2], 1,
+                     swiglu_part_bytes(1, &t[0], (int) t[0].ne[0], (int) t[0].ne[2], (int) t[2].ne[0], (int) t[2].ne[2], 1,
                                        (int) t[3].ne[1], (int) t[3].ne[2], d.type == TSK_TYPE_BF16, &sp);
             return TSK_OK;
         case TSK_OP_MLP_SWIGLU:
@@ -1586,7 +1595,7 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
             const tsk_tensor k1 = linear_as_kernel(&t[0]), k3 = linear_as_kernel(&t[1]), k2 = linear_as_kernel(&t[2]);
             *bytes = swiglu_mlp_ws_bytes(&k1, &k3, &k2, 1, (int) t[0].ne[0], (int) t[0].ne[1], 0,
                                          t[3].type == TSK_TYPE_F32, (int) (t[3].ne[1] * t[3].ne[2] * t[3].ne[3]), 1) +
-                     swiglu_part_bytes(&k1, 1, (int) t[0].ne[1], 1, (int) t[2].ne[1], 0,
+                     swiglu_part_bytes(1, &k1, 1, (int) t[0].ne[1], 1, (int) t[2].ne[1], 0,
                                        (int) (t[3].ne[1] * t[3].ne[2] * t[3].ne[3]), 1, d.type == TSK_TYPE_BF16, &sp);
             return TSK_OK;
         }

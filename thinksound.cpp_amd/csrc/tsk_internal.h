@@ -191,7 +191,11 @@ enum GroupEpi : int {
     // SwiGLU over two weights sharing X: y[n, m] = silu(X W[m]) * (X W3[m]),
     // no bias (convmlp / mlp, src/mmdit.cpp:39-52)
     EPI_SWIGLU_F32 = 15,
-    EPI_SWIGLU_BF16 = 16
+    EPI_SWIGLU_BF16 = 16,
+    // EPI_STORE_F32 whose value is the sum of p.sum_stages 64-wide k stages at a
+    // time, added up in order: the bits of EPI_PARTIAL slices of that length and
+    // launch_sum_slices
+    EPI_STORE_F32_SUMS = 17
 };
 enum GemmFlags : int { GEMM_X_F32 = 1 };
 
@@ -206,6 +210,7 @@ struct GemmProblem {
     int64_t x_group_stride;
     int M, N, K;
     int splits;                    // K slices (EPI_PARTIAL), else 1
+    int sum_stages;                // EPI_STORE_F32_SUMS
     const uint16_t *w3;            // EPI_SWIGLU_*: the second weight (same layout as w)
     const float *wf;               // launch_gemm_f32: f32 weights [M][K] row-major (ld_w)
     const float *wf3;              // launch_gemm_f32x6: a second weight, its outputs M .. 2 M - 1 (nullable)
