@@ -337,7 +337,7 @@ enum tsk_op {
     TSK_OP_ROPE_EXT       = 4,
     TSK_OP_NORM           = 5,
     TSK_OP_IM2COL         = 6,   /* srcs: kernel, x; fixed s0 = 1, p0 = 1, d0 = 1 */
-    TSK_OP_CONV1D         = 7,   /* srcs: w, x, bias; fixed s0 = 1, p0 = 1, d0 = 1 */
+    TSK_OP_CONV1D         = 7,   /* srcs: w, x, bias; tsk_supports_op: s0 = 1, p0 = 1, d0 = 1 */
     TSK_OP_CONV_MLP_SWIGLU = 8,  /* srcs: w1, w3, w2, x */
     TSK_OP_MLP_SWIGLU     = 9,   /* srcs: w1, w3, w2, x */
     TSK_OP_RMS_NORM_Q8_0  = 10   /* srcs: x, w */
@@ -351,7 +351,8 @@ int tsk_supports_op(int op, const tsk_tensor *const *srcs, int n_srcs,
  * (tsk_set_workspace); 0 for operators that need none. Validates the
  * descriptors like the entry point (data pointers are not inspected) and
  * returns its status. Counterpart of a ggml backend's buffer sizing
- * (ggml_backend_buft_get_alloc_size); srcs as for tsk_supports_op. For BF16
+ * (ggml_backend_buft_get_alloc_size); srcs as for tsk_supports_op, a
+ * convolution's dst of any length (its stride, padding and dilation). For BF16
  * weights over a long K the size includes K slices of the product: with a
  * smaller workspace that holds the rest the node runs in one piece, slower,
  * with the same bits. */

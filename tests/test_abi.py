@@ -283,3 +283,18 @@ def test_workspace_size(tsk):
     assert ws(T.OP_RMS_NORM_Q8_0, [xt, fake(T, T.F32, (2048,), 4)], qd) == (0, 400 * 2048 + 400 * 64 * 4)
     assert ws(T.OP_RMS_NORM_MUL, [xt], xt) == (0, 0)
     assert ws(99, [xt], xt)[0] == -6
+    # convolutions of any stride, padding and dilation: dst says how many
+    # output positions the K slices of a long product hold
+    x7, w7 = fake(T, T.F32, (1, 194, 1024), 4), kernel_desc(T, T.BF16, 64, 1024, 7, 2)
+    base = 7 * 1024 * 64 * 2 + 194 * 1024 * 2
+    k7 = {ow: ws(T.OP_CONV1D, [w7, x7], fake(T, T.F32, (1, ow, 64), 4)) for ow in (188, 190, 194, 200, 400)}
+    for ow, (rc, n) in k7.items():
+        assert rc == 0 and n > base
+        rows = max(ow, 194)
+        assert any((n - base) // (64 * 4 * c) >= rows and n - base <= 64 * 4 * c * rows + 256 for c in range(2, 17)), (ow, n)
+    assert k7[190][1] >= k7[194][1]                                 # a stand-in dst of padding 1 is enough too
+    assert ws(T.OP_CONV1D, [w7, x7], fake(T, T.F32, (1, 194, 128), 4))[0] == -3
+    assert ws(T.OP_CONV1D, [w7, x7], fake(T, T.F32, (2, 194, 64), 4))[0] == -3
+    x7b = fake(T, T.BF16, (1, 194, 1024), 2)
+    assert ws(T.OP_CONV1D, [kernel_desc(T, T.BF16, 64, 1024, 7, 2, True), x7b], fake(T, T.F32, (1, 194, 64), 4)) == (0, 0)
+    assert ws(T.OP_CONV1D, [kernel_desc(T, T.F32, 64, 1024, 7, 4, True), x7], fake(T, T.F32, (1, 194, 64), 4)) == (0, 0)

@@ -1096,6 +1096,7 @@ int check_conv_act(const tsk_tensor *t, const char *name) {
     return check_rows(t, name, 16);
 }
 
+// (s0 = 0: the geometry is not known, any output length of dst)
 int validate_conv(const tsk_tensor *w, const tsk_tensor *bias, const tsk_tensor *x, int s0, int p0, int d0,
                   const tsk_tensor *dst) {
     int rc;
@@ -1106,8 +1107,8 @@ int validate_conv(const tsk_tensor *w, const tsk_tensor *bias, const tsk_tensor 
     if (x->ne[0] != IC) return fail(TSK_ERR_SHAPE, "x->ne[0]=%lld != IC=%lld", (long long) x->ne[0], (long long) IC);
     if (IC % 8) return fail(TSK_ERR_SHAPE, "IC=%lld must be a multiple of 8", (long long) IC);
     if (w->type == TSK_TYPE_F32 && x->type != TSK_TYPE_F32) return fail(TSK_ERR_TYPE, "F32 kernels need F32 x");
-    if (s0 < 1 || d0 < 1 || p0 < 0) return fail(TSK_ERR_INVALID_ARG, "stride %d, padding %d, dilation %d", s0, p0, d0);
-    const int64_t OW = conv_out_len(x->ne[1], KW, s0, p0, d0);
+    if (s0 < 0 || d0 < 1 || p0 < 0) return fail(TSK_ERR_INVALID_ARG, "stride %d, padding %d, dilation %d", s0, p0, d0);
+    const int64_t OW = s0 ? conv_out_len(x->ne[1], KW, s0, p0, d0) : dst->ne[1];
     if (OW < 1) return fail(TSK_ERR_SHAPE, "output length %lld < 1", (long long) OW);
     if (dst->ne[0] != OC || dst->ne[1] != OW || dst->ne[2] != x->ne[2])
         return fail(TSK_ERR_SHAPE, "dst must be [OC=%lld, OW=%lld, B=%lld, 1]", (long long) OC, (long long) OW,
@@ -1283,6 +1284,7 @@ extern "C" int tsk_conv1d_pack_weight(const tsk_tensor *w, tsk_tensor *dst, tsk_
 
 extern "C" int tsk_conv1d(const tsk_tensor *w, const tsk_tensor *bias, const tsk_tensor *x, int s0, int p0, int d0,
                           tsk_tensor *dst, tsk_stream stream) {
+    if (s0 < 1) return fail(TSK_ERR_INVALID_ARG, "stride %d", s0);
     int rc = validate_conv(w, bias, x, s0, p0, d0, dst);
     if (rc) return rc;
     if ((rc = require_init())) return rc;
@@ -1578,8 +1580,12 @@ extern "C" int tsk_workspace_size(int op, const tsk_tensor *const *srcs, int n_s
             *bytes = fa_ws_bytes(&t[0], &t[1], &t[2], opt(3), 0.0f, 0.0f, &d);
             return TSK_OK;
         case TSK_OP_CONV1D:
-            if ((rc = need(2)) || (rc = validate_conv(&t[0], opt(2), &t[1], 1, 1, 1, &d))) return rc;
-            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + conv1d_part_bytes(&t[0], &t[1], d.ne[1], &d, &sp);
+            // stride, padding and dilation show in dst's length only; the slices
+            // of as many output positions as inputs too, for a caller whose dst
+            // stands for another geometry
+            if ((rc = need(2)) || (rc = validate_conv(&t[0], opt(2), &t[1], 0, 0, 1, &d))) return rc;
+            *bytes = conv1d_ws_bytes(&t[0], &t[1]) + std::max(conv1d_part_bytes(&t[0], &t[1], d.ne[1], &d, &sp),
+                                                              conv1d_part_bytes(&t[0], &t[1], t[1].ne[1], &d, &sp));
             return TSK_OK;
         case TSK_OP_CONV_MLP_SWIGLU:
             if ((rc = need(4)) || (rc = validate_conv_mlp(&t[0], &t[1], &t[2], &t[3], &d))) return rc;
