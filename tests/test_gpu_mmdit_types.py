@@ -212,6 +212,34 @@ def test_f32_graph_latent_outlier(env):
     m.close()
 
 
+@pytest.mark.parametrize("wt", [BF16, Q8_0, F32])
+def test_graph_of_a_larger_capacity(env, wt):
+    """a capacity of five runs the conditioning vectors' products on tiles, one of up to four on waves: each within the
+    oracle's bound, and the two no further apart than that"""
+    tsk, orc = env
+    args = inputs(2, 40, 10, 32, seed=17)
+    args = (args[0], np.array([0.8, 0.3], np.float32)) + args[1:]
+    flows = []
+    for cap in (5, 2):
+        m, od, _ = build_typed(tsk, orc, wt, max_batch=cap, **SMALL)
+        if wt == F32:
+            flows.append(m.forward(*args))
+            assert rel_l2(flows[-1], od.forward(*args, act_bf16=False, kv_f16=True)) <= 2e-3
+        elif wt == BF16:
+            flows.append(m.forward(*args))
+            ref = od.forward(*args)
+            floor = rel_l2(od.forward(*args, kv_f16=False), ref)
+            assert rel_l2(flows[-1], ref) <= max(2e-3, 2 * floor)
+        else:
+            flows.append(check(m, od, args, f"Q8_0 graph, capacity {cap}"))
+        f1 = m.forward(*(a[1:] for a in args))
+        assert np.array_equal(f1[0], flows[-1][1])                 # a row's bits do not depend on the call's batch
+        m.close()
+    d = rel_l2(*flows)
+    print(f"type {wt}: capacities 5 and 2: rel-L2 {d:.3e}", flush=True)
+    assert d <= 2e-2
+
+
 GGUF_KW = dict(depth=3, fused_depth=1, mlp_hidden=512, max_latent=64, max_clip=16, max_sync=48)
 
 
