@@ -473,11 +473,16 @@ hipError_t coop_product(GemmGroup &g, int epi, float *part, int splits, bool xf3
 // so: up to 4 (weights from memory, us with the launch / without: K = 64, 388
 // rows 6.0 / 4.5, K = 192 convolution of 1292 rows 8.3 / 7.3; K = 1024, 64 rows
 // 10.3 / 11.2, K = 2048 15.3 / 19.4), and up to 16 where K slices stand in for
-// one long product (K = 2816, 64 rows 19.1 / 12.0, K = 4096, 388 rows 32 / 21)
+// one long product (K = 2816, 64 rows 19.1 / 12.0, K = 4096, 388 rows 32 / 21).
+// Every 64-output tile reads and rounds the rows again, so few of tiles times
+// stages (M = 1024: K = 256, 1292 rows = 1344 8.6 / 6.8, 4000 rows = 4032 14.5 /
+// 14.2, 8000 rows 22.7 / 27.4; M = 3072, K = 128, 4000 rows = 6048 20.9 / 19.7,
+// K = 192 23.6 / 26.2), in slices twice as many (K = 4096, 388 rows = 7168 18.5 /
+// 18.2, M = 2048 = 14336 23.7 / 27.7)
 bool coop_xf32(int64_t M, int64_t N, int64_t K, int64_t ic, int64_t ld_w, int splits) {
     if (K % 64 || ic % 64 || ld_w % 8) return false;
     const int64_t stages = K / 64, steps = ((M + 63) / 64) * ((N + 63) / 64) * stages;
-    return stages / splits <= (splits > 1 ? 16 : 4) && steps <= (M <= 1024 && !ic ? 15000 : 4000);
+    return stages / splits <= (splits > 1 ? 16 : 4) && steps <= (splits > 1 ? 8000 : 4000);
 }
 // How tsk_mul_mat runs a validated node, and the scratch it needs.
 struct MulMatPlan {
