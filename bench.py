@@ -325,7 +325,7 @@ def graph_bench(tsk, steps, warmup=3):
     `steps` forwards; the 24-step CFG-5 sampler at 30 s (wall clock, host
     inputs and result); and the same graph with the Q8_0 GGUF's weight types
     (convert/quantize_gguf.py: 2-D linears Q8_0, the 3-D convolution kernels
-    F32, their products as three fp16 ones of split operands: the library's default)"""
+    F32, their products as six bf16 ones of operands in three parts: the library's default)"""
     import numpy as np
     out = {}
     rng = np.random.default_rng(4242)
@@ -380,8 +380,8 @@ def graph_bench(tsk, steps, warmup=3):
     out["q8_0"] = {label: timed_forwards(mq, label, T, Sc, Ss, max(3, steps // 2), 1) for label, T, Sc, Ss in shapes}
     out["q8_0"]["weights"] = ("the Q8_0 GGUF's types: 2-D linears Q8_0 (ggml's reference quantizer), 3-D "
                               "convolution kernels, t_embed MLP and vectors F32")
-    out["q8_0"]["f32_products"] = ("F32 convolution kernels as three fp16 products of scaled hi / lo halves, fp32 "
-                                   "accuracy; TSK_F32_SPLIT=0 runs them on fp32 MFMA")
+    out["q8_0"]["f32_products"] = ("F32 convolution kernels as six bf16 products of operands in three exact parts; "
+                                   "TSK_F32_SPLIT=0 runs them on fp32 MFMA")
     mq.close()
     return out
 
@@ -413,7 +413,9 @@ def vae_bench(tsk, reps=3):
         tf = fl / (ms / 1e3) / 1e12
         out[label] = {"ms": round(ms, 3), "latent_frames": T, "samples": T * v.hop,
                       "realtime_factor": round(T * v.hop / 44100.0 / (ms / 1e3), 1),
-                      "tflops": round(tf, 1), "frac_of_fp32_peak": round(tf / PEAK_FP32_TFLOPS, 4)}
+                      "tflops": round(tf, 1), "frac_of_split_peak": round(6 * tf / PEAK_BF16_TFLOPS, 4)}
+    out["products"] = ("F32 as six bf16 products of operands in three exact parts; frac_of_split_peak is of the bf16 "
+                       "peak / 6")
     v.close()
     return out
 

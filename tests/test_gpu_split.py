@@ -204,12 +204,23 @@ def test_mul_mat_spread_undone_by_the_weights(env):
 
 
 def test_mul_mat_copies_values(env):
-    """against a unit matrix every value comes back, all 24 bits of it, whatever the rest of its row is (down to
-    2^-102, where its smallest part meets fp32's smallest normal number)"""
+    """against a unit matrix every value comes back, all 24 bits of it, whatever the rest of its row is, down to
+    fp32's smallest normal numbers"""
     tsk, _ = env
     rng = np.random.default_rng(5)
-    x = (rng.standard_normal((100, 512)) * 2.0 ** rng.integers(-96, 100, (100, 512))).astype(np.float32)
+    x = (rng.standard_normal((100, 512)) * 2.0 ** rng.integers(-120, 100, (100, 512))).astype(np.float32)
+    x[np.abs(x) < 2.0 ** -126] = 0
     assert np.array_equal(tsk.mul_mat(tsk.to_device(np.eye(512, dtype=np.float32)), tsk.to_device(x)).numpy(), x)
+
+
+def test_mul_mat_tiny(env):
+    """values so small that parts of them are flushed (2^-112 and less): sums in fp32"""
+    tsk, _ = env
+    rng = np.random.default_rng(7)
+    x = (rng.standard_normal((40, 512)) * 2.0 ** -112).astype(np.float32)
+    w = rng.standard_normal((64, 512)).astype(np.float32)
+    y = tsk.mul_mat(tsk.to_device(w), tsk.to_device(x)).numpy()
+    assert rows_close(y, w, x, 2.0 ** -23)
 
 
 def test_conv1d_large_rows_beside_small_ones(env):

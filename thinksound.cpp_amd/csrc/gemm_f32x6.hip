@@ -17,8 +17,8 @@
 // every input measured (K = 1024: 1.3e-7 against 5.7e-7, K = 3072: 2.3e-7
 // against 9.9e-7; a column 2^40 above the rest against zero weights 1.3e-7).
 // At 2.5 PFLOP/s / 6 against 157 TFLOP/s: 2 x 646 rows of a k3 convolution of
-// 1024 -> 1024 channels 153 -> 79 us, 388 rows of 1024 -> 1024 47 -> 20 us, a
-// 30 s VAE decode 35.5 -> 23.4 ms.
+// 1024 -> 1024 channels 153 -> 72 us, 388 rows of 1024 -> 1024 47 -> 19 us, a
+// 30 s VAE decode 35.5 -> 23.5 ms.
 //
 // The operands are read as f32 and split once per workgroup on the way into
 // LDS. (Measured and not kept: a split by every wave from f32 in LDS, 90 us for
@@ -44,8 +44,11 @@ typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 struct Parts {
     bf16x8 p[3];
 };
+// (the empty asm keeps the pair one value: the compiler would convert the low one again instead of shifting it out)
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, bf16x2{(__bf16) a, (__bf16) b});
+    uint32_t u = __builtin_bit_cast(uint32_t, bf16x2{(__bf16) a, (__bf16) b});
+    asm("" : "+v"(u));
+    return u;
 }
 // the parts of eight values
 __device__ __forceinline__ Parts split8(const f32x4 a, const f32x4 b) {
@@ -108,8 +111,8 @@ __device__ __forceinline__ void sin2_x4(const float (&a)[4], float (&s2)[4]) {
     }
 }
 
-// fp32 product of one output whose parts' products are not finite: an infinity
-// or NaN among its operands, or a value within 2^-9 of fp32's largest
+// fp32 product of one output whose parts' products are not finite (an infinity
+// or NaN among its operands, or a value within 2^-9 of fp32's largest) or tiny
 __device__ __forceinline__ float f32_dot(const GemmProblem &p, const float *w, int n, int k0, int k1) {
     float s = 0.0f;
     const float *x = (const float *) p.x;
@@ -140,7 +143,7 @@ enum : int { PLAIN = 0, SNAKE = 1, UNIT = 2 };
 // next one into the other slot and load the one after it into registers.
 // KG = 2 where tiles are few: eight waves per CU hide a step's latency, and the
 // halves' sum in LDS costs no pass over memory (388 rows of 1024 -> 1024: 25 ->
-// 20 us, the convolution above 94 -> 79).
+// 20 us, the convolution above 94 -> 79, before the waves' order below).
 template <int TM, int TN, int WN, int KG, int WPC, int EPI>
 __global__ __launch_bounds__(128 * WN * KG, WPC) void gemm_f32x6_kernel(const X6 a) {
     constexpr int BM = 2 * TM * 16, BN = WN * TN * 16, NG = 128 * WN, NT = NG * KG;
@@ -178,6 +181,7 @@ __global__ __launch_bounds__(128 * WN * KG, WPC) void gemm_f32x6_kernel(const X6
     const int kg = __builtin_amdgcn_readfirstlane(tid >> 6) / (2 * WN);   // the waves' half of K
     const int lr = lane & 15, lg = lane >> 4;
     const int wm = wave & 1, wn = wave >> 1;
+    const bool late = EPI != PLAIN || __builtin_amdgcn_readfirstlane(tid >> 6) >= NT / 128;   // (see the loop)
     const int bm0 = tm * BM, bn0 = tn * BN;
 
     // activation rows relative to a base of the tile, so that 32-bit byte
@@ -311,18 +315,26 @@ __global__ __launch_bounds__(128 * WN * KG, WPC) void gemm_f32x6_kernel(const X6
         if (it >= nk) break;                                  // (the last step of the shorter half)
         const float *st = ring + (it & 1) * STAGE;
         float *nx = ring + (~it & 1) * STAGE;
-        Parts y[TN];
+        // of the two waves on a SIMD one splits first and one multiplies first,
+        // so that each uses one pipe (in one order MFMAs and vector instructions
+        // took turns: 78 -> 73 us for the convolution above, 76 -> 70 at 2 x 194
+        // rows; the VAE's eight waves, at the chip's power limit, lose 4 %)
+        auto multiply = [&]() {
+            Parts y[TN];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) y[j] = parts_at(st, BM + (wn * TN + j) * 16 + lr);
+            for (int j = 0; j < TN; ++j) y[j] = parts_at(st, BM + (wn * TN + j) * 16 + lr);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            mfmas(i, parts_at(st, (wm * TM + i) * 16 + lr), y);
+            for (int i = 0; i < TM; ++i) mfmas(i, parts_at(st, (wm * TM + i) * 16 + lr), y);
+        };
+        if (late) multiply();
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int q = i * NP / TM; q < (i + 1) * NP / TM; ++q) {
-                store(q, nx);                                 // (past the last step: values that nothing reads)
-                load(q);
-            }
+        for (int q = 0; q < NP; ++q) {
+            store(q, nx);                                     // (past the last step: values that nothing reads)
+            load(q);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        if (!late) multiply();
         next_step();
     }
 #pragma unroll
@@ -446,7 +458,7 @@ __global__ __launch_bounds__(128 * WN * KG, WPC) void gemm_f32x6_kernel(const X6
             for (int r = 0; r < 4; ++r) {
                 float v = a4[r];
                 if constexpr (EPI == PLAIN) {
-                    if (!finite_f(v)) v = f32_dot(p, w + (int64_t) (m0 + r) * p.ld_w, n, ks0 * BK, (ks0 + nks) * BK);
+                    if (!finite_f(v) || (v != 0.0f && fabsf(v) < 8.2718061e-25f)) v = f32_dot(p, w + (int64_t) (m0 + r) * p.ld_w, n, ks0 * BK, (ks0 + nks) * BK);
                 }
                 o[r] = v + bv[r];
             }
@@ -527,11 +539,11 @@ X6 problem(const GemmProblem &p, int y_bf16, const F32Snake *snake, const F32Uni
 
 namespace {
 // estimated microseconds of a launch on 128 x 64 tiles (wide) or 64 x 64, one
-// workgroup per CU: 1.6 or 1.05 us per 64 k (measured on 388 rows of K = 1024
-// and 4096, 1292 rows of K = 3072); K slices cost the pass that sums them
+// workgroup per CU: 1.4 or 0.9 us per 64 k (measured on 388 rows of K = 1024,
+// 100 of K = 4096, 1292 of K = 3072); K slices cost the pass that sums them
 double tiles_cost(int64_t M, int64_t N, int64_t K, int S, bool wide) {
     const int64_t units = (M + (wide ? 127 : 63)) / (wide ? 128 : 64) * ((N + 63) / 64) * S, cus = device_info().cus;
-    return (double) ((units + cus - 1) / cus * ((K / BK + 2 * S - 1) / (2 * S))) * (wide ? 1.6 : 1.05) +
+    return (double) ((units + cus - 1) / cus * ((K / BK + 2 * S - 1) / (2 * S))) * (wide ? 1.4 : 0.9) +
            (S > 1 ? 3.5 + 1.3e-6 * S * N * M : 0.0);
 }
 }  // namespace
