@@ -17,8 +17,8 @@
 // every input measured (K = 1024: 1.3e-7 against 5.7e-7, K = 3072: 2.3e-7
 // against 9.9e-7; a column 2^40 above the rest against zero weights 1.3e-7).
 // At 2.5 PFLOP/s / 6 against 157 TFLOP/s: 2 x 646 rows of a k3 convolution of
-// 1024 -> 1024 channels 153 -> 72 us, 388 rows of 1024 -> 1024 47 -> 19 us, a
-// 30 s VAE decode 35.5 -> 23.5 ms.
+// 1024 -> 1024 channels 153 -> 70 us, 388 rows of 1024 -> 1024 47 -> 18 us, a
+// 30 s VAE decode 35.5 -> 22.6 ms.
 //
 // The operands are read as f32 and split once per workgroup on the way into
 // LDS. (Measured and not kept: a split by every wave from f32 in LDS, 90 us for
@@ -67,10 +67,12 @@ __device__ __forceinline__ Parts split8(const f32x4 a, const f32x4 b) {
 // In LDS a row's 32 values of a step are 192 bytes, [32 hi][32 mid][32 lo] of
 // four 16-byte chunks each; chunk g of a part holds the values 4 g .. 4 g + 3 and
 // 16 more (the group a thread stages from two 16-byte loads; the same order
-// for both operands, so the sum's order alone depends on it). Chunk c of a row
-// is at c with its low bits turned by row / 4: the 16 rows of a fragment read
-// hit distinct banks (a row covers 48 of the 64)
-__device__ __forceinline__ int chunk_at(int row, int c) { return c ^ ((row >> 2) & 3); }
+// for both operands, so the sum's order alone depends on it). A row covers 48 of
+// the 64 banks; chunk c of it is at c with bit 1 turned by row / 8: the 16 rows of
+// a fragment read hit distinct banks in the groups that the reads are served
+// in (turned by row / 4 they do not: 33 % of the LDS cycles were conflicts, the
+// convolution above 72 -> 70 us without them)
+__device__ __forceinline__ int chunk_at(int row, int c) { return c ^ ((row >> 2) & 2); }
 
 struct X6 {
     GemmProblem p;
@@ -539,11 +541,11 @@ X6 problem(const GemmProblem &p, int y_bf16, const F32Snake *snake, const F32Uni
 
 namespace {
 // estimated microseconds of a launch on 128 x 64 tiles (wide) or 64 x 64, one
-// workgroup per CU: 1.4 or 0.9 us per 64 k (measured on 388 rows of K = 1024,
+// workgroup per CU: 1.35 or 0.85 us per 64 k (measured on 388 rows of K = 1024,
 // 100 of K = 4096, 1292 of K = 3072); K slices cost the pass that sums them
 double tiles_cost(int64_t M, int64_t N, int64_t K, int S, bool wide) {
     const int64_t units = (M + (wide ? 127 : 63)) / (wide ? 128 : 64) * ((N + 63) / 64) * S, cus = device_info().cus;
-    return (double) ((units + cus - 1) / cus * ((K / BK + 2 * S - 1) / (2 * S))) * (wide ? 1.4 : 0.9) +
+    return (double) ((units + cus - 1) / cus * ((K / BK + 2 * S - 1) / (2 * S))) * (wide ? 1.35 : 0.85) +
            (S > 1 ? 3.5 + 1.3e-6 * S * N * M : 0.0);
 }
 }  // namespace
