@@ -26,7 +26,6 @@ sys.path.insert(0, ROOT)
 PEAK_BF16_TFLOPS = 2500.0     # MI355X dense bf16 MFMA
 PEAK_HBM_GBS = 8000.0         # MI355X HBM3E
 PEAK_INT8_TOPS = 5000.0       # MI355X dense int8 MFMA
-PEAK_FP32_TFLOPS = 157.3      # MI355X dense fp32 MFMA
 
 
 def make_inputs(B, T, seed=4242):

@@ -17,8 +17,8 @@
 // every input measured (K = 1024: 1.3e-7 against 5.7e-7, K = 3072: 2.3e-7
 // against 9.9e-7; a column 2^40 above the rest against zero weights 1.3e-7).
 // At 2.5 PFLOP/s / 6 against 157 TFLOP/s: 2 x 646 rows of a k3 convolution of
-// 1024 -> 1024 channels 153 -> 70 us, 388 rows of 1024 -> 1024 47 -> 18 us, a
-// 30 s VAE decode 35.5 -> 22.6 ms.
+// 1024 -> 1024 channels 151 -> 65 us, 388 rows of 1024 -> 1024 47 -> 18 us, a
+// 30 s VAE decode 35.5 -> 21.6 ms.
 //
 // The operands are read as f32 and split once per workgroup on the way into
 // LDS. (Measured and not kept: a split by every wave from f32 in LDS, 90 us for
